@@ -129,6 +129,23 @@ int fd1d_run_f64(int nx, int t0, int nsteps, const double *ca, const double *cb,
                  int nprobe, const int *probe_k, double *probe_out, void *stream);
 int fd1d_run_max_nx(int elem_size);
 
+/* fd1d_run for a grid of any size: workgroups advance register-resident
+ * segments by many steps per launch, between the caller's state set and a
+ * partner set in work (device, fd1d_run_work_elems(nx) elements; 0: one
+ * workgroup holds the grid, and work may be NULL).  Same results bit for
+ * bit.  probe_out[p*probe_len + s], probe_len >= nsteps.                    */
+int fd1d_run_work(int nx, int t0, int nsteps, const float *ca, const float *cb,
+                  float *ex, float *hy, float *bc,
+                  int src_mode, int src_pos, const float *src_wave,
+                  int nprobe, const int *probe_k, float *probe_out, int probe_len,
+                  float *work, size_t work_elems, void *stream);
+int fd1d_run_work_f64(int nx, int t0, int nsteps, const double *ca, const double *cb,
+                      double *ex, double *hy, double *bc,
+                      int src_mode, int src_pos, const double *src_wave,
+                      int nprobe, const int *probe_k, double *probe_out, int probe_len,
+                      double *work, size_t work_elems, void *stream);
+size_t fd1d_run_work_elems(int nx);
+
 /* ca, cb of a lossy half space i >= nx/2, computed on the device in FP64 and
  * stored FP32, as fd1d/pycuda/fd1d_1_5.py:71-78 (host FP64 there).          */
 int fd1d_dielectric(int nx, double dt, double epsr, double sigma,

@@ -164,6 +164,11 @@ SIGNATURES = {
     "fd1d_run": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P, _I, _IP, _P, _P]),
     "fd1d_run_f64": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P, _I, _IP, _P, _P]),
     "fd1d_run_max_nx": (_I, [_I]),
+    "fd1d_run_work": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P, _I, _IP, _P, _I, _P,
+                           C.c_size_t, _P]),
+    "fd1d_run_work_f64": (_I, [_I, _I, _I, _P, _P, _P, _P, _P, _I, _I, _P, _I, _IP, _P, _I, _P,
+                               C.c_size_t, _P]),
+    "fd1d_run_work_elems": (C.c_size_t, [_I]),
     "fd1d_dielectric": (_I, [_I, _D, _D, _D, _P, _P, _P]),
     "fd1d_dielectric_f64": (_I, [_I, _D, _D, _D, _P, _P, _P]),
     "fd2d_dfield": (_I, [_I, _I, _I, C.POINTER(FdtdPml), _P, _P, _P, _I, _IP, _IP,

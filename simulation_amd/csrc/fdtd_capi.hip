@@ -73,11 +73,9 @@ int check_fd1d_ex(int nx, const T *ca, const T *cb, T *ex, const T *hy, int mode
 }
 
 template <typename T>
-int fd1d_run_impl(int nx, int t0, int nsteps, const T *ca, const T *cb, T *ex, T *hy, T *bc,
-                  int mode, int pos, const T *wave, int nprobe, const int *probe_k,
-                  T *probe_out, void *stream)
+int check_fd1d_run(int nx, int t0, int nsteps, const T *ca, const T *cb, T *ex, T *hy, int mode,
+                   int pos, const T *wave, int nprobe, const int *probe_k, T *probe_out)
 {
-    clear_error();
     int rc = check_fd1d_ex(nx, ca, cb, ex, hy, mode, pos);
     if (rc) return rc;
     if (nx < 3) return fail("fd1d_run: nx=%d < 3", nx);
@@ -87,12 +85,43 @@ int fd1d_run_impl(int nx, int t0, int nsteps, const T *ca, const T *cb, T *ex, T
     if (nprobe && (!probe_k || !probe_out)) return fail("fd1d_run: probe_k/probe_out required");
     for (int p = 0; p < nprobe; ++p)
         if (probe_k[p] < 0 || probe_k[p] >= nx) return fail("fd1d_run: probe %d at %d", p, probe_k[p]);
+    return 0;
+}
+
+template <typename T>
+int fd1d_run_impl(int nx, int t0, int nsteps, const T *ca, const T *cb, T *ex, T *hy, T *bc,
+                  int mode, int pos, const T *wave, int nprobe, const int *probe_k,
+                  T *probe_out, void *stream)
+{
+    clear_error();
+    int rc = check_fd1d_run(nx, t0, nsteps, ca, cb, ex, hy, mode, pos, wave, nprobe, probe_k, probe_out);
+    if (rc) return rc;
     if ((long)2 * sizeof(T) * nx > fd1d_run_lds_limit())
         return fail("fd1d_run: nx=%d exceeds the single-workgroup limit %d", nx,
                     fd1d_run_max_nx((int)sizeof(T)));
     if (nsteps == 0) return 0;
+    if (nx <= fd1d_group_max_nx())
+        return launch_fd1d_blocked<T>(nx, nsteps, ca, cb, ex, hy, bc, mode, pos, wave, nprobe, probe_k,
+                                      probe_out, nsteps, nullptr, S(stream));
     return launch_fd1d_run<T>(nx, nsteps, ca, cb, ex, hy, bc, mode, pos, wave, nprobe, probe_k,
                               probe_out, S(stream));
+}
+
+template <typename T>
+int fd1d_run_work_impl(int nx, int t0, int nsteps, const T *ca, const T *cb, T *ex, T *hy, T *bc,
+                       int mode, int pos, const T *wave, int nprobe, const int *probe_k,
+                       T *probe_out, int probe_len, T *work, size_t work_elems, void *stream)
+{
+    clear_error();
+    int rc = check_fd1d_run(nx, t0, nsteps, ca, cb, ex, hy, mode, pos, wave, nprobe, probe_k, probe_out);
+    if (rc) return rc;
+    if (nprobe && probe_len < nsteps) return fail("fd1d_run_work: probe_len=%d", probe_len);
+    if (work_elems < fd1d_run_work_elems(nx) || (fd1d_run_work_elems(nx) && !work))
+        return fail("fd1d_run_work: work has %zu elements, %zu needed", work ? work_elems : 0,
+                    fd1d_run_work_elems(nx));
+    if (nsteps == 0) return 0;
+    return launch_fd1d_blocked<T>(nx, nsteps, ca, cb, ex, hy, bc, mode, pos, wave, nprobe, probe_k,
+                                  probe_out, probe_len, work, S(stream));
 }
 
 // ---------------------------------------------------------- 2-D TM plan
@@ -408,6 +437,31 @@ int fd1d_run_f64(int nx, int t0, int nsteps, const double *ca, const double *cb,
 {
     return fd1d_run_impl<double>(nx, t0, nsteps, ca, cb, ex, hy, bc, src_mode, src_pos, src_wave,
                                  nprobe, probe_k, probe_out, stream);
+}
+
+size_t fd1d_run_work_elems(int nx)
+{
+    return nx <= fd1d_group_max_nx() ? 0 : 2 * (size_t)nx + 4;
+}
+
+int fd1d_run_work(int nx, int t0, int nsteps, const float *ca, const float *cb, float *ex,
+                  float *hy, float *bc, int src_mode, int src_pos, const float *src_wave,
+                  int nprobe, const int *probe_k, float *probe_out, int probe_len, float *work,
+                  size_t work_elems, void *stream)
+{
+    return fd1d_run_work_impl<float>(nx, t0, nsteps, ca, cb, ex, hy, bc, src_mode, src_pos,
+                                     src_wave, nprobe, probe_k, probe_out, probe_len, work,
+                                     work_elems, stream);
+}
+
+int fd1d_run_work_f64(int nx, int t0, int nsteps, const double *ca, const double *cb, double *ex,
+                      double *hy, double *bc, int src_mode, int src_pos, const double *src_wave,
+                      int nprobe, const int *probe_k, double *probe_out, int probe_len,
+                      double *work, size_t work_elems, void *stream)
+{
+    return fd1d_run_work_impl<double>(nx, t0, nsteps, ca, cb, ex, hy, bc, src_mode, src_pos,
+                                      src_wave, nprobe, probe_k, probe_out, probe_len, work,
+                                      work_elems, stream);
 }
 
 int fd1d_run_max_nx(int elem_size)

@@ -220,6 +220,13 @@ int launch_fd1d_run(int nx, int nsteps, const T *ca, const T *cb, T *ex, T *hy, 
                     int src_mode, int src_pos, const T *src_wave,
                     int nprobe, const int *probe_k, T *probe_out, hipStream_t s);
 int fd1d_run_lds_limit();          // bytes of LDS the single-workgroup run may use
+// The blocked run (fd1d.hip); work: 2*nx + 4 elements, or NULL up to
+// fd1d_group_max_nx() cells.
+template <typename T>
+int launch_fd1d_blocked(int nx, int nsteps, const T *ca, const T *cb, T *ex, T *hy, T *bc,
+                        int src_mode, int src_pos, const T *src_wave, int nprobe,
+                        const int *probe_k, T *probe_out, int probe_len, T *work, hipStream_t s);
+int fd1d_group_max_nx();            // cells the blocked run takes without a work buffer
 template <typename T>
 int launch_fd1d_dielectric(int nx, double dt, double epsr, double sigma, T *ca, T *cb,
                            hipStream_t s);

@@ -5,7 +5,8 @@ Names, argument order and meaning follow fd1d/pycuda/fd1d_1_x.py: the same
 through ctypes), ``dielectric`` for the lossy ca/cb coefficients, host-side
 ``gaussian``/``sinusoidal`` waveforms, and fields as 1-D device arrays of
 ``nx`` cells.  ``run`` replaces the per-step launch loop of ``main()``
-(fd1d/pycuda/fd1d_1_2.py:87-89) by one launch that keeps the grid in LDS.
+(fd1d/pycuda/fd1d_1_2.py:87-89) by launches of many steps over
+register-resident segments (one launch for a grid of up to 592 cells).
 """
 from __future__ import annotations
 
@@ -87,16 +88,32 @@ def hyfield(nx: int, ex: torch.Tensor, hy: torch.Tensor, bc: torch.Tensor | None
 
 def run(nx: int, nsteps: int, ex, hy, bc=None, ca=None, cb=None, src_mode=SRC_NONE,
         src_pos=0, src_wave: torch.Tensor | None = None, probes=(), t0: int = 0):
-    """nsteps steps in one launch; returns probe traces (nprobe, nsteps) on the device."""
+    """nsteps steps without a launch per step; returns probe traces (nprobe,
+    nsteps) on the device."""
     dt = ex.dtype
     pk = np.ascontiguousarray(np.asarray(probes, dtype=np.int32).reshape(-1))
-    pout = torch.zeros((len(pk), max(nsteps, 0)), dtype=dt, device=ex.device)
-    name = "fd1d_run_f64" if dt == torch.float64 else "fd1d_run"
-    pk_c = pk.ctypes.data_as(_lib._IP) if len(pk) else None
-    call(name, int(nx), int(t0), int(nsteps), ptr(ca, dt), ptr(cb, dt), ptr(ex, dt), ptr(hy, dt),
-         ptr(bc, dt), int(src_mode), int(src_pos), ptr(src_wave, dt), len(pk), pk_c,
-         ptr(pout, dt) if len(pk) else None, stream())
+    pout = torch.empty((len(pk), max(nsteps, 0)), dtype=dt, device=ex.device)
+    if nx > _lib.lib().fd1d_run_max_nx(dt.itemsize):
+        name = "fd1d_run_f64" if dt == torch.float64 else "fd1d_run"      # refuses the size
+        call(name, int(nx), int(t0), int(nsteps), ptr(ca, dt), ptr(cb, dt), ptr(ex, dt),
+             ptr(hy, dt), ptr(bc, dt), int(src_mode), int(src_pos), ptr(src_wave, dt), 0, None,
+             None, stream())
+    _advance(nx, nsteps, ex, hy, bc, ca, cb, src_mode, src_pos, src_wave, pk, pout, t0)
     return pout
+
+
+def _advance(nx, nsteps, ex, hy, bc, ca, cb, src_mode, src_pos, src_wave, pk, pout, t0, work=None):
+    """fd1d_run_work: any nx.  src_wave and pout start at the first step; pout
+    (nprobe, length) may be a slice of a longer trace along its columns."""
+    dt = ex.dtype
+    n = _lib.lib().fd1d_run_work_elems(int(nx))
+    if n and work is None:
+        work = torch.empty(n, dtype=dt, device=ex.device)
+    name = "fd1d_run_work_f64" if dt == torch.float64 else "fd1d_run_work"
+    call(name, int(nx), int(t0), int(nsteps), ptr(ca, dt), ptr(cb, dt), ptr(ex, dt), ptr(hy, dt),
+         ptr(bc, dt), int(src_mode), int(src_pos), ptr(src_wave, dt), len(pk),
+         pk.ctypes.data_as(_lib._IP) if len(pk) else None, pout.data_ptr() if len(pk) else None,
+         pout.stride(0) if len(pk) else 0, ptr(work, dt), n, stream())
 
 
 @dataclass
@@ -136,24 +153,31 @@ def simulate(cfg: Fd1dConfig, device=None) -> dict:
     else:
         w = waveform("sinusoidal", cfg.ns, 0, cfg.dtype, freq=cfg.freq)
     wave = torch.from_numpy(w).to(dev)
-    probes = []
+    pk = np.asarray(cfg.probes, dtype=np.int32).reshape(-1)
+    many = False
+    if cfg.nx > _lib.lib().fd1d_run_max_nx(np.dtype(cfg.dtype).itemsize):
+        # past fd1d_run's grid limit probes may count from the end, and be
+        # more than a launch records: those are read between single steps
+        pk = np.where(pk < 0, pk + cfg.nx, pk).astype(np.int32)
+        many = len(pk) > _lib.MAX_PROBES
+    pk = np.ascontiguousarray(pk)
+    trace = torch.empty((len(pk), cfg.ns), dtype=td, device=dev)
+    n = _lib.lib().fd1d_run_work_elems(int(cfg.nx))
+    work = torch.empty(n, dtype=td, device=dev) if n else None
     snaps_ex, snaps_hy, snap_t = [], [], []
-    fits = cfg.nx <= _lib.lib().fd1d_run_max_nx(np.dtype(cfg.dtype).itemsize)
     t = 0
     seg = cfg.snap_every if cfg.snap_every else cfg.ns
     while t < cfg.ns:
         n = min(seg, cfg.ns - t)
-        if fits:
-            pr = run(cfg.nx, n, ex, hy, bc, ca, cb, cfg.src_mode, pos, wave[t:t + n].contiguous(),
-                     cfg.probes, t0=t)
+        if many:
+            at = torch.from_numpy(pk.astype(np.int64)).to(dev)
+            for s in range(t, t + n):
+                _advance(cfg.nx, 1, ex, hy, bc, ca, cb, cfg.src_mode, pos, wave[s:s + 1], (), None,
+                         s, work)
+                trace[:, s] = ex[at]
         else:
-            pr = torch.zeros((len(cfg.probes), n), dtype=td, device=dev)
-            for s in range(n):
-                exfield(t + s + 1, cfg.nx, ca, cb, ex, hy, cfg.src_mode, pos, float(w[t + s]))
-                hyfield(cfg.nx, ex, hy, bc)
-                for p, k in enumerate(cfg.probes):
-                    pr[p, s] = ex[k]
-        probes.append(pr)
+            _advance(cfg.nx, n, ex, hy, bc, ca, cb, cfg.src_mode, pos, wave[t:t + n], pk,
+                     trace[:, t:t + n], t, work)
         t += n
         if cfg.snap_every and t % cfg.snap_every == 0:
             snaps_ex.append(ex.clone())
@@ -162,7 +186,7 @@ def simulate(cfg: Fd1dConfig, device=None) -> dict:
     torch.cuda.synchronize()
     out = dict(ex=ex.cpu().numpy(), hy=hy.cpu().numpy(),
                bc=None if bc is None else bc.cpu().numpy(),
-               probe=torch.cat(probes, dim=1).cpu().numpy() if probes else None,
+               probe=trace.cpu().numpy() if cfg.ns > 0 else None,
                snap_t=snap_t)
     if snaps_ex:
         out["snap_ex"] = torch.stack(snaps_ex).cpu().numpy()

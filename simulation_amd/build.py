@@ -8,7 +8,11 @@ layer (simulation_amd/_lib.py) loads.  Flags:
   -ffp-contract=off     no fused multiply-add: every product and sum rounds
                         on its own, as in the reference's C programs, so the
                         FP32 results are bit-identical to them;
-  -packed-fp32-ops off  no v_pk_*_f32 instructions.
+  -packed-fp32-ops off  no v_pk_*_f32 instructions;
+  -instcombine-max-...  a kernel's by-value argument struct is read in place
+                        however many reads it has; past the default of 300
+                        the compiler copies it to scratch memory (the
+                        plane-wave kernels' 1952 bytes).
 """
 from __future__ import annotations
 
@@ -28,6 +32,7 @@ FLAGS = [
     "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
     "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    "-mllvm", "-instcombine-max-copied-from-constant-users=100000",
     "-Wall", "-Wno-unused-function", "-Wno-unknown-pragmas",
 ]
 

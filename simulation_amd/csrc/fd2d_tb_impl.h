@@ -55,6 +55,7 @@
 #pragma once
 
 #include <algorithm>
+#include <climits>
 
 #include "fdtd_internal.h"
 
@@ -109,6 +110,22 @@ struct alignas(16) NaRing {
     float probe[FDTD_MAX_PROBES][K];
 };
 
+// Row profile values of 64 rows, one row a lane (rows outside the grid hold
+// the nearest one's): a level takes its rows' values by v_readlane.  As scalar
+// loads at each level they cost a wait for memory per level and position,
+// which bounded the tiles of the PML bands and with them every launch of a
+// grid too small to hide them (depth 8: 1530x2047 81 -> 53 us a launch, 60x60
+// 63 -> 39 us; 171 scalar loads and 133 waits a position, 20 now).
+struct RowProf { float gx2, gx3, fx1, fx2, fx3; };
+
+// Sources (lanes 0 ..) and probes (lanes FDTD_MAX_SOURCES ..) of the launch,
+// one a lane: a level finds those of its row with one compare instead of a
+// scalar load for each.
+// tf: the incident values of the TF/SF columns, those of level s in lanes 4s
+// .. 4s+3 (plane-wave launches, depth <= 16).
+struct SpLanes { int row, col; float tf; };
+static_assert(FDTD_MAX_SOURCES + FDTD_MAX_PROBES <= 64, "sources and probes: one a lane");
+
 struct Geom {
     int j0;           // first column of the lane
     int i0, i1;       // owned rows [i0, i1)
@@ -147,6 +164,12 @@ __device__ __forceinline__ float *at(float *base, unsigned off)
 {
     const unsigned bytes = off << 2;
     return reinterpret_cast<float *>(reinterpret_cast<char *>(base) + bytes);
+}
+
+// lane `l`'s value, in every lane
+__device__ __forceinline__ float lane_of(float v, int l)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
 }
 
 // Load the lane's C columns of a row (element offset `row` of the row start).
@@ -309,7 +332,8 @@ __device__ __forceinline__ void iterate(const PR &P, const Geom &g, const ColCoe
                                         int p, const HRow<C> &Hload, const DRow<C> &Dload,
                                         const Carry<C> (&Si)[K], Carry<C> (&So)[K],
                                         const FRow<C, NF> &Fload, const FRow<C, NF> (&SFi)[K],
-                                        FRow<C, NF> (&SFo)[K], int j, bool &vac)
+                                        FRow<C, NF> (&SFo)[K], int j, bool &vac,
+                                        const RowProf &rp, int rbase, const SpLanes &spl)
 {
     const int nx = P.nx, ny = P.ny;
     const unsigned lane = threadIdx.x & 63u;
@@ -375,9 +399,9 @@ __device__ __forceinline__ void iterate(const PR &P, const Geom &g, const ColCoe
         const HRow<C> Hp = Si[s].h;
         float gx2r = 1.f, gx3r = 1.f, fx1q = 0.f, fx2q = 1.f, fx3q = 1.f;
         if (PML && BROW) {
-            const int rc = min(max(r, 0), nx - 1), qc = min(max(q, 0), nx - 1);
-            gx2r = ldu(P.pml.gx2, rc); gx3r = ldu(P.pml.gx3, rc);
-            fx1q = ldu(P.pml.fx1, qc); fx2q = ldu(P.pml.fx2, qc); fx3q = ldu(P.pml.fx3, qc);
+            gx2r = lane_of(rp.gx2, r - rbase); gx3r = lane_of(rp.gx3, r - rbase);
+            fx1q = lane_of(rp.fx1, q - rbase); fx2q = lane_of(rp.fx2, q - rbase);
+            fx3q = lane_of(rp.fx3, q - rbase);
         }
         // ------------------------------------------------ E update, row r
         const float hxl = from_left(Hin.hx[C - 1]);
@@ -394,26 +418,33 @@ __device__ __forceinline__ void iterate(const PR &P, const Geom &g, const ColCoe
             if (BROW) dz = (r >= 1) ? dz : Din.dz[c];            // row 0: no update
             Dn.dz[c] = dz;
         }
-        for (int k = 0; SP && k < P.nsrc; ++k) {
-            if (r == P.src_i[k]) {
+        unsigned long long here = 0;              // sources and probes of row r
+        if constexpr (SP && !PR::one_sp) here = __builtin_amdgcn_ballot_w64(spl.row == r);
+        if constexpr (SP && PR::one_sp)
+            here = (P.nsrc && r == P.src_i[0] ? 1ull : 0ull) |
+                   (P.nprobe && r == P.probe_i[0] ? 1ull << FDTD_MAX_SOURCES : 0ull);
+        if (SP && here) {
+            for (unsigned m = (unsigned)here & ((1u << FDTD_MAX_SOURCES) - 1u); m; m &= m - 1u) {
+                const int k = __builtin_ctz(m);
                 // a scalar load (the same address in every lane): no vector
                 // load behind a branch in the loop, so the waits for the
                 // prefetched row stay counted
                 const float v = ldu(P.src_wave + (size_t)k * P.wave_len, t - 1);
+                const int jk = PR::one_sp ? P.src_j[0] : __builtin_amdgcn_readlane(spl.col, k);
 #pragma unroll
                 for (int c = 0; c < C; ++c)
-                    if (g.j0 + c == P.src_j[k]) Dn.dz[c] = v;
+                    if (g.j0 + c == jk) Dn.dz[c] = v;
             }
         }
         // plane wave: the TF/SF correction of dz on the box's columns
         // (fd2d/pycuda/fd2d_3_4.py:164-170), after the D update
         if (SP && NF > 0 && P.tf_npml && r >= P.tf_npml - 1 && r <= nx - P.tf_npml) {
-            const float *iv = P.inc + (size_t)(t - P.inc_t0 - 1) * P.inc_stride;
+            const float h0 = lane_of(spl.tf, 4 * s), h1 = lane_of(spl.tf, 4 * s + 1);
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 const int j = g.j0 + c;
-                if (j == P.tf_npml - 1) Dn.dz[c] = Dn.dz[c] + 0.5f * iv[0];
-                if (j == ny - P.tf_npml) Dn.dz[c] = Dn.dz[c] - 0.5f * iv[1];
+                if (j == P.tf_npml - 1) Dn.dz[c] = Dn.dz[c] + 0.5f * h0;
+                if (j == ny - P.tf_npml) Dn.dz[c] = Dn.dz[c] - 0.5f * h1;
             }
         }
 #pragma unroll
@@ -439,15 +470,17 @@ __device__ __forceinline__ void iterate(const PR &P, const Geom &g, const ColCoe
                     Fn.i[f][c] = Fin.i[f][c] - P.tw_s[s][f] * En[c];
                 }
         }
-        if (SP && P.nprobe && r >= g.i0 && r < g.i1) {
-            for (int pr = 0; pr < P.nprobe; ++pr)
-                if (r == P.probe_i[pr]) {
+        if (SP && here && r >= g.i0 && r < g.i1) {
+            for (unsigned m = (unsigned)(here >> FDTD_MAX_SOURCES); m; m &= m - 1u) {
+                const int pr = __builtin_ctz(m);
+                const int jp = PR::one_sp ? P.probe_j[0]
+                                          : __builtin_amdgcn_readlane(spl.col, FDTD_MAX_SOURCES + pr);
 #pragma unroll
-                    for (int c = 0; c < C; ++c) {
-                        const int j = g.j0 + c;
-                        if (j == P.probe_j[pr] && j >= g.vj0 && j < g.vj1) ring.probe[pr][s] = En[c];
-                    }
+                for (int c = 0; c < C; ++c) {
+                    const int j = g.j0 + c;
+                    if (j == jp && j >= g.vj0 && j < g.vj1) ring.probe[pr][s] = En[c];
                 }
+            }
         }
         // ------------------------------------------------ H update, row q
         HRow<C> Hout;
@@ -504,23 +537,23 @@ __device__ __forceinline__ void iterate(const PR &P, const Geom &g, const ColCoe
         // of hy on its top and bottom rows (fd2d/pycuda/fd2d_3_4.py:211-226)
         if (SP && NF > 0 && P.tf_npml) {
             const int a = P.tf_npml - 1, b = ny - P.tf_npml, qb = nx - P.tf_npml;
-            const float *iv = P.inc + (size_t)(t - P.inc_t0 - 1) * P.inc_stride + 2 - a;
             if (q >= a && q <= qb) {
+                const float e0 = lane_of(spl.tf, 4 * s + 2), e1 = lane_of(spl.tf, 4 * s + 3);
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
                     const int j = g.j0 + c;
-                    if (j == P.tf_npml - 2) Hout.hx[c] = Hout.hx[c] + 0.5f * iv[a];
-                    if (j == b) Hout.hx[c] = Hout.hx[c] - 0.5f * iv[b];
+                    if (j == P.tf_npml - 2) Hout.hx[c] = Hout.hx[c] + 0.5f * e0;
+                    if (j == b) Hout.hx[c] = Hout.hx[c] - 0.5f * e1;
                 }
             }
             if (q == P.tf_npml - 2 || q == qb) {
+                const float *iv = P.inc + (size_t)(t - P.inc_t0 - 1) * P.inc_stride + 2 - a;
+                const float sgn = q == qb ? 0.5f : -0.5f;     // x + (-0.5) v is x - 0.5 v
 #pragma unroll
                 for (int c = 0; c < C; ++c) {
                     const int j = g.j0 + c;
-                    if (j >= a && j <= b) {
-                        if (q == P.tf_npml - 2) Hout.hy[c] = Hout.hy[c] - 0.5f * iv[j];
-                        if (q == qb) Hout.hy[c] = Hout.hy[c] + 0.5f * iv[j];
-                    }
+                    const float v = ldg(iv + min(max(j, a), b));
+                    if (j >= a && j <= b) Hout.hy[c] = Hout.hy[c] + sgn * v;
                 }
             }
         }
@@ -656,6 +689,32 @@ __device__ __forceinline__ bool sweep(const PR &P, const Geom &g, NaRing<K, C> &
         }
     const int pbeg = max(g.i0 - K, 0);
     const int pend = g.i1 - 1 + K;
+    const int lane = (int)(threadIdx.x & 63u);
+    // lanes without a source or probe hold a row no level reaches (rows above
+    // the grid are negative)
+    SpLanes spl{INT_MIN, INT_MIN, 0.f};
+    if constexpr (SP && NF > 0) {
+        if (P.tf_npml && lane < 4 * K) {
+            const float *iv = P.inc + (size_t)(P.t_first + lane / 4 - P.inc_t0 - 1) * P.inc_stride;
+            const int w = lane & 3;
+            spl.tf = ldg(iv + (w < 3 ? w : 3 + P.ny - 2 * P.tf_npml));
+        }
+    }
+    if constexpr (SP && !PR::one_sp) {
+        if (lane < P.nsrc) { spl.row = P.src_i[lane]; spl.col = P.src_j[lane]; }
+        const int pr = lane - FDTD_MAX_SOURCES;
+        if (pr >= 0 && pr < P.nprobe) { spl.row = P.probe_i[pr]; spl.col = P.probe_j[pr]; }
+    }
+    // position p reads the profile values of rows p-K .. p: rows rbase ..
+    // rbase+63 are held, and replaced every 64-K positions
+    RowProf rp{};
+    int rbase = pbeg - K;
+    auto load_prof = [&]() __attribute__((always_inline)) {
+        const int r = min(max(rbase + lane, 0), P.nx - 1);
+        rp.gx2 = ldg(P.pml.gx2 + r); rp.gx3 = ldg(P.pml.gx3 + r);
+        rp.fx1 = ldg(P.pml.fx1 + r); rp.fx2 = ldg(P.pml.fx2 + r); rp.fx3 = ldg(P.pml.fx3 + r);
+    };
+    if constexpr (PML && BROW) load_prof();
     // row p+1 is in flight while row p is computed (rows past the grid read a
     // clamped row)
     HRow<C> H0, H1;
@@ -678,7 +737,7 @@ __device__ __forceinline__ bool sweep(const PR &P, const Geom &g, NaRing<K, C> &
         for (; p < c0 + 2 * K - 1; ++p) {
             load_row<C, LOSSY, PML, VEC, BCOL, VAC, ZIZ>(P, p + 1, g.j0, H1, D1);
             iterate<K, C, LOSSY, PML, VEC, BROW, BCOL, SP, NF, BS, true, VAC, REC, ZIZ>(
-                P, g, cc, ring, p, H0, D0, St[0], St[0], F0, SF[0], SF[0], p - c0, vac);
+                P, g, cc, ring, p, H0, D0, St[0], St[0], F0, SF[0], SF[0], p - c0, vac, rp, rbase, spl);
             H0 = H1;
             D0 = D1;
         }
@@ -687,21 +746,28 @@ __device__ __forceinline__ bool sweep(const PR &P, const Geom &g, NaRing<K, C> &
             load_row<C, LOSSY, PML, VEC, BCOL, VAC, ZIZ>(P, p + 1, g.j0, H1, D1);
             if constexpr (NF > 0) load_ft<C, NF, VEC, BCOL>(P, p + 1, g.j0, F1);
             iterate<K, C, LOSSY, PML, VEC, BROW, BCOL, SP, NF, BS, false, VAC, REC, ZIZ>(
-                P, g, cc, ring, p, H0, D0, St[0], St[NS - 1], F0, SF[0], SF[NS - 1], 0, vac);
+                P, g, cc, ring, p, H0, D0, St[0], St[NS - 1], F0, SF[0], SF[NS - 1], 0, vac, rp, rbase, spl);
             load_row<C, LOSSY, PML, VEC, BCOL, VAC, ZIZ>(P, p + 2, g.j0, H0, D0);
             if constexpr (NF > 0) load_ft<C, NF, VEC, BCOL>(P, p + 2, g.j0, F0);
             iterate<K, C, LOSSY, PML, VEC, BROW, BCOL, SP, NF, BS, false, VAC, REC, ZIZ>(
-                P, g, cc, ring, p + 1, H1, D1, St[NS - 1], St[0], F1, SF[NS - 1], SF[0], 0, vac);
+                P, g, cc, ring, p + 1, H1, D1, St[NS - 1], St[0], F1, SF[NS - 1], SF[0], 0, vac, rp, rbase, spl);
         }
         if (p == pend)
             iterate<K, C, LOSSY, PML, VEC, BROW, BCOL, SP, NF, BS, false, VAC, REC, ZIZ>(
-                P, g, cc, ring, p, H0, D0, St[0], St[NS - 1], F0, SF[0], SF[NS - 1], 0, vac);
+                P, g, cc, ring, p, H0, D0, St[0], St[NS - 1], F0, SF[0], SF[NS - 1], 0, vac, rp, rbase, spl);
     } else {
         for (int p = pbeg; p <= pend; ++p) {
+            if constexpr (PML && BROW) {
+                if (p > rbase + 63) {
+                    rbase = p - K;
+                    load_prof();
+                    __builtin_amdgcn_s_waitcnt(0);       // the waits below stay counted
+                }
+            }
             load_row<C, LOSSY, PML, VEC, BCOL, VAC, ZIZ>(P, p + 1, g.j0, H1, D1);
             if constexpr (NF > 0) load_ft<C, NF, VEC, BCOL>(P, p + 1, g.j0, F1);
             iterate<K, C, LOSSY, PML, VEC, BROW, BCOL, SP, NF, BS, false, VAC, REC, ZIZ>(
-                P, g, cc, ring, p, H0, D0, St[0], St[0], F0, SF[0], SF[0], 0, vac);
+                P, g, cc, ring, p, H0, D0, St[0], St[0], F0, SF[0], SF[0], 0, vac, rp, rbase, spl);
             H0 = H1;
             D0 = D1;
             if constexpr (NF > 0) F0 = F1;
@@ -714,7 +780,6 @@ __device__ __forceinline__ bool sweep(const PR &P, const Geom &g, NaRing<K, C> &
         // visible to the other lanes of the wave.
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const int lane = (int)(threadIdx.x & 63u);
         const int js = g.j0 - lane * C;           // first column of the strip
         for (int pr = 0; pr < P.nprobe; ++pr) {
             const int pi = P.probe_i[pr], pj = P.probe_j[pr];
@@ -871,7 +936,11 @@ tm_tb_kernel(const TbParams P)
                 return;
             }
         }
+        // four bodies: most of these tiles need only the row terms or only
+        // the column terms, and few the source, probe and TF/SF ones
         if (!brow && !sp) sweep<K, C, LOSSY, PML, VEC, false, true, false, NF, NF == 0>(P, g, ring);
+        else if (!bcol && !sp) sweep<K, C, LOSSY, PML, VEC, true, false, false, NF, NF == 0>(P, g, ring);
+        else if (!sp) sweep<K, C, LOSSY, PML, VEC, true, true, false, NF, NF == 0>(P, g, ring);
         else sweep<K, C, LOSSY, PML, VEC, true, true, true, NF, NF == 0>(P, g, ring);
     }
 }
@@ -980,15 +1049,17 @@ int launch_kv(const TbParams &p_in, bool lossy, bool pml, hipStream_t s)
         // instantiation that carries the planes (nf = 0: none are read or
         // written); the others have no TF/SF code at all, so the waits of
         // their source and probe tiles stay counted
-        if (!pml || p.nf > TB_MAX_FREQ)
-            return fail("fused plane wave / running DFT: PML form and at most %d frequencies",
-                        TB_MAX_FREQ);
-        if (lossy)
-            hipLaunchKernelGGL((tm_tb_kernel<K, C, true, true, VEC, TB_WHOLE, TB_MAX_FREQ>), grid,
-                               dim3(64), 0, s, p);
-        else
-            hipLaunchKernelGGL((tm_tb_kernel<K, C, false, true, VEC, TB_WHOLE, TB_MAX_FREQ>), grid,
-                               dim3(64), 0, s, p);
+        if (!pml || p.nf > TB_MAX_FREQ || K > TB_MAX_TFSF_DEPTH)
+            return fail("fused plane wave / running DFT: PML form, at most %d frequencies and %d "
+                        "steps a launch", TB_MAX_FREQ, TB_MAX_TFSF_DEPTH);
+        if constexpr (K <= TB_MAX_TFSF_DEPTH) {
+            if (lossy)
+                hipLaunchKernelGGL((tm_tb_kernel<K, C, true, true, VEC, TB_WHOLE, TB_MAX_FREQ>),
+                                   grid, dim3(64), 0, s, p);
+            else
+                hipLaunchKernelGGL((tm_tb_kernel<K, C, false, true, VEC, TB_WHOLE, TB_MAX_FREQ>),
+                                   grid, dim3(64), 0, s, p);
+        }
         return hip_check(hipGetLastError(), "fd2d_tm_run launch");
     }
     if (lossy && pml) hipLaunchKernelGGL((tm_tb_kernel<K, C, true, true, VEC, TB_WHOLE>), grid, dim3(64), 0, s, p);
@@ -1070,6 +1141,7 @@ struct BatchParams {
     static constexpr int tf_npml = 0, inc_t0 = 0, inc_stride = 0;
     static constexpr const float *inc = nullptr;
     static constexpr int nf = 0;
+    static constexpr bool one_sp = true;
 };
 
 // A persistent kernel over a work list of (grid, strip, row block) units of
@@ -1164,7 +1236,8 @@ tm_tb_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ 
             else sweep<K, C, true, true, VEC, false, false, false, 0, true, C == 1>(P, g, ring);
         } else {
             if (vac.mode == 1 && threadIdx.x == 0) vac.work[u] = vac.tag;
-            sweep<K, C, true, true, VEC, true, true, true, 0, true>(P, g, ring);
+            if (!sp) sweep<K, C, true, true, VEC, true, true, false, 0, true>(P, g, ring);
+            else sweep<K, C, true, true, VEC, true, true, true, 0, true>(P, g, ring);
         }
     }
 }

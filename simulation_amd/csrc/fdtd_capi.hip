@@ -1095,7 +1095,7 @@ static int tfsf_fused(const fd2d_tm_desc *d, const fd2d_tfsf_desc *b, int t0, in
         int h;
         tm_defaults(d->nx, &dd.depth, &h);
     }
-    if (dd.depth > 8) dd.depth = 8;
+    if (dd.depth > TB_MAX_TFSF_DEPTH) dd.depth = TB_MAX_TFSF_DEPTH;
     if (b->nf && !dd.rows) {
         const int h = d->nx / 220;
         dd.rows = h < 4 ? 4 : (h > 512 ? 512 : h);

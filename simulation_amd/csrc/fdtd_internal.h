@@ -71,12 +71,14 @@ struct CylList {
 constexpr int TB_MAX_DEPTH = 12;    // temporally blocked launches: steps per launch
 constexpr int MW_MAX_DEPTH = 8;     // multi-wave form: steps per launch
 constexpr int LBC_MAX_DEPTH = 10;   // learned boundary: steps per launch (frame tables, LDS)
+constexpr int TB_MAX_TFSF_DEPTH = 8;    // plane-wave launches: steps per launch
 constexpr int TB_MAX_FREQ = 3;      // fused running DFT: frequencies
 constexpr int TB_MAX_LIST_RB = 64;  // boundary launch: whole row blocks listed
 constexpr int TB_MAX_LIST_SX = 64;  // boundary launch: whole strips listed
 constexpr int TB_MAX_LIST_T = 128;  // boundary launch: single tiles listed
 
 struct TbParams {
+    static constexpr bool one_sp = false;   // lists of sources and probes
     int nx, ny;
     const float *dz_i, *iz_i, *hx_i, *hy_i, *ihx_i, *ihy_i;
     float *dz_o, *iz_o, *hx_o, *hy_o, *ihx_o, *ihy_o, *ez_o;

@@ -11,6 +11,7 @@
 #include <math.h>
 
 #include "fdtd_internal.h"
+#include "lanes.h"
 
 namespace fdtd {
 namespace {
@@ -100,161 +101,254 @@ __global__ void __launch_bounds__(256) debye_kernel(int nx, float dt, float chi,
     }
 }
 
-// Fused run: each workgroup owns DF_W cells and evolves, for K <= DF_MAXK
-// steps, the region of its cells widened by K on both sides (one step moves
-// information one cell each way: dx[i] takes hy[i-1], hy[i] takes ex[i+1]),
-// so its own cells are exact after K steps.  ex and hy sit in LDS (the only
-// fields read across cells), the rest in registers; per step two barriers.
-// Reads one state set and writes the other (dx ix sx ex hy bc: a block near
-// the right edge may simulate the boundary it does not own); the DFT planes
-// and the incident-probe DFT are updated in place by their single owner.
+// Fused run, as the blocked run of fd1d.hip: a wavefront holds 64 cells, one a
+// lane, with every field and coefficient in registers and its neighbours'
+// ex, hy by DPP shifts; the waves of a workgroup overlap by twice DF_HALO
+// cells and exchange them through LDS every DF_HALO steps; workgroups overlap
+// by twice the launch's steps.  A launch reads one state set and writes the
+// other (dx ix sx ex hy bc), or works in place when one workgroup holds the
+// grid.  The DFT planes and the incident-probe DFT are updated in place by
+// their single owner: only the waves that own cells carry them (NF > 0).
+// The steps' twiddles and source values go to LDS once a launch.
 // Operands as the per-step kernels above, so the bits are theirs.
-template <int NF>
-__global__ void __launch_bounds__(DF_NT) dform_tb_kernel(const DformTbParams P)
+//
+// What bounds it: instruction issue (14 a cell and step, 26 with three
+// frequencies, two waves a SIMD).  38000 cells, Debye, three frequencies, 1024
+// steps: 1590 us as 32-step launches with the fields in LDS and two barriers a
+// step, 202 us now (218 with each row read when it is used).
+struct SegD {
+    float dx, ix, sx, ex, hy, na, nb, nc, nd;
+    float b0, b1, b2, b3;
+    int lane, rl, sl, pl;
+    unsigned long long pm;
+};
+
+// A step's twiddles and source value, read from LDS a step ahead.
+struct StepRow { float4 a, b; };
+
+__device__ __forceinline__ StepRow step_row(const float *tab, int s)
 {
-    constexpr int CPT = (DF_W + 2 * DF_MAXK + DF_NT - 1) / DF_NT;
-    __shared__ float ex_s[DF_W + 2 * DF_MAXK], hy_s[DF_W + 2 * DF_MAXK];
-    const int nx = P.nx, K = P.K, tid = threadIdx.x;
-    const int o0 = blockIdx.x * DF_W, o1 = min(o0 + DF_W, nx);
-    const int r0 = max(o0 - K, 0), r1 = min(o1 + K, nx), R = r1 - r0;
-    const bool debye = P.ncx != nullptr;
-    const bool left_abc = r0 == 0, right_abc = r1 == nx;   // the region holds that grid edge
-    float dx[CPT], ix[CPT], sx[CPT], na[CPT], nb[CPT], nc[CPT], nd[CPT];
-    float fr[CPT][NF ? NF : 1], fi[CPT][NF ? NF : 1];
-    float b0 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;          // bc of the edge cells' threads
-    float rin[NF ? NF : 1], iin[NF ? NF : 1];
+    const float4 *t = reinterpret_cast<const float4 *>(tab + 8 * s);
+    return StepRow{t[0], t[1]};
+}
+
+template <bool DEBYE, bool L, bool R, bool SP, int NF>
+__device__ __forceinline__ void dform_step(SegD &g, const DformTbParams &P, const StepRow &row, int s,
+                                           int pk, int st, bool inc, float (&fr)[NF ? NF : 1],
+                                           float (&fi)[NF ? NF : 1], float (&rin)[NF ? NF : 1],
+                                           float (&iin)[NF ? NF : 1], float &tr, float *out)
+{
+    float d = g.dx + 0.5f * (lane_left(g.hy) - g.hy);
+    const float c[3] = {row.a.x, row.a.z, row.b.x}, sn[3] = {row.a.y, row.a.w, row.b.y};
+    if (SP) {
+        const float u = d + row.b.z;
+        d = g.lane == g.sl ? u : d;
+    }
+    float e, ix, sx = g.sx;
+    if (DEBYE) {
+        e = g.na * (d - g.ix - g.nc * g.sx);
+        ix = g.ix + g.nb * e;
+        sx = g.nc * g.sx + g.nd * e;
+    } else {
+        e = g.na * (d - g.ix);
+        ix = g.ix + g.nb * e;
+    }
+    if (L) {                                       // cell 0: no update
+        const bool z = g.lane == 0;
+        d = z ? g.dx : d;
+        ix = z ? g.ix : ix;
+        sx = z ? g.sx : sx;
+        e = z ? g.ex : e;
+    }
+    g.dx = d;
+    g.ix = ix;
+    g.sx = sx;
 #pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * DF_NT, i = r0 + j;
-        dx[c] = ix[c] = sx[c] = na[c] = nb[c] = nc[c] = nd[c] = 0.f;
+    for (int f = 0; f < NF; ++f) {
+        fr[f] = fr[f] + c[f] * e;
+        fi[f] = fi[f] - sn[f] * e;
+    }
+    if (SP && NF > 0 && inc) {
 #pragma unroll
-        for (int f = 0; f < (NF ? NF : 1); ++f) { fr[c][f] = 0.f; fi[c][f] = 0.f; }
-        if (j < R) {
-            dx[c] = P.dx_i[i]; ix[c] = P.ix_i[i];
-            na[c] = P.nax[i]; nb[c] = P.nbx[i];
-            if (debye) { sx[c] = P.sx_i[i]; nc[c] = P.ncx[i]; nd[c] = P.ndx[i]; }
-            ex_s[j] = P.ex_i[i];
-            hy_s[j] = P.hy_i[i];
-            if (i >= o0 && i < o1) {
-#pragma unroll
-                for (int f = 0; f < NF; ++f)
-                    if (f < P.nf) {
-                        fr[c][f] = P.r_pt[(long)f * nx + i];
-                        fi[c][f] = P.i_pt[(long)f * nx + i];
-                    }
-            }
-            if (i == 0 && left_abc) { b0 = P.bc_i[0]; b1 = P.bc_i[1]; }
-            if (i == nx - 2 && right_abc) { b2 = P.bc_i[2]; b3 = P.bc_i[3]; }
+        for (int f = 0; f < NF; ++f) {
+            rin[f] = rin[f] + c[f] * e;
+            iin[f] = iin[f] - sn[f] * e;
         }
     }
-    const bool own_inc = NF > 0 && P.r_in && o0 <= DF_INC_PROBE && DF_INC_PROBE < o1;
-#pragma unroll
-    for (int f = 0; f < (NF ? NF : 1); ++f) { rin[f] = 0.f; iin[f] = 0.f; }
-    if (own_inc && DF_INC_PROBE - r0 >= 0 && (DF_INC_PROBE - r0) % DF_NT == tid) {
-#pragma unroll
-        for (int f = 0; f < NF; ++f)
-            if (f < P.nf) { rin[f] = P.r_in[f]; iin[f] = P.i_in[f]; }
+    const float e1 = L ? lane_right(e) : 0.f, e2 = R ? lane_left(e) : 0.f;
+    if (L) {
+        e = g.lane == 0 ? g.b0 : e;
+        g.b0 = g.b1;
+        g.b1 = e1;
     }
+    if (R) {
+        e = g.lane == g.rl ? g.b3 : e;
+        g.b3 = g.b2;
+        g.b2 = e2;
+    }
+    g.ex = e;
+    if (SP && g.pm) {
+        const float x = lane_get(e, g.pl);
+        tr = g.lane == s ? x : tr;
+        for (unsigned long long m = g.pm & (g.pm - 1); m; m &= m - 1) {
+            const int p = __builtin_ctzll(m);
+            if (g.lane == __builtin_amdgcn_readlane(pk, p) - st) out[(long)p * P.probe_len + s] = e;
+        }
+    }
+    const float w = g.hy + 0.5f * (e - lane_right(e));
+    g.hy = R && g.lane == g.rl ? g.hy : w;         // cell nx-1: no update
+}
+
+template <bool DEBYE, bool L, bool R, bool SP, int NF>
+__device__ __forceinline__ void dform_steps(SegD &g, const DformTbParams &P, const float *tab,
+                                            float *xch, int pk, int st, int i, int w0, int w1,
+                                            bool many, bool mine)
+{
+    float fr[NF ? NF : 1], fi[NF ? NF : 1], rin[NF ? NF : 1], iin[NF ? NF : 1];
+    const bool own = i >= w0 && i < w1;
+    const bool inc = SP && NF > 0 && P.r_in && DF_INC_PROBE >= w0 && DF_INC_PROBE < w1;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        fr[f] = own ? P.r_pt[(long)f * P.nx + i] : 0.f;
+        fi[f] = own ? P.i_pt[(long)f * P.nx + i] : 0.f;
+        rin[f] = inc ? P.r_in[f] : 0.f;
+        iin[f] = inc ? P.i_in[f] : 0.f;
+    }
+    const int pf = g.pm ? __builtin_ctzll(g.pm) : 0;
+    int flip = 5 * P.region;
+    const int chunk = many ? DF_HALO : 64;
+    for (int done = 0; done < P.K;) {
+        const int n = min(chunk, P.K - done);
+        float tr = 0.f;
+        float *out = P.probe_out + (P.t_first - 1 + done);
+        const float *row = tab + 8 * done;
+        int s = 0;
+        StepRow r0 = step_row(row, 0), r1;
+        // unrolled by hand: the compiler does not unroll loops with lane shifts
+#pragma unroll 1
+        for (; s + 4 <= n; s += 4) {
+            r1 = step_row(row, s + 1);
+            dform_step<DEBYE, L, R, SP, NF>(g, P, r0, s, pk, st, inc, fr, fi, rin, iin, tr, out);
+            r0 = step_row(row, s + 2);
+            dform_step<DEBYE, L, R, SP, NF>(g, P, r1, s + 1, pk, st, inc, fr, fi, rin, iin, tr, out);
+            r1 = step_row(row, s + 3);
+            dform_step<DEBYE, L, R, SP, NF>(g, P, r0, s + 2, pk, st, inc, fr, fi, rin, iin, tr, out);
+            r0 = step_row(row, s + 4);
+            dform_step<DEBYE, L, R, SP, NF>(g, P, r1, s + 3, pk, st, inc, fr, fi, rin, iin, tr, out);
+        }
+#pragma unroll 1
+        for (; s < n; ++s) {
+            r1 = step_row(row, s + 1);
+            dform_step<DEBYE, L, R, SP, NF>(g, P, r0, s, pk, st, inc, fr, fi, rin, iin, tr, out);
+            r0 = r1;
+        }
+        if (SP && g.pm && g.lane < n) out[(long)pf * P.probe_len + g.lane] = tr;
+        done += n;
+        if (many && done < P.K) {
+            if (mine) {
+                xch[0] = g.dx;
+                xch[P.region] = g.ix;
+                if (DEBYE) xch[2 * P.region] = g.sx;
+                xch[3 * P.region] = g.ex;
+                xch[4 * P.region] = g.hy;
+            }
+            __syncthreads();
+            if (!mine) {
+                g.dx = xch[0];
+                g.ix = xch[P.region];
+                if (DEBYE) g.sx = xch[2 * P.region];
+                g.ex = xch[3 * P.region];
+                g.hy = xch[4 * P.region];
+            }
+            xch += flip;
+            flip = -flip;
+        }
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+        if (own) {
+            P.r_pt[(long)f * P.nx + i] = fr[f];
+            P.i_pt[(long)f * P.nx + i] = fi[f];
+        }
+        if (inc && i == DF_INC_PROBE) {
+            P.r_in[f] = rin[f];
+            P.i_in[f] = iin[f];
+        }
+    }
+}
+
+template <bool DEBYE, int NF>
+__global__ void __launch_bounds__(64 * DF_WAVES) dform_tb_kernel(const DformTbParams P)
+{
+    extern __shared__ __align__(16) float sm[];    // steps' table, then the exchange buffers
+    const int nx = P.nx, lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nw = blockDim.x >> 6;
+    const int wg = blockIdx.x;
+    const bool last = wg == (int)gridDim.x - 1;
+    constexpr int stride = 64 - 2 * DF_HALO;
+    const int o0 = wg * P.own, o1 = last ? nx : o0 + P.own;
+    const int g0 = max(0, min(o0 - P.depth, nx - P.region));
+    const int st = g0 + max(0, min(wv * stride, P.region - 64));
+    const int st1 = g0 + max(0, min((wv + 1) * stride, P.region - 64));
+    const int i = st + lane;
+    const int p0 = wv ? st + DF_HALO : st, p1 = wv + 1 < nw ? st1 + DF_HALO : g0 + P.region;
+    const int w0 = max(p0, o0), w1 = min(p1, o1);
+    for (int k = threadIdx.x; k < 8 * P.K; k += blockDim.x) sm[k] = P.tab[k / 8][k % 8];
+    SegD g;
+    g.lane = lane;
+    const bool in = i < nx;
+    g.dx = in ? P.dx_i[i] : 0.f;
+    g.ix = in ? P.ix_i[i] : 0.f;
+    g.ex = in ? P.ex_i[i] : 0.f;
+    g.hy = in ? P.hy_i[i] : 0.f;
+    g.na = in ? P.nax[i] : 0.f;
+    g.nb = in ? P.nbx[i] : 0.f;
+    g.sx = DEBYE && in ? P.sx_i[i] : 0.f;
+    g.nc = DEBYE && in ? P.ncx[i] : 0.f;
+    g.nd = DEBYE && in ? P.ndx[i] : 0.f;
+    const bool left = st == 0, right = st + 64 >= nx;
+    g.rl = nx - 1 - st;
+    g.b0 = g.b1 = g.b2 = g.b3 = 0.f;
+    if (left) { g.b0 = P.bc_i[0]; g.b1 = P.bc_i[1]; }
+    if (right) { g.b2 = P.bc_i[2]; g.b3 = P.bc_i[3]; }
+    g.sl = P.src_pos - st;
+    const bool src = P.src_pos >= 1 && g.sl >= 0 && g.sl < 64;
+    if (!src) g.sl = -1;
+    const int pk = lane < P.nprobe ? P.probe_k[lane] : -1;
+    g.pm = __builtin_amdgcn_ballot_w64(pk >= w0 && pk < w1);
+    g.pl = (__builtin_amdgcn_readlane(pk, g.pm ? __builtin_ctzll(g.pm) : 0) - st) & 63;
+    const bool inc = NF > 0 && P.r_in && DF_INC_PROBE >= w0 && DF_INC_PROBE < w1;
+    const bool sp = src || g.pm || inc;
+    const bool own = w0 < w1;                      // the wave carries DFT planes
+    const bool many = nw > 1, mine = i >= p0 && i < p1;
+    float *xch = sm + 8 * (DF_MAXK + 1) + (i - g0);
     __syncthreads();
-    for (int s = 0; s < K; ++s) {
-        // D update, source, E update, DFT (ex of every cell after the E update)
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) {
-            const int j = tid + c * DF_NT, i = r0 + j;
-            if (j >= R) continue;
-            if (i >= 1) {
-                const float hl = hy_s[j > 0 ? j - 1 : 0];          // j = 0: a cut (stale)
-                float d = dx[c] + 0.5f * (hl - hy_s[j]);
-                if (i == P.src_pos) d = d + P.src_val[s];
-                dx[c] = d;
-                float e;
-                if (debye) {
-                    const float sv = sx[c];
-                    e = na[c] * (d - ix[c] - nc[c] * sv);
-                    ix[c] = ix[c] + nb[c] * e;
-                    sx[c] = nc[c] * sv + nd[c] * e;
-                } else {
-                    e = na[c] * (d - ix[c]);
-                    ix[c] = ix[c] + nb[c] * e;
-                }
-                ex_s[j] = e;
-            }
-            const float ev = ex_s[j];
-#pragma unroll
-            for (int f = 0; f < NF; ++f)
-                if (f < P.nf) {
-                    fr[c][f] = fr[c][f] + P.tw_c[s][f] * ev;
-                    fi[c][f] = fi[c][f] - P.tw_s[s][f] * ev;
-                }
-            if (own_inc && i == DF_INC_PROBE) {
-#pragma unroll
-                for (int f = 0; f < NF; ++f)
-                    if (f < P.nf) {
-                        rin[f] = rin[f] + P.tw_c[s][f] * ev;
-                        iin[f] = iin[f] - P.tw_s[s][f] * ev;
-                    }
-            }
-        }
-        __syncthreads();
-        // two-step boundary at the grid edges, H update, probes
-#pragma unroll
-        for (int c = 0; c < CPT; ++c) {
-            const int j = tid + c * DF_NT, i = r0 + j;
-            if (j >= R || i >= nx - 1) continue;
-            float e0 = ex_s[j];
-            float e1 = ex_s[j + 1 < R ? j + 1 : j];                // the right cut (stale)
-            if (i == 0 && left_abc) {
-                const float ob0 = b0;
-                ex_s[0] = ob0;
-                b0 = b1;
-                b1 = e1;
-                e0 = ob0;
-            }
-            if (i == nx - 2 && right_abc) {
-                const float ob3 = b3;
-                ex_s[j + 1] = ob3;
-                b3 = b2;
-                b2 = e0;
-                e1 = ob3;
-            }
-            hy_s[j] = hy_s[j] + 0.5f * (e0 - e1);
-            if (i >= o0 && i < o1) {
-                for (int p = 0; p < P.nprobe; ++p)
-                    if (P.probe_k[p] == i)
-                        P.probe_out[(long)p * P.probe_len + (P.t_first - 1 + s)] = e0;
-            }
-            if (i == nx - 2 && right_abc && nx - 1 >= o0 && nx - 1 < o1) {
-                for (int p = 0; p < P.nprobe; ++p)
-                    if (P.probe_k[p] == nx - 1)
-                        P.probe_out[(long)p * P.probe_len + (P.t_first - 1 + s)] = e1;
-            }
-        }
-        __syncthreads();
+    // every wave passes the same number of barriers (P.K decides)
+#define DFORM_RUN(l, r, x, nf) \
+    dform_steps<DEBYE, l, r, x, nf>(g, P, sm, xch, pk, st, i, w0, w1, many, mine)
+    if (left || right) {
+        if (left && right) DFORM_RUN(true, true, true, NF);
+        else if (left) DFORM_RUN(true, false, true, NF);
+        else DFORM_RUN(false, true, true, NF);
+    } else if (sp) {
+        DFORM_RUN(false, false, true, NF);
+    } else if (NF > 0 && own) {
+        DFORM_RUN(false, false, false, NF);
+    } else {
+        DFORM_RUN(false, false, false, 0);
     }
-    // the owned cells go out
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-        const int j = tid + c * DF_NT, i = r0 + j;
-        if (j >= R || i < o0 || i >= o1) continue;
-        P.dx_o[i] = dx[c];
-        P.ix_o[i] = ix[c];
-        if (debye) P.sx_o[i] = sx[c];
-        P.ex_o[i] = ex_s[j];
-        P.hy_o[i] = hy_s[j];
-#pragma unroll
-        for (int f = 0; f < NF; ++f)
-            if (f < P.nf) {
-                P.r_pt[(long)f * nx + i] = fr[c][f];
-                P.i_pt[(long)f * nx + i] = fi[c][f];
-            }
-        if (i == 0) { P.bc_o[0] = b0; P.bc_o[1] = b1; }
-        if (i == nx - 2) { P.bc_o[2] = b2; P.bc_o[3] = b3; }
-        if (own_inc && i == DF_INC_PROBE) {
-#pragma unroll
-            for (int f = 0; f < NF; ++f)
-                if (f < P.nf) { P.r_in[f] = rin[f]; P.i_in[f] = iin[f]; }
-        }
+#undef DFORM_RUN
+    // in place: every wave has read its cells before any are written
+    if (many) __syncthreads();
+    if (i >= w0 && i < w1) {
+        P.dx_o[i] = g.dx;
+        P.ix_o[i] = g.ix;
+        if (DEBYE) P.sx_o[i] = g.sx;
+        P.ex_o[i] = g.ex;
+        P.hy_o[i] = g.hy;
     }
+    if (wg == 0 && left && lane == 0) { P.bc_o[0] = g.b0; P.bc_o[1] = g.b1; }
+    if (last && right && lane == g.rl) { P.bc_o[2] = g.b2; P.bc_o[3] = g.b3; }
 }
 
 inline int nblk(long n) { return (int)((n + 255) / 256); }
@@ -303,12 +397,23 @@ int launch_debye(int nx, float dt, float chi, float tau, float epsr, float sigma
     return hip_check(hipGetLastError(), "dielectric (Debye)");
 }
 
-int launch_dform_tb(const DformTbParams &p, hipStream_t s)
+template <bool DEBYE>
+static int launch_dform_nf(const DformTbParams &p, int groups, int waves, hipStream_t s)
 {
-    const dim3 grid((p.nx + DF_W - 1) / DF_W);
-    if (p.nf) hipLaunchKernelGGL(dform_tb_kernel<DF_NF>, grid, dim3(DF_NT), 0, s, p);
-    else hipLaunchKernelGGL(dform_tb_kernel<0>, grid, dim3(DF_NT), 0, s, p);
+    const size_t lds = sizeof(float) * (8 * (DF_MAXK + 1) + (waves > 1 ? 10 * (size_t)p.region : 0));
+    const dim3 grid(groups), nt(64 * waves);
+    switch (p.nf) {
+    case 0: hipLaunchKernelGGL((dform_tb_kernel<DEBYE, 0>), grid, nt, lds, s, p); break;
+    case 1: hipLaunchKernelGGL((dform_tb_kernel<DEBYE, 1>), grid, nt, lds, s, p); break;
+    case 2: hipLaunchKernelGGL((dform_tb_kernel<DEBYE, 2>), grid, nt, lds, s, p); break;
+    default: hipLaunchKernelGGL((dform_tb_kernel<DEBYE, 3>), grid, nt, lds, s, p); break;
+    }
     return hip_check(hipGetLastError(), "fd1d_dform_run launch");
+}
+
+int launch_dform_tb(const DformTbParams &p, int groups, int waves, hipStream_t s)
+{
+    return p.ncx ? launch_dform_nf<true>(p, groups, waves, s) : launch_dform_nf<false>(p, groups, waves, s);
 }
 
 }  // namespace fdtd

@@ -887,40 +887,55 @@ size_t fd1d_dform_work_elems(int nx)
     return nx < 1 ? 0 : 5 * (size_t)nx + 4;
 }
 
-// The fused D/E-form run: an even number L of launches of up to DF_MAXK
-// steps, ping-ponging between the caller's state set and the partner set in
-// work (so the result ends in the caller's arrays).
+// The fused D/E-form run.  A grid one workgroup holds runs in place; a larger
+// one takes an even number L of launches between the caller's state set and
+// the partner set in work, so the result ends in the caller's arrays.  A
+// launch costs about as much as 50 steps: as deep as the region allows with
+// 64 cells owned, and with no more workgroups than CUs (256) while half the
+// region suffices for that.
 static int dform_fused(const fd1d_dform_desc *d, int t0, int nsteps, hipStream_t s)
 {
     const int nx = d->nx;
-    int L = (nsteps + DF_MAXK - 1) / DF_MAXK;
-    L += L % 2;
+    const bool one = nx <= DF_REGION;
+    int own = (nx + 255) / 256;
+    own = own < 64 ? 64 : (own > DF_REGION / 2 ? DF_REGION / 2 : own);
+    const int kmax = one ? DF_MAXK : std::min(DF_MAXK, (DF_REGION - own) / 2);
+    int L = (nsteps + kmax - 1) / kmax;
+    if (!one) L += L % 2;
     float *w = d->work;
     float *A[6] = {d->dx, d->ix, d->sx, d->ex, d->hy, d->bc};
     float *B[6] = {w, w + nx, w + 2 * (size_t)nx, w + 3 * (size_t)nx, w + 4 * (size_t)nx,
                    w + 5 * (size_t)nx};
+    DformTbParams p{};
+    p.nx = nx;
+    p.region = one ? std::max(nx, 64) : DF_REGION;
+    p.depth = one ? 0 : nsteps / L + (nsteps % L ? 1 : 0);
+    p.own = one ? nx : p.region - 2 * p.depth;
+    const int groups = (nx + p.own - 1) / p.own;
+    constexpr int stride = 64 - 2 * DF_HALO;
+    const int waves = (p.region - 64 + stride - 1) / stride + 1;
+    p.nax = d->md.nax; p.nbx = d->md.nbx; p.ncx = d->md.ncx; p.ndx = d->md.ndx;
+    p.src_pos = d->src_pos >= 1 ? d->src_pos : -1;
+    p.nf = d->nf;
+    p.r_pt = d->ft.r_pt; p.i_pt = d->ft.i_pt; p.r_in = d->ft.r_in; p.i_in = d->ft.i_in;
+    p.nprobe = d->nprobe;
+    for (int q = 0; q < d->nprobe; ++q) p.probe_k[q] = d->probe_k[q];
+    p.probe_out = d->probe_out; p.probe_len = d->probe_len;
     int done = 0;
     for (int l = 0; l < L; ++l) {
         const int k = nsteps / L + (l < nsteps % L ? 1 : 0);
-        float **in = (l % 2 == 0) ? A : B;
-        float **out = (l % 2 == 0) ? B : A;
-        DformTbParams p{};
-        p.nx = nx; p.t_first = t0 + done + 1; p.K = k;
+        float **in = (one || l % 2 == 0) ? A : B;
+        float **out = (one || l % 2) ? A : B;
+        p.t_first = t0 + done + 1; p.K = k;
         p.dx_i = in[0]; p.ix_i = in[1]; p.sx_i = in[2]; p.ex_i = in[3]; p.hy_i = in[4]; p.bc_i = in[5];
         p.dx_o = out[0]; p.ix_o = out[1]; p.sx_o = out[2]; p.ex_o = out[3]; p.hy_o = out[4]; p.bc_o = out[5];
-        p.nax = d->md.nax; p.nbx = d->md.nbx; p.ncx = d->md.ncx; p.ndx = d->md.ndx;
-        p.src_pos = d->src_pos >= 1 ? d->src_pos : -1;
-        p.nf = d->nf;
-        p.r_pt = d->ft.r_pt; p.i_pt = d->ft.i_pt; p.r_in = d->ft.r_in; p.i_in = d->ft.i_in;
         for (int q = 0; q < k; ++q) {
             const int t = p.t_first + q;
-            p.src_val[q] = p.src_pos >= 1 ? d->src_wave[t - 1] : 0.0f;
-            for (int f = 0; f < d->nf; ++f) dft_twiddle(t, d->freq[f], d->dt, &p.tw_c[q][f], &p.tw_s[q][f]);
+            p.tab[q][2 * DF_NF] = p.src_pos >= 1 ? d->src_wave[t - 1] : 0.0f;
+            for (int f = 0; f < d->nf; ++f)
+                dft_twiddle(t, d->freq[f], d->dt, &p.tab[q][2 * f], &p.tab[q][2 * f + 1]);
         }
-        p.nprobe = d->nprobe;
-        for (int q = 0; q < d->nprobe; ++q) p.probe_k[q] = d->probe_k[q];
-        p.probe_out = d->probe_out; p.probe_len = d->probe_len;
-        int rc = launch_dform_tb(p, s);
+        int rc = launch_dform_tb(p, groups, waves, s);
         if (rc) return rc;
         done += k;
     }

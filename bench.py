@@ -533,17 +533,18 @@ def bench_tfsf(a):
                                f"cylinder r={rgrid} eps_r=30 sigma=0.3, DFT at 3 frequencies "
                                f"(fd2d/clang/test_3_4.c)", "grid": [n, n], "npml": npml,
                    "freq": list(freq),
-                   # with DFT planes the fused run defaults to depth 4 and
-                   # rows max(4, n/220); without, to the plain TM plan
-                   "depth": s.tm.depth or (4 if len(freq) else s.tm.plan(K)["depth"]),
-                   "rows": s.tm.rows or (max(4, min(512, n // 220)) if len(freq)
-                                         else s.tm.plan(K)["rows"]),
+                   # the fused run's defaults: register tiles of 32 rows,
+                   # depth 8 (12 while the tiles fit one a CU); strips from 17
+                   # million cells on: with DFT planes depth 4 and rows
+                   # max(4, n/220)
+                   "depth": s.tm.depth or (8 if n * n <= 17000000 else 4),
+                   "rows": s.tm.rows or (32 if n * n <= 17000000 else max(4, min(512, n // 220))),
                    "cols": s.tm.cols or 1,
                    "per_step_kernels_value": round(per_step, 1)},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 4), "traffic": None,
-                     "kernel": "fused fd2d_tfsf_run, effective per step (tm_tb_kernel "
-                               "with TF/SF + DFT, both parts, and the incident chunk)",
+                     "kernel": "fused fd2d_tfsf_run, effective per step (tm_rt_kernel "
+                               "with TF/SF + DFT, and the incident chunk)",
                      "avg_launch_ms": round(step_ms, 4), "alg_bytes_per_launch": b_alg * n * n},
         "cpu_baseline": cpu,
     }

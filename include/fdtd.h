@@ -307,7 +307,9 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream);
 
 /* The launch plan fd2d_tm_run would use for this descriptor and nsteps:
  * number of launches and the chosen depth/rows/cols.  Defaults (measured on
- * MI355X): one column per lane; depth 10 from nx = 2048 on, else 8; rows =
+ * MI355X): with form, depth, rows and cols all 0, grids of up to 2.7 million
+ * cells run register tiles of `rows` rows (32 or 48; depth 7 to 14 by the
+ * number of tiles); otherwise strips of one column per lane; depth 10 from nx = 2048 on, else 8; rows =
  * nx/128 for 4096 <= nx < 12288, else nx/170, clamped to [8, 512]; the
  * multi-wave form: depth 8, rows = nx/32 clamped to [32, 512].  Depths go up
  * to 12.  Host only.                                                       */

@@ -30,9 +30,12 @@ def candidates(nx: int):
     nx/170, nx/128 and nx/96 rows and at depth 8 with nx/128 (MI355X sweeps
     put the optimum at depth 10 at 2048^2 and depth 11 from 4096^2 on, rows
     ~nx/170 at 2048^2 and ~nx/128 from 4096^2 on), two columns per lane at
-    depth 8, and the multi-wave form with short blocks."""
+    depth 8, and the multi-wave form with short blocks; below 2048 rows also
+    the library's own choice (register tiles up to 2.7 million cells)."""
     def r(d):
         return min(512, max(8, nx // d))
+    if nx < 2048:
+        yield 0, 0, 0, 0
     for depth in ((10, 11) if nx >= 4096 else (10,)):
         for rows in sorted({r(170), r(128), r(96)}):
             yield depth, rows, 1, 1
@@ -92,7 +95,7 @@ def tune(solver: fd2d.TMSolver, steps: int = 80, use_cache: bool = True, configs
     """Time (depth, rows, cols[, form]) candidates on this solver's grid and
     set the fastest on it.  The solver's state, probe traces and step are
     restored."""
-    key = (f"tm2|{_device()}|{solver.nx}x{solver.ny}|lossy={int(solver.lossy)}"
+    key = (f"tm3|{_device()}|{solver.nx}x{solver.ny}|lossy={int(solver.lossy)}"
            f"|pml={int(solver.pml is not None)}")
     db = _load() if use_cache and configs is None else {}
     if key in db:
@@ -110,7 +113,8 @@ def tune(solver: fd2d.TMSolver, steps: int = 80, use_cache: bool = True, configs
             # whole pairs of full-depth launches where the run is long enough
             # (a long run's launches are nearly all full depth), else the
             # run's own length
-            n = base - base % (2 * depth) if base >= 2 * depth else base - base % 2
+            pair = 2 * (depth or max(solver.plan(base)["depth"], 1))
+            n = base - base % pair if base >= pair else base - base % 2
 
             def go(n=n):
                 solver.t = 0

@@ -1,0 +1,401 @@
+// fd2d_rt.hip -- fused 2-D TM time stepping of small grids: register tiles
+// (gfx950).
+//
+// One launch advances the grid by K leapfrog steps (K a run-time number).
+// Semantics per step are those of the reference's per-step kernels dfield ->
+// hard source -> efield -> hfield (fd2d/pycuda/fd2d_3_2.py:219-260,
+// fd2d/pycuda/fd2d_3_4.py:175-226 with the plane wave and the running DFT),
+// operand for operand: the bits of tm_tb_kernel (fd2d_tb_impl.h).
+//
+// Why another form.  tm_tb_kernel's wave sweeps a strip row by row through K
+// levels: a launch lasts (rows + 2K) positions of K dependent levels however
+// few tiles there are, and short row blocks recompute 2K warm-up rows each.
+// That pays on grids that fill the chip with tall strips; on a grid of up to
+// some 1600 cells a side it leaves most SIMDs idle or busy with warm-up rows.
+//
+// Here a workgroup of up to 16 waves holds a tile of 64 columns by waves * R
+// rows in registers for the whole launch: a wave has R = 4 rows, one column a
+// lane, every field and coefficient of its cells in VGPRs.  Columns beside a
+// lane's come by DPP shifts, the rows above and below a wave's from LDS (one
+// row of hy down, one row of ez up), so a step costs two barriers and no
+// memory.  Tiles overlap by K cells on either side of the cut they share
+// (recomputed, never written twice).  Waves whose rows have left the cone of
+// the tile's own rows skip the rest of the launch's steps but their barriers.
+// Two rows a wave, 16 waves (the same tile) measured within 6%; eight rows
+// spill and lose on every grid.
+//
+// Two bodies a wave chooses from: rows and columns inside the band of default
+// profile values (constants, no edge tests; the terms 0 * ihx and 0 * ihy
+// left out as in tm_tb_kernel), or the general one.
+//
+// What bounds it: on small grids the step itself (about 0.85 us a step for a
+// 32-row tile at two waves a SIMD: instruction issue, then the two barriers)
+// and some 4 us a launch for the loads, stores and the gap; from 1000^2 on
+// the overlap (a third to a half of the cells computed) and the tiles' loads.
+// MI355X, strips before -> tiles, 192 steps, lossy, npml 8: 100^2 1055 -> 220
+// us, 400^2 1070 -> 274, 700^2 1085 -> 370, 1100^2 1109 -> 676, 1600^2 1181
+// -> 1120.
+#include "fdtd_internal.h"
+#include "lanes.h"
+
+#include <climits>
+
+namespace fdtd {
+namespace {
+
+using gfloat = const __attribute__((address_space(1))) float;
+using cfloat = const __attribute__((address_space(4))) float;
+
+__device__ __forceinline__ float ldg(const float *p, unsigned i) { return ((gfloat *)p)[i]; }
+// a row's profile value: a scalar load (the same index in every lane)
+__device__ __forceinline__ float ldu(const float *p, int i)
+{
+    return ((cfloat *)p)[__builtin_amdgcn_readfirstlane(i)];
+}
+// LDS traffic done, then the barrier (global loads and stores stay in flight)
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <int N> struct Int { static constexpr int v = N; };
+
+constexpr int R = RT_ROWS;
+
+template <bool LOSSY, bool PML, bool TF, int NF>
+__global__ void __launch_bounds__(64 * RT_WAVES) tm_rt_kernel(const RtParams P)
+{
+    __shared__ float up[RT_WAVES + 1][64];   // up[w]: hy of the row above wave w's first
+    __shared__ float dn[RT_WAVES + 1][64];   // dn[w]: ez of wave w's first row
+    __shared__ float srcv[FDTD_MAX_SOURCES * RT_MAX_STEPS];
+
+    const int nx = P.nx, ny = P.ny, K = P.K;
+    const int W = (int)blockDim.x >> 6, T = W * R;
+    const int lane = (int)threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    // workgroup L runs on XCD L % 8: the workgroups of one XCD take a
+    // contiguous run of tiles, which share their halos in its L2
+    const unsigned nt = gridDim.x, xcd = blockIdx.x % 8u, q8 = nt / 8u, rem = nt % 8u;
+    const unsigned tile = xcd * q8 + min(xcd, rem) + blockIdx.x / 8u;
+    const int bx = (int)(tile % (unsigned)P.nsx), by = (int)(tile / (unsigned)P.nsx);
+    const int nsy = (int)(nt / (unsigned)P.nsx);
+    // the tile's window starts at (bi, bj) -- the last one of a row or column
+    // ends with the grid -- and its own cells are rows [o0, o1), columns [c0, c1)
+    const int bi = min(by * (T - 2 * K), max(nx - T, 0));
+    const int bj = min(bx * (64 - 2 * K), max(ny - 64, 0));
+    const int o0 = by ? by * (T - 2 * K) + K : 0, o1 = by == nsy - 1 ? nx : by * (T - 2 * K) + T - K;
+    const int c0 = bx ? bx * (64 - 2 * K) + K : 0, c1 = bx == P.nsx - 1 ? ny : bx * (64 - 2 * K) + 64 - K;
+    const int i0 = bi + w * R, j = bj + lane, jc = min(j, ny - 1);
+    const bool own_col = j >= c0 && j < c1;
+
+    float dz[R], iz[LOSSY ? R : 1], hx[R], hy[R], ax[PML ? R : 1], ay[PML ? R : 1];
+    float na[R], nb[LOSSY ? R : 1], e[R];
+    float fr[NF ? NF : 1][R], fi[NF ? NF : 1][R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const unsigned o = (unsigned)min(i0 + r, nx - 1) * (unsigned)ny + (unsigned)jc;
+        dz[r] = ldg(P.dz_i, o);
+        hx[r] = ldg(P.hx_i, o);
+        hy[r] = ldg(P.hy_i, o);
+        na[r] = ldg(P.naz, o);
+        if constexpr (LOSSY) { iz[r] = ldg(P.iz_i, o); nb[r] = ldg(P.nbz, o); }
+        if constexpr (PML) { ax[r] = ldg(P.ihx_i, o); ay[r] = ldg(P.ihy_i, o); }
+        e[r] = 0.f;
+        if constexpr (NF > 0) {
+            // planes are read and written by the cell's owner alone
+            const bool own = own_col && i0 + r >= o0 && i0 + r < o1;
+            const size_t plane = (size_t)nx * (size_t)ny;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                fr[f][r] = own ? ldg(P.ft_r + f * plane, o) : 0.f;
+                fi[f][r] = own ? ldg(P.ft_i + f * plane, o) : 0.f;
+            }
+        }
+    }
+    // profile values: columns in lanes, rows in scalar registers
+    float gy2 = 1.f, gy3 = 1.f, fy1 = 0.f, fy2 = 1.f, fy3 = 1.f;
+    float gx2[R], gx3[R], fx1[R], fx2[R], fx3[R];
+    if constexpr (PML) {
+        gy2 = ldg(P.pml.gy2, jc); gy3 = ldg(P.pml.gy3, jc);
+        fy1 = ldg(P.pml.fy1, jc); fy2 = ldg(P.pml.fy2, jc); fy3 = ldg(P.pml.fy3, jc);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int i = min(i0 + r, nx - 1);
+            gx2[r] = ldu(P.pml.gx2, i); gx3[r] = ldu(P.pml.gx3, i);
+            fx1[r] = ldu(P.pml.fx1, i); fx2[r] = ldu(P.pml.fx2, i); fx3[r] = ldu(P.pml.fx3, i);
+        }
+    }
+    const bool plain = i0 >= P.rlo && i0 + R <= P.rhi && bj >= P.clo && bj + 64 <= P.chi;
+    const bool rows_own = i0 < o1 && i0 + R > o0;
+
+    // sources and probes of the wave's cells: one a lane (row, column), and
+    // those the wave has as a mask
+    int sp_row = INT_MIN, sp_col = INT_MIN;
+    if (lane < P.nsrc) {
+        sp_row = P.src_i[lane]; sp_col = P.src_j[lane];
+    } else if (lane >= FDTD_MAX_SOURCES && lane < FDTD_MAX_SOURCES + P.nprobe) {
+        sp_row = P.probe_i[lane - FDTD_MAX_SOURCES]; sp_col = P.probe_j[lane - FDTD_MAX_SOURCES];
+    }
+    unsigned long long spm;
+    {
+        const bool in = sp_row >= i0 && sp_row < i0 + R && sp_col >= bj && sp_col < bj + 64;
+        const bool mine = sp_row >= o0 && sp_row < o1 && sp_col >= c0 && sp_col < c1;
+        spm = __builtin_amdgcn_ballot_w64(in && (lane < FDTD_MAX_SOURCES || mine));
+    }
+    const unsigned smask = (unsigned)spm & ((1u << FDTD_MAX_SOURCES) - 1u);
+    const unsigned pmask = (unsigned)(spm >> FDTD_MAX_SOURCES);
+    for (int k = (int)threadIdx.x; k < P.nsrc * K; k += (int)blockDim.x)
+        srcv[k] = P.src_wave[(size_t)(k / K) * P.wave_len + (P.t_first - 1 + k % K)];
+    // plane wave: whether the wave holds cells the TF/SF box corrects; the
+    // step's four column values sit in lanes 0 .. 3, the row values one a
+    // lane, both loaded a step ahead
+    const int m = TF ? P.tf_npml : 0;
+    bool tfw = false;
+    float tfv = 0.f, tfr = 0.f;
+    if constexpr (TF) {
+        auto col_in = [&](int c) { return c >= bj && c < bj + 64; };
+        auto row_in = [&](int i) { return i >= i0 && i < i0 + R; };
+        tfw = i0 + R > m - 2 && i0 <= nx - m &&
+              (col_in(m - 2) || col_in(m - 1) || col_in(ny - m) || row_in(m - 2) || row_in(nx - m));
+    }
+    auto load_tf = [&](int s) __attribute__((always_inline)) {
+        const float *iv = P.inc + (size_t)(P.t_first + s - P.inc_t0 - 1) * P.inc_stride;
+        tfv = ldg(iv, lane < 3 ? lane : 3 + ny - 2 * m);
+        tfr = ldg(iv, (unsigned)(2 + min(max(j, m - 1), ny - m) - (m - 1)));
+    };
+    if (TF && tfw) load_tf(0);
+
+    up[w + 1][lane] = hy[R - 1];
+    if (w == 0) {
+        up[0][lane] = 0.f;
+        dn[W][lane] = 0.f;
+    }
+    lds_barrier();
+
+    const bool colD = j >= 1, colH = j <= ny - 2;
+    // D, source, E of the wave's rows; hu: hy of the row above
+    auto e_phase = [&](auto G, auto SP, int s, float hu) __attribute__((always_inline)) {
+        auto d_row = [&](int r, float hl) __attribute__((always_inline)) {
+            const float hp = r ? hy[r ? r - 1 : 0] : hu;
+            const float curl = hy[r] - hp - hx[r] + hl;
+            if (PML && G.v) dz[r] = gx3[r] * gy3 * dz[r] + gx2[r] * gy2 * 0.5f * curl;
+            else dz[r] = dz[r] + 0.5f * curl;
+        };
+        if (G.v) {
+            // row 0 and column 0 have no update: one region of masked lanes
+            // for all rows (a select per value costs more, and the compiler
+            // makes a branch per row of it); the shifts need every lane
+            float hl[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) hl[r] = lane_left(hx[r]);
+            if (colD) {
+#pragma unroll
+                for (int r = R - 1; r >= 1; --r) d_row(r, hl[r]);
+                if (i0 >= 1) d_row(0, hl[0]);
+            }
+        } else {
+#pragma unroll
+            for (int r = R - 1; r >= 0; --r) d_row(r, lane_left(hx[r]));
+        }
+        if (SP.v) {
+            for (unsigned mk = smask; mk; mk &= mk - 1u) {
+                const int k = __builtin_ctz(mk);
+                const int rk = __builtin_amdgcn_readlane(sp_row, k) - i0;
+                const bool at = j == __builtin_amdgcn_readlane(sp_col, k);
+                const float v = srcv[k * K + s];
+#pragma unroll
+                for (int r = 0; r < R; ++r) dz[r] = at && r == rk ? v : dz[r];
+            }
+            if (TF && tfw) {
+                const float h0 = lane_get(tfv, 0), h1 = lane_get(tfv, 1);
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (i0 + r >= m - 1 && i0 + r <= nx - m) {
+                        if (j == m - 1) dz[r] = dz[r] + 0.5f * h0;
+                        if (j == ny - m) dz[r] = dz[r] - 0.5f * h1;
+                    }
+            }
+        }
+#pragma unroll
+        for (int r = R - 1; r >= 0; --r) {
+            if constexpr (LOSSY) {
+                e[r] = na[r] * (dz[r] - iz[r]);
+                iz[r] = iz[r] + nb[r] * e[r];
+            } else {
+                e[r] = na[r] * dz[r];
+            }
+        }
+        dn[w][lane] = e[0];
+        if constexpr (NF > 0) {
+            if (rows_own) {
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    const float c = P.tw[s][f], sn = P.tw[s][TB_MAX_FREQ + f];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        fr[f][r] = fr[f][r] + c * e[r];
+                        fi[f][r] = fi[f][r] - sn * e[r];
+                    }
+                }
+            }
+        }
+        for (unsigned mk = pmask; mk; mk &= mk - 1u) {
+            const int k = __builtin_ctz(mk);
+            const int rk = __builtin_amdgcn_readlane(sp_row, FDTD_MAX_SOURCES + k) - i0;
+            float v = e[0];
+#pragma unroll
+            for (int r = 1; r < R; ++r) v = r == rk ? e[r] : v;
+            if (j == __builtin_amdgcn_readlane(sp_col, FDTD_MAX_SOURCES + k))
+                P.probe_out[(size_t)k * P.probe_len + (P.t_first + s - 1)] = v;
+        }
+    };
+    // H of the wave's rows; ed: ez of the row below
+    auto h_phase = [&](auto G, auto SP, int s, float ed) __attribute__((always_inline)) {
+        auto h_row = [&](int r, float eR, float heR) __attribute__((always_inline)) {
+            const float ez = e[r], eD = r + 1 < R ? e[r + 1 < R ? r + 1 : 0] : ed;
+            const float he = 0.5f * ez;
+            if (PML && !G.v) {
+                // profile values at their defaults: 0 * ihx and 0 * ihy add
+                // nothing (tm_tb_kernel has the argument)
+                ax[r] = ax[r] + (ez - eR);
+                ay[r] = ay[r] + (ez - eD);
+                hx[r] = hx[r] + (he - heR);
+                hy[r] = hy[r] - (he - 0.5f * eD);
+            } else if constexpr (PML) {
+                ax[r] = ax[r] + (ez - eR);
+                ay[r] = ay[r] + (ez - eD);
+                hx[r] = fy3 * hx[r] + fy2 * (he - 0.5f * eR + fx1[r] * ax[r]);
+                hy[r] = fx3[r] * hy[r] - fx2[r] * (he - 0.5f * eD + fy1 * ay[r]);
+            } else {
+                hx[r] = hx[r] + 0.5f * (ez - eR);
+                hy[r] = hy[r] - 0.5f * (ez - eD);
+            }
+        };
+        if (G.v) {
+            // row nx-1 and column ny-1 have no update
+            float eR[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) eR[r] = lane_right(e[r]);
+            if (colH) {
+                if (i0 + R <= nx - 1) {
+#pragma unroll
+                    for (int r = 0; r < R; ++r) h_row(r, eR[r], 0.f);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < R; ++r)
+                        if (i0 + r <= nx - 2) h_row(r, eR[r], 0.f);
+                }
+            }
+        } else {
+            // 0.5 * (right ez) is the right lane's 0.5 * ez, shifted as it is
+#pragma unroll
+            for (int r = 0; r < R; ++r) h_row(r, lane_right(e[r]), PML ? lane_right(0.5f * e[r]) : 0.f);
+        }
+        if (SP.v && TF && tfw) {
+            const float e0 = lane_get(tfv, 2), e1 = lane_get(tfv, 3);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int i = i0 + r;
+                if (i >= m - 1 && i <= nx - m) {
+                    if (j == m - 2) hx[r] = hx[r] + 0.5f * e0;
+                    if (j == ny - m) hx[r] = hx[r] - 0.5f * e1;
+                }
+                if (i == m - 2 || i == nx - m) {
+                    const float sgn = i == nx - m ? 0.5f : -0.5f;
+                    if (j >= m - 1 && j <= ny - m) hy[r] = hy[r] + sgn * tfr;
+                }
+            }
+            if (s + 1 < K) load_tf(s + 1);
+        }
+        up[w + 1][lane] = hy[R - 1];
+    };
+    const bool sp = smask != 0 || tfw;
+#pragma unroll 1
+    for (int s = 0; s < K; ++s) {
+        // rows a later own cell depends on: K-s on either side of [o0, o1)
+        const bool act = i0 < nx && i0 + R > o0 - (K - s) && i0 < o1 + (K - s);
+        if (act) {
+            const float hu = up[w][lane];
+            if (sp) e_phase(Int<1>{}, Int<1>{}, s, hu);
+            else if (plain) e_phase(Int<0>{}, Int<0>{}, s, hu);
+            else e_phase(Int<1>{}, Int<0>{}, s, hu);
+        }
+        lds_barrier();
+        if (act) {
+            const float ed = dn[w + 1][lane];
+            if (sp) h_phase(Int<1>{}, Int<1>{}, s, ed);
+            else if (plain) h_phase(Int<0>{}, Int<0>{}, s, ed);
+            else h_phase(Int<1>{}, Int<0>{}, s, ed);
+        }
+        lds_barrier();
+    }
+    if (!rows_own || !own_col) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = i0 + r;
+        if (i < o0 || i >= o1) continue;
+        const unsigned o = (unsigned)i * (unsigned)ny + (unsigned)j;
+        P.dz_o[o] = dz[r];
+        P.hx_o[o] = hx[r];
+        P.hy_o[o] = hy[r];
+        if constexpr (LOSSY) P.iz_o[o] = iz[r];
+        if constexpr (PML) { P.ihx_o[o] = ax[r]; P.ihy_o[o] = ay[r]; }
+        if (P.ez_o) P.ez_o[o] = e[r];
+        if constexpr (NF > 0) {
+            const size_t plane = (size_t)nx * (size_t)ny;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                P.ft_r[f * plane + o] = fr[f][r];
+                P.ft_i[f * plane + o] = fi[f][r];
+            }
+        }
+    }
+}
+
+template <bool TF, int NF>
+void launch_form(const RtParams &p, int waves, int tiles, bool lossy, bool pml, hipStream_t s)
+{
+    const dim3 g(tiles), b(64 * waves);
+    if (pml && lossy) hipLaunchKernelGGL((tm_rt_kernel<true, true, TF, NF>), g, b, 0, s, p);
+    else if (pml) hipLaunchKernelGGL((tm_rt_kernel<false, true, TF, NF>), g, b, 0, s, p);
+    else if constexpr (!TF) {
+        if (lossy) hipLaunchKernelGGL((tm_rt_kernel<true, false, false, 0>), g, b, 0, s, p);
+        else hipLaunchKernelGGL((tm_rt_kernel<false, false, false, 0>), g, b, 0, s, p);
+    }
+}
+
+}  // namespace
+
+int rt_tiles(int nx, int ny, int waves, int K)
+{
+    auto along = [K](int n, int span) {
+        return n <= span ? 1 : 1 + (n - span + span - 2 * K - 1) / (span - 2 * K);
+    };
+    return along(nx, waves * R) * along(ny, 64);
+}
+
+int preload_rt()
+{
+    return preload_kernel(reinterpret_cast<const void *>(&tm_rt_kernel<true, true, false, 0>));
+}
+
+int launch_fd2d_rt(const RtParams &p, int waves, int nf, bool lossy, bool pml, hipStream_t s)
+{
+    if (waves < 1 || waves > RT_WAVES || p.K < 1 || p.K > RT_MAX_STEPS || 2 * p.K >= waves * R ||
+        2 * p.K >= 64)
+        return fail("register tiles: %d steps a launch in tiles of %dx64", p.K, waves * R);
+    const bool tf = nf || p.tf_npml;
+    if (tf && !pml) return fail("register tiles: plane wave and DFT take the PML form");
+    RtParams q = p;
+    q.nsx = rt_tiles(1, p.ny, waves, p.K);
+    const int tiles = rt_tiles(p.nx, p.ny, waves, p.K);
+    if (!tf) launch_form<false, 0>(q, waves, tiles, lossy, pml, s);
+    else if (nf == 0) launch_form<true, 0>(q, waves, tiles, lossy, pml, s);
+    else if (nf == 1) launch_form<true, 1>(q, waves, tiles, lossy, pml, s);
+    else if (nf == 2) launch_form<true, 2>(q, waves, tiles, lossy, pml, s);
+    else if (nf == 3) launch_form<true, 3>(q, waves, tiles, lossy, pml, s);
+    else return fail("register tiles: %d frequencies", nf);
+    return hip_check(hipGetLastError(), "register tiles launch");
+}
+
+}  // namespace fdtd

@@ -133,7 +133,58 @@ struct Plan {
     int mw;                // 1: multi-wave form (rows = rows of its interior blocks)
     int frows;             // rows of the single-wave tiles (strips, or the frame of the
                            // multi-wave form)
+    int rt;                // 1: register tiles (depth: steps of a launch, rows: of a tile)
 };
+
+// Register tiles (fd2d_rt.hip), where the caller leaves form, depth, rows and
+// columns to the library and the grid is small enough; tf: a plane-wave run.
+// MI355X, us of 192 steps (lossy, npml 8; strips / tiles of 8, 12, 16 waves
+// at their best depth): 400^2 1070 / 274, 286, 293; 500^2 1089 / 323, 309,
+// 305; 600^2 1080 / 349, 353, 350; 850^2 1108 / 518, 466, 572; 1100^2 1109 /
+// 676, 659, 796; 1400^2 1132 / 908, 913, 1178; 1600^2 1181 / 1098, 1115,
+// 1549; 1531x2047 1254 / 1284, 1312, 1793.  So: while the tiles of 8 waves
+// number at most the 256 CUs, the deepest such launch (4 us a launch against
+// 0.85 us a step); then 12 waves, first one tile a CU, then two; past that 8
+// waves at depth 7, where the overlap costs as much as the launches.  Strips
+// are ahead from about 3 million cells on.
+// Plane waves (strips / tiles of 8 waves, 256 steps, three frequencies):
+// 150^2 2038 / 784 at depth 12, 832 at 8; 400^2 2191 / 953, 863; 1024^2 3413
+// / 2378, 1914; 1500^2 4970 / 3972, 2961; 128 steps: 4096^2 17230 / 9342 with
+// three frequencies, 6990 / 6555 without.
+constexpr long RT_MAX_CELLS = 2700000, RT_MAX_CELLS_TF = 17000000;
+bool plan_rt(const fd2d_tm_desc *d, int nsteps, bool tf, Plan *pl)
+{
+    if (d->form != FDTD_TM_FORM_AUTO || d->depth || d->rows || d->cols || nsteps < 2) return false;
+    if ((long)d->nx * d->ny > (tf ? RT_MAX_CELLS_TF : RT_MAX_CELLS)) return false;
+    auto deepest = [&](int waves, std::initializer_list<int> depths, int most) {
+        for (int k : depths)
+            if (rt_tiles(d->nx, d->ny, waves, k) <= most) return k;
+        return 0;
+    };
+    int W = 8, K;
+    if (tf) {
+        K = deepest(8, {12}, 256);
+        if (!K) K = 8;
+    } else {
+        K = deepest(8, {14, 12, 10, 8}, 256);
+        if (!K) {
+            W = 12;
+            K = deepest(12, {12, 10, 8}, 256);
+            if (!K) K = deepest(12, {12, 10, 8}, 512);
+            if (!K) { W = 8; K = 7; }
+        }
+    }
+    // an even number of launches: the result ends in the caller's state set
+    int L = (nsteps + K - 1) / K;
+    L += L % 2;
+    *pl = Plan{};
+    pl->rt = 1;
+    pl->launches = L;
+    pl->depth = (nsteps + L - 1) / L;
+    pl->rows = W * RT_ROWS;
+    pl->cols = 1;
+    return true;
+}
 
 // Rows of an interior block of the multi-wave form when the caller gives
 // none.
@@ -175,6 +226,8 @@ void tm_defaults(int nx, int *depth, int *rows)
 
 int plan_tm(const fd2d_tm_desc *d, int nsteps, Plan *pl)
 {
+    if (plan_rt(d, nsteps, false, pl)) return 0;
+    pl->rt = 0;
     int D0 = 8, H0 = 16;
     tm_defaults(d->nx, &D0, &H0);
     int D = d->depth ? d->depth : (d->form == FDTD_TM_FORM_MULTIWAVE ? 8 : D0);
@@ -352,6 +405,7 @@ int fdtd_preload(void)
     if (!rc) rc = preload_fd2d();
     if (!rc) rc = preload_tb();
     if (!rc) rc = preload_mw();
+    if (!rc) rc = preload_rt();
     if (!rc) rc = preload_dform1d();
     if (!rc) rc = preload_tfsf();
     if (!rc) rc = preload_lbc();
@@ -622,6 +676,42 @@ int fd2d_energy_diff(int wn, int wm, int nxa, int nya, int ia0, int ja0, const f
     return hip_check(hipStreamSynchronize(S(stream)), "fd2d_energy_diff sync");
 }
 
+// The n steps t0+1 .. of a run in pl.launches register-tile launches; p: the
+// run's parameters as the strip launches take them, freq: of its DFT planes.
+static int rt_run(const fd2d_tm_desc *d, const TbParams &p, const Plan &pl, int t0, int n,
+                  const float *freq, float dt, hipStream_t s)
+{
+    RtParams q{};
+    q.nx = p.nx; q.ny = p.ny;
+    q.naz = p.naz; q.nbz = p.nbz; q.pml = p.pml;
+    q.rlo = p.rlo; q.rhi = p.rhi; q.clo = p.clo; q.chi = p.chi;
+    q.nsrc = p.nsrc; q.src_wave = p.src_wave; q.wave_len = p.wave_len;
+    for (int k = 0; k < p.nsrc; ++k) { q.src_i[k] = p.src_i[k]; q.src_j[k] = p.src_j[k]; }
+    q.nprobe = p.nprobe; q.probe_out = p.probe_out; q.probe_len = p.probe_len;
+    for (int k = 0; k < p.nprobe; ++k) { q.probe_i[k] = p.probe_i[k]; q.probe_j[k] = p.probe_j[k]; }
+    q.tf_npml = p.tf_npml; q.inc = p.inc; q.inc_t0 = p.inc_t0; q.inc_stride = p.inc_stride;
+    q.ft_r = p.ft_r; q.ft_i = p.ft_i;
+    const bool lossy = d->md.nbz != nullptr, pml = pml_all(&d->pml);
+    float *A[6] = {d->dz, d->iz, d->hx, d->hy, d->ihx, d->ihy};
+    float *B[6] = {d->dz2, d->iz2, d->hx2, d->hy2, d->ihx2, d->ihy2};
+    int done = 0;
+    for (int l = 0; l < pl.launches; ++l) {
+        float **in = l % 2 ? B : A, **out = l % 2 ? A : B;
+        q.dz_i = in[0]; q.iz_i = in[1]; q.hx_i = in[2]; q.hy_i = in[3]; q.ihx_i = in[4]; q.ihy_i = in[5];
+        q.dz_o = out[0]; q.iz_o = out[1]; q.hx_o = out[2]; q.hy_o = out[3]; q.ihx_o = out[4]; q.ihy_o = out[5];
+        q.ez_o = l == pl.launches - 1 ? d->ez : nullptr;
+        q.K = n / pl.launches + (l < n % pl.launches ? 1 : 0);
+        q.t_first = t0 + done + 1;
+        for (int k = 0; k < q.K; ++k)
+            for (int f = 0; f < p.nf; ++f)
+                dft_twiddle(q.t_first + k, freq[f], dt, &q.tw[k][f], &q.tw[k][TB_MAX_FREQ + f]);
+        const int rc = launch_fd2d_rt(q, pl.rows / RT_ROWS, p.nf, lossy, pml, s);
+        if (rc) return rc;
+        done += q.K;
+    }
+    return 0;
+}
+
 static int tm_validate(const fd2d_tm_desc *d, int t0, int nsteps)
 {
     if (!d) return fail("fd2d_tm: desc is NULL");
@@ -703,7 +793,7 @@ static std::vector<TileRecord> &tile_records()
 // Tiles of the single-wave strip form of a plan: strips x row blocks.
 static size_t tm_tiles(const fd2d_tm_desc *d, const Plan &pl)
 {
-    if (pl.mw) return 0;
+    if (pl.mw || pl.rt) return 0;
     const int w = 64 * pl.cols - 2 * pl.halo;
     return (size_t)((d->ny + w - 1) / w) * (size_t)((d->nx + pl.rows - 1) / pl.rows);
 }
@@ -755,6 +845,7 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream)
     p.nprobe = d->nprobe;
     for (int k = 0; k < d->nprobe; ++k) { p.probe_i[k] = d->probe_i[k]; p.probe_j[k] = d->probe_j[k]; }
     p.probe_out = d->probe_out; p.probe_len = d->probe_len;
+    if (pl.rt) return rt_run(d, p, pl, t0, nsteps, nullptr, 0.f, S(stream));
     float *A[6] = {d->dz, d->iz, d->hx, d->hy, d->ihx, d->ihy};
     float *B[6] = {d->dz2, d->iz2, d->hx2, d->hy2, d->ihx2, d->ihy2};
     const int L = pl.launches;
@@ -1099,6 +1190,7 @@ static int tfsf_fused(const fd2d_tm_desc *d, const fd2d_tfsf_desc *b, int t0, in
     // 4 and short row blocks (more waves; MI355X sweeps at 1024^2, npml 80, 3
     // frequencies: 38k Mcell-updates/s at depth 8 rows 16, 60k at depth 4
     // rows 4)
+    const fd2d_tm_desc *own = d;           // as the caller gave it
     fd2d_tm_desc dd = *d;
     dd.form = FDTD_TM_FORM_STRIP;          // TF/SF corrections and DFT: strip form
     if (b->nf && !dd.depth) dd.depth = 4;
@@ -1120,7 +1212,7 @@ static int tfsf_fused(const fd2d_tm_desc *d, const fd2d_tfsf_desc *b, int t0, in
         const int n = nsteps - done < INC_CHUNK ? nsteps - done : INC_CHUNK;
         const int tc = t0 + done;                  // steps tc+1 .. tc+n
         Plan pl;
-        rc = plan_tm(d, n, &pl);
+        if (!plan_rt(own, n, true, &pl)) rc = plan_tm(d, n, &pl);
         if (rc) return rc;
         if (pl.tail_unfused || pl.launches == 0) {
             // too short for an even number of launches: the per-step kernels
@@ -1163,6 +1255,12 @@ static int tfsf_fused(const fd2d_tm_desc *d, const fd2d_tfsf_desc *b, int t0, in
         p.probe_out = d->probe_out; p.probe_len = d->probe_len;
         p.tf_npml = b->npml; p.inc = b->work; p.inc_t0 = tc; p.inc_stride = stride;
         p.nf = b->nf; p.ft_r = b->ft.r_pt; p.ft_i = b->ft.i_pt;
+        if (pl.rt) {
+            rc = rt_run(d, p, pl, tc, n, b->freq, b->dt, s0);
+            if (rc) return rc;
+            done += n;
+            continue;
+        }
         float *A[6] = {d->dz, d->iz, d->hx, d->hy, d->ihx, d->ihy};
         float *B[6] = {d->dz2, d->iz2, d->hx2, d->hy2, d->ihx2, d->ihy2};
         const int L = pl.launches;

@@ -133,6 +133,38 @@ struct TbParams {
     int rb_list[TB_MAX_LIST_RB], sx_list[TB_MAX_LIST_SX], t_list[TB_MAX_LIST_T];
 };
 
+// Arguments of one register-tile launch (fd2d_rt.hip); fields as in TbParams.
+constexpr int RT_ROWS = 4;          // rows of a wave
+constexpr int RT_WAVES = 16;        // waves of a tile, at most
+constexpr int RT_MAX_STEPS = 16;    // steps of a launch (twiddles in the arguments)
+struct RtParams {
+    int nx, ny, K, nsx;             // grid, steps of the launch, tiles along a row
+    const float *dz_i, *iz_i, *hx_i, *hy_i, *ihx_i, *ihy_i;
+    float *dz_o, *iz_o, *hx_o, *hy_o, *ihx_o, *ihy_o, *ez_o;
+    const float *naz, *nbz;
+    PmlPtrs pml;
+    int rlo, rhi, clo, chi;
+    int t_first;
+    int nsrc;
+    int src_i[FDTD_MAX_SOURCES], src_j[FDTD_MAX_SOURCES];
+    const float *src_wave;
+    int wave_len;
+    int nprobe;
+    int probe_i[FDTD_MAX_PROBES], probe_j[FDTD_MAX_PROBES];
+    float *probe_out;
+    int probe_len;
+    int tf_npml, inc_t0, inc_stride;
+    const float *inc;
+    float *ft_r, *ft_i;
+    float tw[RT_MAX_STEPS][2 * TB_MAX_FREQ];    // per step: cosines, then sines
+};
+// Tiles of waves * RT_ROWS rows by 64 columns that cover the grid, each
+// sharing 2K rows or columns with its neighbours.
+int rt_tiles(int nx, int ny, int waves, int K);
+// One launch of p.K steps.  The input and output sets must differ.
+int launch_fd2d_rt(const RtParams &p, int waves, int nf, bool lossy, bool pml, hipStream_t s);
+int preload_rt();
+
 // Arguments of one learned-boundary frame launch (lbc_frame.hip).
 struct LbcFrameParams {
     int nx, ny, K;                              // grid, steps of the launch

@@ -16,6 +16,7 @@
 #include <math.h>
 
 #include "fdtd_internal.h"
+#include "lanes.h"
 
 namespace fdtd {
 namespace {
@@ -155,52 +156,156 @@ __global__ void __launch_bounds__(1024) inc_chunk_kernel(int ny, float *ezi, flo
     }
 }
 
-// The same with the incident grid held in LDS for the whole chunk (ezi,
-// hxi: 2 ny floats; bc in registers of thread 0): per step only barriers, no
-// global round trips; the table rows go out as plain stores.
-__global__ void __launch_bounds__(1024) inc_chunk_lds_kernel(int ny, float *ezi, float *hxi,
+// The same with the incident grid in registers: a wave holds 64 M cells, M a
+// lane, and owns all but the outer INC_HALO on either side it shares with a
+// neighbour.  A step then needs DPP shifts only; every INC_HALO steps the
+// waves pass their owned edge cells through LDS.  The chunk's source values
+// and twiddles sit one step a lane.  What bounds it is the chain of one step
+// (some 25 dependent operations).  MI355X, 64 steps, with the launch: ny 150
+// ~60 us with the grid in LDS (four barriers a step), ~110 us with the probe's
+// DFT (a round trip to memory a step).
+constexpr int INC_HALO = 8;
+
+template <int M>
+__global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi, float *hxi,
                                                              float *bc, float *r_in, float *i_in,
                                                              float *table, IncChunk a)
 {
-    extern __shared__ float sm[];
-    float *e = sm, *h = sm + ny;
-    const int tid = threadIdx.x, m = a.npml, nbox = ny - 2 * m + 2;
-    for (int j = tid; j < ny; j += blockDim.x) { e[j] = ezi[j]; h[j] = hxi[j]; }
-    float b0 = 0.f, b1 = 0.f, b2 = 0.f, b3 = 0.f;
-    if (tid == 0) { b0 = bc[0]; b1 = bc[1]; b2 = bc[2]; b3 = bc[3]; }
-    __syncthreads();
-    for (int s = 0; s < a.n; ++s) {
-        for (int j = tid + 1; j < ny; j += blockDim.x) e[j] = e[j] + 0.5f * (h[j - 1] - h[j]);
-        __syncthreads();
-        if (tid == 0) {
-            e[0] = b0;
-            b0 = b1;
-            b1 = e[1];
-            e[ny - 1] = b3;
-            b3 = b2;
-            b2 = e[ny - 2];
-            e[a.inc_pos] = a.wave[s];
+    constexpr int H = INC_HALO, S = 64 * M;
+    // owned edge cells: [wave][left, right][ezi, hxi][cell]
+    __shared__ float xch[16][2][2][H];
+    const int lane = (int)threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), W = (int)blockDim.x >> 6;
+    const int base = w * (S - 2 * H), k0 = lane * M, j0 = base + k0;
+    const int o0 = w ? base + H : 0, o1 = w == W - 1 ? ny : base + S - H;
+    const int m = a.npml;
+    float e[M], h[M];
+#pragma unroll
+    for (int c = 0; c < M; ++c) {
+        const int j = min(j0 + c, ny - 1);
+        e[c] = ezi[j];
+        h[c] = hxi[j];
+    }
+    float b0 = bc[0], b1 = bc[1], b2 = bc[2], b3 = bc[3];
+    float wv = 0.f, twc[TB_MAX_FREQ], tws[TB_MAX_FREQ], ri[TB_MAX_FREQ], ii[TB_MAX_FREQ];
+    static_assert(INC_CHUNK <= 64, "one step a lane");
+    if (lane < a.n) wv = a.wave[lane];
+    const bool dft = r_in && a.probe >= o0 && a.probe < o1;      // the wave owns the probe
+#pragma unroll
+    for (int f = 0; f < TB_MAX_FREQ; ++f) {
+        twc[f] = tws[f] = ri[f] = ii[f] = 0.f;
+        if (dft && f < a.nf) {
+            if (lane < a.n) { twc[f] = a.c[lane][f]; tws[f] = a.s[lane][f]; }
+            ri[f] = r_in[f];
+            ii[f] = i_in[f];
         }
-        __syncthreads();
+    }
+    const bool src = a.inc_pos >= base && a.inc_pos < base + S;
+    const bool right = ny - 1 < base + S;                        // the window holds cell ny-1
+    // cell j's value (in the window), in every lane
+    auto cell = [&](const float (&v)[M], int j) __attribute__((always_inline)) {
+        const int k = j - base;
+        float x = v[0];
+#pragma unroll
+        for (int c = 1; c < M; ++c) x = k % M == c ? v[c] : x;
+        return lane_get(x, k / M);
+    };
+#pragma unroll 1
+    for (int s = 0; s < a.n; ++s) {
+        const float hl = lane_left(h[M - 1]);
+#pragma unroll
+        for (int c = M - 1; c >= 0; --c) e[c] = e[c] + 0.5f * ((c ? h[c ? c - 1 : 0] : hl) - h[c]);
+        // two-step boundary (it replaces cells 0 and ny-1), then the source
+        if (w == 0) {
+            if (lane == 0) e[0] = b0;
+            b0 = b1;
+            b1 = cell(e, 1);
+        }
+        if (right) {
+#pragma unroll
+            for (int c = 0; c < M; ++c) e[c] = j0 + c == ny - 1 ? b3 : e[c];
+            b3 = b2;
+            b2 = cell(e, ny - 2);
+        }
+        if (src) {
+            const float v = lane_get(wv, s);
+#pragma unroll
+            for (int c = 0; c < M; ++c) e[c] = j0 + c == a.inc_pos ? v : e[c];
+        }
         float *row = table + (size_t)s * a.stride;
-        if (tid == 0) {
-            row[0] = h[m - 2];
-            row[1] = h[ny - m];
-            if (r_in) {
-                const float v = e[a.probe];
-                for (int f = 0; f < a.nf; ++f) {
-                    r_in[f] = r_in[f] + a.c[s][f] * v;
-                    i_in[f] = i_in[f] - a.s[s][f] * v;
-                }
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            const int j = j0 + c;
+            if (j >= o0 && j < o1) {
+                if (j >= m - 1 && j <= ny - m) row[2 + j - (m - 1)] = e[c];
+                if (j == m - 2) row[0] = h[c];
+                if (j == ny - m) row[1] = h[c];
             }
         }
-        for (int k = tid; k < nbox; k += blockDim.x) row[2 + k] = e[m - 1 + k];
-        __syncthreads();
-        for (int j = tid; j < ny - 1; j += blockDim.x) h[j] = h[j] + 0.5f * (e[j] - e[j + 1]);
-        __syncthreads();
+        if (dft) {
+            const float v = cell(e, a.probe);
+#pragma unroll
+            for (int f = 0; f < TB_MAX_FREQ; ++f) {
+                ri[f] = ri[f] + lane_get(twc[f], s) * v;
+                ii[f] = ii[f] - lane_get(tws[f], s) * v;
+            }
+        }
+        const float er = lane_right(e[0]);
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            const float v = h[c] + 0.5f * (e[c] - (c + 1 < M ? e[c + 1 < M ? c + 1 : 0] : er));
+            h[c] = j0 + c == ny - 1 ? h[c] : v;
+        }
+        if (W > 1 && s % H == H - 1) {
+#pragma unroll
+            for (int c = 0; c < M; ++c) {
+                const int k = k0 + c;
+                if (k >= H && k < 2 * H) { xch[w][0][0][k - H] = e[c]; xch[w][0][1][k - H] = h[c]; }
+                if (k >= S - 2 * H && k < S - H) {
+                    xch[w][1][0][k - (S - 2 * H)] = e[c];
+                    xch[w][1][1][k - (S - 2 * H)] = h[c];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int c = 0; c < M; ++c) {
+                const int k = k0 + c;
+                if (w > 0 && k < H) { e[c] = xch[w - 1][1][0][k]; h[c] = xch[w - 1][1][1][k]; }
+                if (w < W - 1 && k >= S - H) {
+                    e[c] = xch[w + 1][0][0][k - (S - H)];
+                    h[c] = xch[w + 1][0][1][k - (S - H)];
+                }
+            }
+            __syncthreads();
+        }
     }
-    for (int j = tid; j < ny; j += blockDim.x) { ezi[j] = e[j]; hxi[j] = h[j]; }
-    if (tid == 0) { bc[0] = b0; bc[1] = b1; bc[2] = b2; bc[3] = b3; }
+#pragma unroll
+    for (int c = 0; c < M; ++c) {
+        const int j = j0 + c;
+        if (j >= o0 && j < o1) { ezi[j] = e[c]; hxi[j] = h[c]; }
+    }
+    if (lane == 0) {
+        if (w == 0) { bc[0] = b0; bc[1] = b1; }
+        if (w == W - 1) { bc[2] = b2; bc[3] = b3; }
+        if (dft) {
+#pragma unroll
+            for (int f = 0; f < TB_MAX_FREQ; ++f)
+                if (f < a.nf) { r_in[f] = ri[f]; i_in[f] = ii[f]; }
+        }
+    }
+}
+
+// Launches the register form with M cells a lane if 16 waves hold ny cells.
+template <int M>
+bool inc_chunk_reg(int ny, float *ezi, float *hxi, float *bc, float *r_in, float *i_in,
+                   float *table, const IncChunk &a, hipStream_t s)
+{
+    constexpr int S = 64 * M, O = S - 2 * INC_HALO;
+    const int waves = ny <= S ? 1 : 1 + (ny - S + O - 1) / O;
+    if (waves > 16) return false;
+    hipLaunchKernelGGL((inc_chunk_reg_kernel<M>), dim3(1), dim3(64 * waves), 0, s, ny, ezi, hxi, bc,
+                       r_in, i_in, table, a);
+    return true;
 }
 
 }  // namespace
@@ -210,11 +315,13 @@ int preload_tfsf() { return preload_kernel(reinterpret_cast<const void *>(&set_k
 int launch_inc_chunk(int ny, float *ezi, float *hxi, float *bc, float *r_in, float *i_in,
                      float *table, const IncChunk &a, hipStream_t s)
 {
-    const size_t lds = 2 * (size_t)ny * sizeof(float);
-    if (lds <= 64 * 1024)
-        hipLaunchKernelGGL(inc_chunk_lds_kernel, dim3(1), dim3(1024), lds, s, ny, ezi, hxi, bc, r_in,
-                           i_in, table, a);
-    else
+    // the fewest cells a lane that 16 waves allow; past 16144 cells (and on
+    // grids whose two ends share cells) the form in global memory
+    if (ny < 4 || !(inc_chunk_reg<1>(ny, ezi, hxi, bc, r_in, i_in, table, a, s) ||
+                    inc_chunk_reg<2>(ny, ezi, hxi, bc, r_in, i_in, table, a, s) ||
+                    inc_chunk_reg<4>(ny, ezi, hxi, bc, r_in, i_in, table, a, s) ||
+                    inc_chunk_reg<8>(ny, ezi, hxi, bc, r_in, i_in, table, a, s) ||
+                    inc_chunk_reg<16>(ny, ezi, hxi, bc, r_in, i_in, table, a, s)))
         hipLaunchKernelGGL(inc_chunk_kernel, dim3(1), dim3(1024), 0, s, ny, ezi, hxi, bc, r_in, i_in,
                            table, a);
     return hip_check(hipGetLastError(), "incident chunk");

@@ -79,8 +79,8 @@ def parse():
                     help="learned: network parameters (.npz from simulation_amd.learned); "
                          "default: the committed weights, else the zero network")
     ap.add_argument("--waves", type=int, default=0,
-                    help="batch: waves of the batch launch (0: as many as stay resident, "
-                         "a persistent sweep of the unit list; -1: one wave per unit)")
+                    help="batch: waves of the batch launch (0, or -1: one per unit; else "
+                         "that many, each sweeping several units)")
     ap.add_argument("--no-graph", action="store_true",
                     help="batch: time the eager launches instead of one captured graph launch")
     ap.add_argument("--fresh-medium", action="store_true",
@@ -320,7 +320,7 @@ def bench_batch(a):
     0), 1-5 lossy cylinders each, npml=8, hard Gaussian point source, one probe
     per grid; `steps` fused steps per grid (default 3000), timed as one
     captured HIP graph launch (--no-graph: the eager fd2d_batch_run
-    launches).  Each launch of the persistent kernel advances every grid by
+    launches).  Each launch advances every grid by
     up to `depth` steps; its minimum HBM bytes are 60 B per cell of the batch
     (every state array read and written once, naz and nbz read once)."""
     import torch
@@ -364,18 +364,18 @@ def bench_batch(a):
     achieved = min_bytes / (launch_ms * 1e-3) / 1e9
     effective = B_ALG * cells * K / (ev_ms * 1e-3) / 1e9
     # a launch reads and writes every state array once whatever its number of
-    # fused steps, so launches of 7 and 8 steps share the record of depth 8
-    key = f"fd2d_batch_c3_seed0_d{D}_r{b.desc.rows or 128}_c{b.desc.cols}"
+    # fused steps, so launches of 9 and 10 steps share the record of depth 10
+    key = f"fd2d_batch_c3_seed0_d{D}_r{b.desc.rows}_c{b.desc.cols}"
     rec = {
         "metric": METRIC, "value": round(cells * K / wall / 1e6, 1), "unit": "Mcell-updates/s",
         "n_gpus": 1, "steps": K, "warmup": a.warmup, "ms_per_step": round(wall * 1e3 / K, 4),
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32",
         "data": "synthetic (seeded grid sizes, cylinders and sources; fields start at zero)",
         "config": {"workload": "256 batched 2-D TM grids, sides U[128,1024] (seed 0), 1-5 lossy "
-                               "cylinders, npml=8, hard Gaussian source, persistent launches"
+                               "cylinders, npml=8, hard Gaussian source"
                                + (", one captured HIP graph" if graph else ", eager launches"),
                    "cells": cells, "grids": len(specs), "steps_per_launch": sorted(set(depths)),
-                   "rows": b.desc.rows or 128,
+                   "rows": b.desc.rows,
                    "cols": b.desc.cols, "waves": b.desc.waves, "units": b.desc.nunits,
                    "launches": L},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK,

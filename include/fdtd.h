@@ -323,7 +323,7 @@ size_t fd2d_tm_tile_elems(const fd2d_tm_desc *d, int nsteps);
 
 /* ------------------------------------------------------ batched grids
  * Many independent TM grids of different sizes advanced together by one
- * persistent kernel per fused step group.  No reference counterpart: the
+ * launch per fused step group.  No reference counterpart: the
  * reference runs one grid per program (fd2d/pycuda/fd2d_3_4.py:269-389);
  * each grid here evolves exactly as fd2d_tm_run would evolve it alone (bit
  * for bit).  All grids of a batch share the form (lossy PML: md.nbz and the
@@ -348,9 +348,8 @@ typedef struct fd2d_batch_desc {
     const fd2d_grid *grids_dev;   /* device copy of the grid records */
     const int *units_dev;         /* device work list, 4 ints per unit */
     int nunits;
-    int depth, rows, cols;        /* fixed when the work list is made (rows 0:
-                                     the default, see fd2d_batch_units) */
-    int waves;                    /* workgroups of the persistent launch */
+    int depth, rows, cols;        /* fixed when the work list is made */
+    int waves;                    /* workgroups of a launch */
     int vec;                      /* 1: every grid allows vector loads */
     int wave_len;                 /* smallest wave_len over grids with a source
                                      (INT_MAX: none), set by fd2d_batch_upload */
@@ -369,8 +368,9 @@ typedef struct fd2d_batch_desc {
 } fd2d_batch_desc;
 
 /* Number of work units (and so ints/4 of units_dev) a batch needs for the
- * given depth (0 = 8), rows per block (0 = 128, or the whole grid when it
- * has fewer rows) and columns per lane (0 = 1).  A unit is 4 ints: grid, strip,
+ * given depth, rows per block (both 0: by the cells of all grids, 6 and 12
+ * below 5 million, 8 and 24 below 8 million, 10 and 32 below 30 million, else
+ * 10 and 48) and columns per lane (0 = 1).  A unit is 4 ints: grid, strip,
  * first row, one past the last row.                                       */
 int fd2d_batch_units(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols,
                      int *nunits);
@@ -378,10 +378,10 @@ int fd2d_batch_units(const fd2d_grid *grids, int ngrids, int depth, int rows, in
 /* Validate the grids (host array), write the work list and the grid records
  * into the caller's device buffers (asynchronously on stream; the host
  * arrays may be released on return) and fill *out.  units_dev holds
- * 4*max_units ints, grids_dev ngrids records.  waves = 0 picks the number of
- * waves the device keeps resident.  The units are ordered for the waves of
- * the persistent launch (wave w takes units w, w + waves, ...): sorted by
- * estimated cost and dealt out round by round in alternating directions.   */
+ * 4*max_units ints, grids_dev ngrids records.  waves = 0 gives every unit a
+ * workgroup of its own; otherwise `waves` persistent ones take units w, w +
+ * waves, ..., sorted by estimated cost and dealt out round by round in
+ * alternating directions.                                                  */
 int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols,
                       int waves, fd2d_grid *grids_dev, int *units_dev, int max_units,
                       fd2d_batch_desc *out, void *stream);

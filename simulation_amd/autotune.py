@@ -1,7 +1,7 @@
 """Autotuner for the temporally blocked launches.
 
 Chooses the temporal depth (leapfrog steps fused per launch), rows per block
-and columns per lane -- plus, for batches, the number of resident waves --
+and columns per lane -- plus, for batches, the number of waves --
 by timing candidate launch shapes on the device, and caches the winner in a
 JSON file keyed by device name, problem shape and form.  Every candidate
 computes the same values bit for bit (the shape only changes which cells are
@@ -45,12 +45,14 @@ def candidates(nx: int):
 
 
 def batch_candidates():
-    """(depth, rows, cols, waves) shapes tried for a batch: depth 8 with
-    96-160 rows and depth 10 with 128 (on MI355X the 256-grid batch of sides
-    128-1024 peaks at depth 8, 128 rows), and two columns per lane."""
-    for rows in (96, 128, 160):
-        yield 8, rows, 1, 0
-    yield 10, 128, 1, 0
+    """(depth, rows, cols, waves) shapes tried for a batch: depth 10 with 32-64
+    rows (on MI355X the 256-grid batch of sides 128-1024 peaks at depth 10,
+    48 rows), shallower and shorter ones for smaller batches, and two columns
+    per lane."""
+    for rows in (32, 48, 64):
+        yield 10, rows, 1, 0
+    yield 8, 24, 1, 0
+    yield 6, 12, 1, 0
     yield 8, 128, 2, 0
 
 
@@ -149,7 +151,7 @@ def tune_batch(b, steps: int = 48, use_cache: bool = True, configs=None,
     if b.t != 0:
         raise ValueError("tune_batch runs before the first step")
     sig = hashlib.sha1(repr([(s.nx, s.ny, s.npml) for s in b.specs]).encode()).hexdigest()[:16]
-    key = f"batch|{_device()}|{len(b.specs)} grids|{sig}"
+    key = f"batch2|{_device()}|{len(b.specs)} grids|{sig}"
     db = _load() if use_cache and configs is None else {}
     if key in db:
         best = db[key]

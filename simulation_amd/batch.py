@@ -2,7 +2,7 @@
 
 Hundreds of independent grids of different sizes, each with its own lossy
 cylinders, PML profiles, hard Gaussian source and probe, advance together: a
-persistent kernel walks a work list of (grid, strip, row block) units, each
+launch covers a work list of (grid, strip, row block) units, each
 launch fuses ``depth`` leapfrog steps for every grid, and a whole run can be
 captured into one HIP graph and replayed as a single launch.  Every grid
 evolves exactly as it would alone through ``fd2d.TMSolver`` (bit for bit).

@@ -1144,11 +1144,14 @@ struct BatchParams {
     static constexpr bool one_sp = true;
 };
 
-// A persistent kernel over a work list of (grid, strip, row block) units of
-// many independent grids (fd2d_grid records in device memory); each unit is
-// swept exactly as the single-grid kernels sweep it.  Lossy PML form only.
+// A kernel over a work list of (grid, strip, row block) units of many
+// independent grids (fd2d_grid records in device memory), one workgroup a
+// unit or persistent waves; each unit is swept exactly as the single-grid
+// kernels sweep it.  Lossy PML form only.  Four waves a SIMD up to depth 7;
+// past that they spill (40 bytes a lane at depth 8: 31.9 ms against 27.9 at
+// three waves, the 256-grid batch of sides 128-1024, 144 steps, 64 rows).
 template <int K, int C, bool VEC>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(C == 1 && K <= 8 ? 4 : 1)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(C == 1 && K <= 7 ? 4 : C == 1 && K <= 11 ? 3 : 1)))
 tm_tb_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ units, int nunits,
                    int parity, int t_first, int write_ez, int halo, BatchVac vac)
 {
@@ -1236,7 +1239,9 @@ tm_tb_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ 
             else sweep<K, C, true, true, VEC, false, false, false, 0, true, C == 1>(P, g, ring);
         } else {
             if (vac.mode == 1 && threadIdx.x == 0) vac.work[u] = vac.tag;
-            if (!sp) sweep<K, C, true, true, VEC, true, true, false, 0, true>(P, g, ring);
+            if (!brow && !sp) sweep<K, C, true, true, VEC, false, true, false, 0, true>(P, g, ring);
+            else if (!bcol && !sp) sweep<K, C, true, true, VEC, true, false, false, 0, true>(P, g, ring);
+            else if (!sp) sweep<K, C, true, true, VEC, true, true, false, 0, true>(P, g, ring);
             else sweep<K, C, true, true, VEC, true, true, true, 0, true>(P, g, ring);
         }
     }
@@ -1249,20 +1254,6 @@ int launch_batch_kv(const fd2d_grid *grids, const int *units, int nunits, int wa
     hipLaunchKernelGGL((tm_tb_batch_kernel<K, C, VEC>), dim3(waves), dim3(64), 0, s, grids, units,
                        nunits, parity, t_first, write_ez, halo, vac);
     return hip_check(hipGetLastError(), "fd2d_batch_run launch");
-}
-
-template <int K, int C, bool VEC>
-int batch_resident_kv(int *waves)
-{
-    int per_cu = 0, dev = 0, ncu = 0;
-    int rc = hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                           &per_cu, (const void *)tm_tb_batch_kernel<K, C, VEC>, 64, 0),
-                       "occupancy query");
-    if (!rc) rc = hip_check(hipGetDevice(&dev), "hipGetDevice");
-    if (!rc) rc = hip_check(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev),
-                            "CU count");
-    if (!rc) *waves = per_cu * ncu;
-    return rc;
 }
 
 }  // namespace tb
@@ -1281,15 +1272,6 @@ int launch_fd2d_batch_depth(const fd2d_grid *grids, const int *units, int nunits
     if (cols == 1)
         return tb::launch_batch_kv<K, 1, false>(grids, units, nunits, waves, parity, t_first, write_ez,
                                                 halo, vac, s);
-    return fail("columns per lane %d not built", cols);
-}
-
-template <int K>
-int fd2d_batch_resident_depth(int cols, bool vec, int *waves)
-{
-    if (cols == 2 && vec) return tb::batch_resident_kv<K, 2, true>(waves);
-    if (cols == 2) return tb::batch_resident_kv<K, 2, false>(waves);
-    if (cols == 1) return tb::batch_resident_kv<K, 1, false>(waves);
     return fail("columns per lane %d not built", cols);
 }
 

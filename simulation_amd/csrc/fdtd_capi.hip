@@ -303,30 +303,31 @@ int aux_for_current_device(Aux **out)
 // ------------------------------------------------------- batched grids
 
 struct BatchGeom {
-    int depth, rows, cols, halo;   // rows 0: the default (batch_grid_rows)
+    int depth, rows, cols, halo;
 };
 
-int batch_geom(int depth, int rows, int cols, BatchGeom *g)
+// The launch shape of a batch; depth, rows, cols 0: the library's choice, by
+// the cells of all grids together -- few cells want many short units, whose
+// warm-up rows cost less than idle SIMDs.  MI355X, ms of 120 steps at depth /
+// rows, sides and cells: 96-200, 4.5M: 6/12 2.38, 8/24 2.74, 10/32 3.34;
+// 300-500, 6.6M: 2.60, 2.16, 2.61; 700-900, 10M: 3.65, 2.83, 2.64; 300-700,
+// 27M: 10.4, 7.91, 7.23; 150-900, 38M: 13.7, 10.4, 9.56 (10/48: 9.56);
+// 128-1024, 97M, 144 steps: 10/32 23.4, 10/48 22.7, 10/64 23.2.  (8/128 with
+// persistent waves, before: 6.12, 5.93, 5.98, 10.4, 14.5, 34.5.)
+int batch_geom(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols, BatchGeom *g)
 {
-    g->depth = depth ? depth : 8;
+    long long cells = 0;
+    for (int k = 0; k < ngrids; ++k) cells += (long long)grids[k].nx * grids[k].ny;
+    g->depth = depth ? depth : cells < 5000000 ? 6 : cells < 8000000 ? 8 : 10;
+    g->rows = rows ? rows
+                   : cells < 5000000 ? 12 : cells < 8000000 ? 24 : cells < 30000000 ? 32 : 48;
     g->cols = cols ? cols : 1;
-    g->rows = rows;
     if (!tb_supported(g->depth, g->cols))
         return fail("fd2d_batch: depth=%d cols=%d not supported", g->depth, g->cols);
     g->halo = ((g->depth + g->cols - 1) / g->cols) * g->cols;
     if (64 * g->cols - 2 * g->halo < 8) return fail("fd2d_batch: depth too large for the strip");
     if (g->rows < 0) return fail("fd2d_batch: rows=%d", g->rows);
     return 0;
-}
-
-// Rows of a grid's blocks: the caller's, or (rows = 0) 128 -- on MI355X the
-// 256-grid batch of sides 128-1024, with the units dealt out as below, ran
-// 374k Mcell-updates/s at 128 rows, 360k at 112, 343k at 160, 343k at 64
-// (and, dealt out in list order, 330k at 64 and 329k at 128).
-int batch_grid_rows(const BatchGeom &g, int nx)
-{
-    const int h = g.rows ? g.rows : 128;
-    return h < nx ? h : nx;
 }
 
 int check_grid(const fd2d_grid &G, int k)
@@ -1515,13 +1516,13 @@ int fd2d_batch_units(const fd2d_grid *grids, int ngrids, int depth, int rows, in
     clear_error();
     if (!grids || ngrids <= 0 || !nunits) return fail("fd2d_batch_units: grids/ngrids/nunits");
     BatchGeom g;
-    int rc = batch_geom(depth, rows, cols, &g);
+    int rc = batch_geom(grids, ngrids, depth, rows, cols, &g);
     if (rc) return rc;
     const int w = 64 * g.cols - 2 * g.halo;
     long long n = 0;
     for (int k = 0; k < ngrids; ++k) {
         if (grids[k].nx < 2 || grids[k].ny < 2) return fail("fd2d_batch_units: grid %d size", k);
-        const int h = batch_grid_rows(g, grids[k].nx);
+        const int h = std::min(g.rows, grids[k].nx);
         n += (long long)((grids[k].ny + w - 1) / w) * ((grids[k].nx + h - 1) / h);
     }
     if (n > (1LL << 30)) return fail("fd2d_batch_units: too many units");
@@ -1537,7 +1538,7 @@ int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, i
     if (!grids || ngrids <= 0 || !grids_dev || !units_dev || !out)
         return fail("fd2d_batch_upload: grids, grids_dev, units_dev and out are required");
     BatchGeom g;
-    int rc = batch_geom(depth, rows, cols, &g);
+    int rc = batch_geom(grids, ngrids, depth, rows, cols, &g);
     if (rc) return rc;
     bool vec = g.cols == 2;
     int min_wave = INT_MAX, min_probe = INT_MAX;
@@ -1555,7 +1556,7 @@ int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, i
     std::vector<int> edge, inner;
     for (int k = 0; k < ngrids; ++k) {
         const fd2d_grid &G = grids[k];
-        const int h = batch_grid_rows(g, G.nx);
+        const int h = std::min(g.rows, G.nx);
         const int ns = (G.ny + w - 1) / w, nb = (G.nx + h - 1) / h;
         const int rlo = G.band_rows[1] > G.band_rows[0] ? std::max(G.band_rows[0], 1) : 0;
         const int rhi = G.band_rows[1] > G.band_rows[0] ? std::min(G.band_rows[1], G.nx - 1) : 0;
@@ -1580,24 +1581,44 @@ int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, i
     if (n > max_units) return fail("fd2d_batch_upload: %d units exceed max_units=%d", n, max_units);
     const size_t nedge = edge.size() / 4;
     edge.insert(edge.end(), inner.begin(), inner.end());
-    // Balance the waves of the persistent launch: wave `slot` takes the units
-    // at slot, slot + nw, slot + 2 nw, ...  The units are sorted by their
-    // estimated cost, longest first (rows swept: the block and its 2K rows of
-    // warm-up; the general body of edge, PML, source and probe units costs
-    // about 1.75 interior rows per row), and dealt out round by round in a
-    // snake: round r gives its units to slots 0..nw-1 when r is even and to
-    // nw-1..0 when odd, so a wave that drew a long unit in one round draws a
-    // short one in the next.  The last, partial round is dealt in order so
-    // the list stays dense.  The sort is stable: units of equal cost keep
-    // their grid and strip order, so neighbours still run side by side.
-    // (MI355X, the 256-grid batch: 330k -> 374k Mcell-updates/s at 128 rows;
-    // edge costs 1.0 / 1.4 / 2.5: 360k / 370k / 359k.)
+    // The order of the units.  waves <= 0: one workgroup a unit, which the
+    // dispatcher hands to whatever SIMD is free.  Workgroup b runs on XCD
+    // b % 8 and takes slot (b % 8) n/8 + b/8, so XCD x works down the x-th
+    // eighth of the list: that is an eighth of the edge units (the slower
+    // ones, first) and then an eighth of the inner ones, both in grid, row and
+    // strip order, so that units which share halos run side by side under one
+    // L2.  MI355X, the 256-grid batch, depth 10, 64 rows: persistent waves
+    // 29.2 ms; one workgroup a unit, runs of 1 / 4 / 16 / 64 / 256 units dealt
+    // to the XCDs in turn 27.1 / 25.2 / 24.4 / 23.9 / 23.4, eighths 23.2.
     if (waves <= 0) {
-        rc = fd2d_batch_resident(g.depth, g.cols, vec, &waves);
-        if (rc) return rc;
-    }
-    waves = std::max(1, std::min(waves, n));
-    {
+        waves = n;
+        std::vector<int> lay;
+        lay.reserve(4 * (size_t)n);
+        size_t e = 0, i = nedge;
+        for (int x = 0; x < 8; ++x) {
+            // the slots of XCD x, and its share of the edge units among them
+            const size_t slots = (size_t)n / 8 + ((size_t)x < (size_t)n % 8 ? 1 : 0);
+            const size_t left = (size_t)n - i, share = std::max(nedge * (x + 1) / 8, e) - e;
+            const size_t ne = std::min(std::max(share, slots - std::min(slots, left)),
+                                       std::min(slots, nedge - e));
+            lay.insert(lay.end(), edge.begin() + 4 * e, edge.begin() + 4 * (e + ne));
+            e += ne;
+            lay.insert(lay.end(), edge.begin() + 4 * i, edge.begin() + 4 * (i + slots - ne));
+            i += slots - ne;
+        }
+        edge.swap(lay);
+    } else {
+        // Balance the waves of a persistent launch: wave `slot` takes the
+        // units at slot, slot + nw, slot + 2 nw, ...  The units are sorted by
+        // their estimated cost, longest first (rows swept: the block and its
+        // 2K rows of warm-up; the general body of edge, PML, source and probe
+        // units costs about 1.75 interior rows per row), and dealt out round
+        // by round in a snake: round r gives its units to slots 0..nw-1 when r
+        // is even and to nw-1..0 when odd, so a wave that drew a long unit in
+        // one round draws a short one in the next.  The last, partial round is
+        // dealt in order so the list stays dense.  The sort is stable: units
+        // of equal cost keep their grid and strip order.
+        waves = std::min(waves, n);
         const int nw = waves;
         auto cost = [&](int q) {
             const double gen = (size_t)q < nedge ? 1.75 : 1.0;

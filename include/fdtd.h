@@ -309,10 +309,11 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream);
  * number of launches and the chosen depth/rows/cols.  Defaults (measured on
  * MI355X): with form, depth, rows and cols all 0, grids of up to 2.7 million
  * cells run register tiles of `rows` rows (32 or 48; depth 7 to 14 by the
- * number of tiles); otherwise strips of one column per lane; depth 10 from nx = 2048 on, else 8; rows =
- * nx/128 for 4096 <= nx < 12288, else nx/170, clamped to [8, 512]; the
- * multi-wave form: depth 8, rows = nx/32 clamped to [32, 512].  Depths go up
- * to 12.  Host only.                                                       */
+ * number of tiles); otherwise strips of one column per lane, by the cells N
+ * of the grid: depth 8 below 5.5 million, 10 below 11 million, else 11; rows
+ * N/330000 below 6.6 million, N/230000 (at most 80) below 100 million, else
+ * 96, at least 8.  The multi-wave form: depth 8, rows = nx/32 clamped to [32,
+ * 512].  Depths go up to 12.  Host only.                                   */
 int fd2d_tm_plan(const fd2d_tm_desc *d, int nsteps,
                  int *launches, int *depth, int *rows, int *cols);
 

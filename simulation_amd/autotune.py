@@ -25,17 +25,14 @@ CACHE = os.environ.get("FDTD_TUNE_CACHE",
 
 
 def candidates(nx: int):
-    """(depth, rows, cols, form) shapes tried for an nx-row grid: single-wave
+    """(depth, rows, cols, form) shapes tried for an nx-row grid: the library's
+    own choice (by the grid's cells: register tiles or strips), single-wave
     strips at depth 10 (and from 4096 rows on depth 11) with row blocks of
-    nx/170, nx/128 and nx/96 rows and at depth 8 with nx/128 (MI355X sweeps
-    put the optimum at depth 10 at 2048^2 and depth 11 from 4096^2 on, rows
-    ~nx/170 at 2048^2 and ~nx/128 from 4096^2 on), two columns per lane at
-    depth 8, and the multi-wave form with short blocks; below 2048 rows also
-    the library's own choice (register tiles up to 2.7 million cells)."""
+    nx/170, nx/128 and nx/96 rows and at depth 8 with nx/128, two columns per
+    lane at depth 8, and the multi-wave form with short blocks."""
     def r(d):
         return min(512, max(8, nx // d))
-    if nx < 2048:
-        yield 0, 0, 0, 0
+    yield 0, 0, 0, 0
     for depth in ((10, 11) if nx >= 4096 else (10,)):
         for rows in sorted({r(170), r(128), r(96)}):
             yield depth, rows, 1, 1

@@ -186,8 +186,13 @@ bool plan_rt(const fd2d_tm_desc *d, int nsteps, bool tf, Plan *pl)
     return true;
 }
 
-// Rows of an interior block of the multi-wave form when the caller gives
-// none.
+// Rows of the multi-wave form's frame tiles, and of its interior blocks when
+// the caller gives none.
+int mw_frame_rows(int nx)
+{
+    const int h = nx >= 4096 && nx < 12288 ? nx / 128 : nx / 170;
+    return std::min(std::max(h, 8), 512);
+}
 int mw_default_rows(int nx)
 {
     long h = nx / 32;
@@ -196,32 +201,25 @@ int mw_default_rows(int nx)
     return (int)h;
 }
 
-// Default depth and rows of the single-wave strips, from sweeps on MI355X
-// (lossy PML form, one column per lane; Mcell-updates/s at 1000-2000 steps):
-//   2048^2:  depth 10, rows 12 (355k; rows 16/24: 260k/206k; depth 8 rows 16:
-//            278k; depth 11 rows 12/16: 342k/305k)
-//   4096^2:  depth 11, rows 32 (621k; rows 40: 626k; depth 10 rows 32/42:
-//            592k/595k; depth 8 rows 16/32/48: 449k/494k/461k)
-//   8192^2:  depth 11, rows 64 (737k-757k; rows 56/72/85/96: 699k/732k/724k/
-//            725k; depth 10 rows 64: 698k-715k; depth 8 rows 64: 586k;
-//            depth 12: 576k)
-//   16384^2: depth 11, rows 96 (815k; rows 128: 817k; depth 10 rows 96:
-//            774k; depth 8 rows 96: 606k)
-// Depths 10 and 11 keep two carry sets in 3 waves per SIMD (depth 12 needs
-// 192 VGPRs: 2 waves); depth 11 moves the arrays once per 11 steps instead
-// of 10 and wins from 4096^2 on, where its one more halo column and warm-up
-// row per side cost less.  Rows follow nx/128 for 4096 <= nx < 12288 and
-// ~nx/170 outside.  With the free-space tiles that move no iz (fewer bytes
-// per launch) the two depths are close below 16384^2: 8192^2 depth 10/11
-// rows 64: 852k/839k, rows 85: 831k/841k; 4096^2 rows 32: 679k/684k;
-// 16384^2 rows 96: 855k/886k (the autotuner picks per grid).
-void tm_defaults(int nx, int *depth, int *rows)
+// Default depth and rows of the single-wave strips, by the grid's cells N:
+// what decides is how many rounds of waves (three a SIMD, 3072) the tiles
+// make, so short blocks on small grids though each computes 2K warm-up rows.
+// MI355X, lossy, npml 8, us a step, best depth/rows of a sweep beside the
+// rows the grid's nx alone gave before: 1531x2047 8/9 6.62 (before 7.03);
+// 2048^2 8/12 7.04 (10/12 8.25); 9000x500 8/20 8.35, 8/12 8.83 (11/70 18.3);
+// 2300^2 8/16 8.40 (9.89); 2500^2 10/20 9.03 (10.2); 2700^2 10/32 11.2 (14.0);
+// 3000^2 10/40 12.9 (10/17 15.8); 3500^2 11/56 17.0, 10/56 17.4 (20.2); 4096^2
+// 11/48 21.4, 11/80 21.5 (11/32 23.1); 2000x9000 11/80 22.2 (8/11 31.6);
+// 5000^2 11/72 29.7 (32.3); 7000^2 11/80 52.9, 10/80 55.3 (55.7); 8192^2 11/80
+// 72.2, 10/80 72.1, 8/96 81.5 (11/64 72.6); 12000^2 11/96 146 (148); 16384^2 with 16
+// cylinders, 44 steps, 11/96 13.5 ms, 11/128 13.6 (fewer free-space tiles).  Depths 10 and 11 keep two carry
+// sets in 3 waves per SIMD (depth 12 needs 192 VGPRs: 2 waves).
+void tm_defaults(int nx, int ny, int *depth, int *rows)
 {
-    *depth = nx >= 4096 ? 11 : (nx >= 2048 ? 10 : 8);
-    long h = nx >= 4096 && nx < 12288 ? nx / 128 : nx / 170;
-    if (h < 8) h = 8;
-    if (h > 512) h = 512;
-    *rows = (int)h;
+    const double n = (double)nx * ny;
+    *depth = n < 5.5e6 ? 8 : n < 11e6 ? 10 : 11;
+    const double h = n < 6.6e6 ? n / 330e3 : n < 100e6 ? std::min(n / 230e3, 80.0) : 96.0;
+    *rows = std::max(8, (int)h);
 }
 
 int plan_tm(const fd2d_tm_desc *d, int nsteps, Plan *pl)
@@ -229,7 +227,7 @@ int plan_tm(const fd2d_tm_desc *d, int nsteps, Plan *pl)
     if (plan_rt(d, nsteps, false, pl)) return 0;
     pl->rt = 0;
     int D0 = 8, H0 = 16;
-    tm_defaults(d->nx, &D0, &H0);
+    tm_defaults(d->nx, d->ny, &D0, &H0);
     int D = d->depth ? d->depth : (d->form == FDTD_TM_FORM_MULTIWAVE ? 8 : D0);
     int C = d->cols ? d->cols : 1;
     if (!tb_supported(D, C)) return fail("fd2d_tm: depth=%d cols=%d not supported", D, C);
@@ -240,14 +238,13 @@ int plan_tm(const fd2d_tm_desc *d, int nsteps, Plan *pl)
     if (d->form == FDTD_TM_FORM_MULTIWAVE && (C != 1 || D > MW_MAX_DEPTH))
         return fail("fd2d_tm: the multi-wave form takes one column per lane and depth <= %d "
                     "(cols=%d depth=%d)", MW_MAX_DEPTH, C, D);
-    const long h = H0;
     const int mw = d->form == FDTD_TM_FORM_MULTIWAVE;
-    int H = d->rows ? d->rows : (mw ? mw_default_rows(d->nx) : (int)h);
+    int H = d->rows ? d->rows : (mw ? mw_default_rows(d->nx) : H0);
     if (H < 1) return fail("fd2d_tm: rows=%d", H);
     // strip halo: the deepest launch's cone, rounded up to whole lanes (set
     // again below from the launches of this call)
     pl->depth = D; pl->cols = C; pl->rows = H; pl->halo = ((D + C - 1) / C) * C;
-    pl->mw = mw; pl->frows = mw ? (int)h : H;
+    pl->mw = mw; pl->frows = mw ? mw_frame_rows(d->nx) : H;
     pl->launches = 0; pl->tail_unfused = 0;
     if (nsteps <= 0) return 0;
     if (nsteps == 1) { pl->tail_unfused = 1; return 0; }
@@ -1201,7 +1198,7 @@ static int tfsf_fused(const fd2d_tm_desc *d, const fd2d_tfsf_desc *b, int t0, in
     // scratch memory); the depth changes no result
     if (!dd.depth) {
         int h;
-        tm_defaults(d->nx, &dd.depth, &h);
+        tm_defaults(d->nx, d->ny, &dd.depth, &h);
     }
     if (dd.depth > TB_MAX_TFSF_DEPTH) dd.depth = TB_MAX_TFSF_DEPTH;
     if (b->nf && !dd.rows) {

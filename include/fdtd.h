@@ -92,6 +92,11 @@ float fdtd_gaussian_f32(int t, int t0, float sigma);
 double fdtd_gaussian_f64(int t, int t0, double sigma);
 float fdtd_sinusoidal_f32(int t, float ds, float freq);
 double fdtd_sinusoidal_f64(int t, double ds, double freq);
+/* The same at t = t_first .. t_first + n - 1, into the host array out. */
+int fdtd_gaussian_fill_f32(int t_first, int n, int t0, float sigma, float *out);
+int fdtd_gaussian_fill_f64(int t_first, int n, int t0, double sigma, double *out);
+int fdtd_sinusoidal_fill_f32(int t_first, int n, float ds, float freq, float *out);
+int fdtd_sinusoidal_fill_f64(int t_first, int n, double ds, double freq, double *out);
 
 /* ------------------------------------------------------------- 1-D */
 

@@ -157,6 +157,10 @@ SIGNATURES = {
     "fdtd_gaussian_f64": (_D, [_I, _I, _D]),
     "fdtd_sinusoidal_f32": (_F, [_I, _F, _F]),
     "fdtd_sinusoidal_f64": (_D, [_I, _D, _D]),
+    "fdtd_gaussian_fill_f32": (_I, [_I, _I, _I, _F, C.POINTER(_F)]),
+    "fdtd_gaussian_fill_f64": (_I, [_I, _I, _I, _D, C.POINTER(_D)]),
+    "fdtd_sinusoidal_fill_f32": (_I, [_I, _I, _F, _F, C.POINTER(_F)]),
+    "fdtd_sinusoidal_fill_f64": (_I, [_I, _I, _D, _D, C.POINTER(_D)]),
     "fd1d_exfield": (_I, [_I, _I, _P, _P, _P, _P, _I, _I, _F, _P]),
     "fd1d_exfield_f64": (_I, [_I, _I, _P, _P, _P, _P, _I, _I, _D, _P]),
     "fd1d_hyfield": (_I, [_I, _P, _P, _P, _P]),

@@ -437,6 +437,40 @@ double fdtd_sinusoidal_f64(int t, double ds, double freq)
     return sin(2 * M_PI * freq * dt * t);
 }
 
+static int fill_check(const char *fn, int n, const void *out)
+{
+    clear_error();
+    return n < 0 || (n && !out) ? fail("%s: n=%d", fn, n) : 0;
+}
+
+int fdtd_gaussian_fill_f32(int t_first, int n, int t0, float sigma, float *out)
+{
+    const int rc = fill_check("fdtd_gaussian_fill_f32", n, out);
+    for (int s = 0; !rc && s < n; ++s) out[s] = fdtd_gaussian_f32(t_first + s, t0, sigma);
+    return rc;
+}
+
+int fdtd_gaussian_fill_f64(int t_first, int n, int t0, double sigma, double *out)
+{
+    const int rc = fill_check("fdtd_gaussian_fill_f64", n, out);
+    for (int s = 0; !rc && s < n; ++s) out[s] = fdtd_gaussian_f64(t_first + s, t0, sigma);
+    return rc;
+}
+
+int fdtd_sinusoidal_fill_f32(int t_first, int n, float ds, float freq, float *out)
+{
+    const int rc = fill_check("fdtd_sinusoidal_fill_f32", n, out);
+    for (int s = 0; !rc && s < n; ++s) out[s] = fdtd_sinusoidal_f32(t_first + s, ds, freq);
+    return rc;
+}
+
+int fdtd_sinusoidal_fill_f64(int t_first, int n, double ds, double freq, double *out)
+{
+    const int rc = fill_check("fdtd_sinusoidal_fill_f64", n, out);
+    for (int s = 0; !rc && s < n; ++s) out[s] = fdtd_sinusoidal_f64(t_first + s, ds, freq);
+    return rc;
+}
+
 // ------------------------------------------------------------------ 1-D
 
 int fd1d_exfield(int t, int nx, const float *ca, const float *cb, float *ex, const float *hy,

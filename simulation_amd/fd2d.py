@@ -22,7 +22,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._dev import fptr, ptr, require_gpu, stream
+from ._dev import fptr, pack, ptr, require_gpu, stream
 from ._lib import call
 
 # state tensors a TM descriptor points to
@@ -46,7 +46,7 @@ def time_step(ds: float = 0.01) -> float:
 def _pml_struct(pml: pmlayer | None):
     if pml is None:
         return None
-    return C.byref(_lib.FdtdPml(*[fptr(getattr(pml, k)) for k in pmlayer._fields]))
+    return C.byref(pack(_lib.FdtdPml, *[getattr(pml, k) for k in pmlayer._fields]))
 
 
 def new_pmlayer(nx: int, ny: int, device=None) -> pmlayer:
@@ -95,7 +95,7 @@ def dfield(t: int, nx: int, ny: int, pml: pmlayer | None, dz, hx, hy, sources=()
 
 def efield(nx: int, ny: int, md: medium, dz, iz, ez) -> None:
     """E from D (fd2d/pycuda/fd2d_3_4.py:175-185; md.nbz None = fd2d_3_1.py:73-82)."""
-    m = _lib.FdtdMedium(fptr(md.naz), fptr(md.nbz))
+    m = pack(_lib.FdtdMedium, md.naz, md.nbz)
     call("fd2d_efield", int(nx), int(ny), C.byref(m), ptr(dz), ptr(iz), ptr(ez), stream())
 
 
@@ -161,7 +161,7 @@ def incthy(nx: int, ny: int, npml: int, ezi, hy) -> None:
 
 
 def _ft_struct(ft: ftrans) -> _lib.FdtdFtrans:
-    return _lib.FdtdFtrans(fptr(ft.r_pt), fptr(ft.i_pt), fptr(ft.r_in), fptr(ft.i_in))
+    return pack(_lib.FdtdFtrans, *ft)
 
 
 def fourier(t: int, nf: int, nx: int, ny: int, dt: float, freq, ezi, ez, ft: ftrans) -> None:

@@ -60,21 +60,29 @@ constexpr int RMAX = ((RMAX_C > RMAX_E ? RMAX_C : RMAX_E) + 3) / 4 * 4;   // kee
 constexpr int PMAX = 136;                     // positions per workgroup (130 at K = 10)
 
 struct FrameSmem {
-    float dz[RMAX], iz[RMAX], ez[RMAX], hx[RMAX], hy[RMAX], na[RMAX], nb[RMAX];
+    // ez, hx, hy of the region (the other fields are in registers), then one
+    // element that stays 0: the source of constant samples
+    float fld[3 * RMAX + 4];
     float ring[PMAX][HIST][NS];
-    float pred[PMAX][OUT];
     float L[OUT][IN];       // linear path (FP32)
     float b1[HID], b2[HID];
-    int pos[PMAX];          // edge << 24 | tau
     int own[PMAX];          // global history index, or -1 when not owned
-    // where each sample value comes from: bits 0-11 region cell, 12-13 field
-    // (0 ez, 1 hx, 2 hy, 3 constant 0), bit 15 negate
-    uint16_t src[PMAX][NS];
+    int16_t dst[PMAX][OUT]; // region cell of each prediction, or -1
+    uint8_t by[RMAX];       // position that predicts a cell, or 255
 };
+static_assert(PMAX < 255, "positions in a byte");
 
 static_assert(sizeof(FrameSmem) + 64 <= 160 * 1024, "frame kernel LDS above 160 KiB");
 static_assert(CH + 3 * KMAX + 2 + 2 * (3 * KMAX + 3) <= PMAX && PMAX % 8 == 0,
               "positions of a frame workgroup above PMAX");
+// cells and samples of a workgroup at depth K fit n a thread
+constexpr bool fits(int K, int ncell, int nsamp)
+{
+    const int corner = (3 * K + 6) * (CH + 2 * K + 1), edge = (2 * K + 6) * (CH + 3 * K + 2);
+    return corner <= ncell * NT && edge <= ncell * NT &&
+           (CH + 3 * K + 2 + 2 * (3 * K + 3)) * NS <= nsamp * NT;
+}
+static_assert(fits(8, 3, 7) && fits(KMAX, 4, 8), "cells and samples a thread");
 
 // A workgroup's positions and sample sources depend only on the grid shape
 // and the depth: built once (frame_setup_kernel) into global memory.
@@ -300,13 +308,50 @@ __global__ void __launch_bounds__(NT) frame_setup_kernel(int nx, int ny, int K, 
     if (tid == 0) T.np = np;
 }
 
+// Lane exchanges within the vector unit (__shfl_xor goes through LDS).  lane
+// ^ 8: a rotation by 8 within rows of 16.  lane ^ 16 and lane ^ 32: the swap
+// leaves the lower row (half) of each pair in one register and the upper in
+// the other, in every lane, so a commutative operation of the two is that of
+// the lane and its partner.
+__device__ __forceinline__ float xor8(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                                 0x128 /* row_ror:8 */, 0xf, 0xf, false));
+}
+struct Pair { float a, b; };
+__device__ __forceinline__ Pair swap16(float v)
+{
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return {__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1])};
+}
+__device__ __forceinline__ Pair swap32(float v)
+{
+    const unsigned u = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return {__builtin_bit_cast(float, (unsigned)r[0]), __builtin_bit_cast(float, (unsigned)r[1])};
+}
+__device__ __forceinline__ float add16(float v) { const Pair p = swap16(v); return p.a + p.b; }
+__device__ __forceinline__ float add32(float v) { const Pair p = swap32(v); return p.a + p.b; }
+__device__ __forceinline__ float max16(float v) { const Pair p = swap16(v); return fmaxf(p.a, p.b); }
+__device__ __forceinline__ float max32(float v) { const Pair p = swap32(v); return fmaxf(p.a, p.b); }
+
+// NCELL cells and NSAMP samples a thread (3 and 7 up to depth 8, 4 and 8 up
+// to 10): fixed for the launch, so their fields and addresses stay in
+// registers (with all fields and the sample table in LDS, predictions through
+// a buffer of their own and the exchanges by __shfl_xor: 48 us a launch of 8
+// steps at 2048^2 against 36).  What bounds it is the latency of a level:
+// three phases between barriers (network with D and E; H; samples) on two
+// waves a SIMD, of which the network's exponentials and matrix products are
+// the longest.
+template <int NCELL, int NSAMP>
 __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     FrameSmem &S = *reinterpret_cast<FrameSmem *>(smem_raw);
-    const int nx = P.nx, ny = P.ny, K = P.K, W = K + 3;
+    const int nx = P.nx, ny = P.ny, K = P.K;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
-    constexpr int NW = NT / 64;
+    constexpr int NW = NT / 64, EZ = 0, HX = RMAX, HY = 2 * RMAX, ZERO = 3 * RMAX;
 
     Geo G;
     int kind, q;
@@ -318,26 +363,52 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
     const int np = T.np;
     __shared__ int nact_s[KMAX + 4];
     if (tid <= K) nact_s[tid] = T.nact[tid];
-    for (int k = tid; k < np; k += NT) {
-        S.pos[k] = T.pos[k];
-        S.own[k] = T.own[k];
-    }
-    {
-        const uint32_t *s32 = reinterpret_cast<const uint32_t *>(&T.src[0][0]);
-        uint32_t *d32 = reinterpret_cast<uint32_t *>(&S.src[0][0]);
-        for (int k = tid; k < np * NS / 2; k += NT) d32[k] = s32[k];
-    }
+    for (int k = tid; k < np; k += NT) S.own[k] = T.own[k];
+    for (int k = tid; k < RMAX / 4; k += NT) reinterpret_cast<uint32_t *>(S.by)[k] = 0xFFFFFFFFu;
+    if (tid == 0) S.fld[ZERO] = 0.0f;
     // ---------------------------------------------------------- load
-    for (int k = tid; k < RH * RW; k += NT) {
-        const int r = k / RW, cc = k % RW;
-        const long o = (long)(G.ri0 + r) * ny + (G.rj0 + cc);
-        S.dz[k] = P.dz_i[o];
-        S.iz[k] = P.iz_i ? P.iz_i[o] : 0.0f;
-        S.hx[k] = P.hx_i[o];
-        S.hy[k] = P.hy_i[o];
-        S.na[k] = P.naz[o];
-        S.nb[k] = P.nbz ? P.nbz[o] : 0.0f;
-        S.ez[k] = 0.0f;
+    // thread tid holds cells tid + n NT
+    float dz[NCELL], iz[NCELL], hx[NCELL], hy[NCELL], na[NCELL], nb[NCELL];
+    const int DR = NT / RW, DC = NT % RW;
+    unsigned e_ok = 0, h_ok = 0, mine = 0;       // bit n: D update, H update, owned
+    {
+        int r = tid / RW, cc = tid % RW;
+#pragma unroll
+        for (int n = 0; n < NCELL; ++n) {
+            const int k = tid + n * NT;
+            dz[n] = iz[n] = hx[n] = hy[n] = na[n] = nb[n] = 0.0f;
+            if (k < NC) {
+                const int i = G.ri0 + r, j = G.rj0 + cc;
+                const long o = (long)i * ny + j;
+                dz[n] = P.dz_i[o];
+                iz[n] = P.iz_i ? P.iz_i[o] : 0.0f;
+                hx[n] = P.hx_i[o];
+                hy[n] = P.hy_i[o];
+                na[n] = P.naz[o];
+                nb[n] = P.nbz ? P.nbz[o] : 0.0f;
+                S.fld[EZ + k] = 0.0f;
+                S.fld[HX + k] = hx[n];
+                S.fld[HY + k] = hy[n];
+                if (i >= 1 && j >= 1 && r >= 1 && cc >= 1) e_ok |= 1u << n;
+                if (i < nx - 1 && j < ny - 1 && r + 1 < RH && cc + 1 < RW) h_ok |= 1u << n;
+                if (i >= G.oi0 && i < G.oi1 && j >= G.oj0 && j < G.oj1) mine |= 1u << n;
+            }
+            r += DR; cc += DC;
+            if (cc >= RW) { cc -= RW; ++r; }
+        }
+    }
+    // thread tid takes samples tid + n NT (position / NS, sample % NS): the
+    // element of fld and bit 31 for a negated one
+    unsigned from[NSAMP];
+    {
+        const uint16_t *src = &T.src[0][0];
+#pragma unroll
+        for (int n = 0; n < NSAMP; ++n) {
+            const int k = tid + n * NT;
+            const unsigned sv = k < np * NS ? src[k] : 3u << 12;
+            const unsigned f = (sv >> 12) & 3u;
+            from[n] = (f == 3u ? (unsigned)ZERO : f * RMAX + (sv & 0xFFFu)) | (sv & 0x8000u) << 16;
+        }
     }
     // history ring: the sample of level l (l = -3..K) in slot (-l) & 3, so
     // the history's ages 0..3 (levels 0, -1, -2, -3) land in slots 0..3: one
@@ -361,21 +432,33 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
     // nothing (y = 0, so the odd part 0.5 (y - y') is +0, as computed): skip
     // those layers
     const bool mlp = P.w[W_MLP] != 0;
-    // cell loops without divisions: thread tid starts at cell tid and steps
-    // by NT = DR rows + DC columns
-    const int DR = NT / RW, DC = NT % RW;
-    const int r_start = tid / RW, c_start = tid % RW;
     __syncthreads();
+    // where predictions go, and which cells they replace (no cell has two:
+    // the top and bottom edges own the corners)
+    for (int k = tid; k < np * OUT; k += NT) {
+        const int p = k / OUT, d = k % OUT;
+        const int ps = T.pos[p], e = ps >> 24, t = ps & 0xFFFFFF;
+        int i, j;
+        cell_of(e, d, t, nx, ny, i, j);
+        const int r = i - G.ri0, cc = j - G.rj0;
+        const bool in = r >= 0 && r < RH && cc >= 0 && cc < RW;
+        S.dst[p][d] = (int16_t)(in ? r * RW + cc : -1);
+        if (in) S.by[r * RW + cc] = (uint8_t)p;
+    }
+    __syncthreads();
+    int by[NCELL];
+#pragma unroll
+    for (int n = 0; n < NCELL; ++n) by[n] = tid + n * NT < NC ? S.by[tid + n * NT] : 255;
 
     for (int lev = 1; lev <= K; ++lev) {
         // ------------------------------------------------------ network
-        // tiles of 8 positions, tile q on wave q % NW; no barrier before the
-        // D/E update, which touches neither the ring nor pred
-        const int na = nact_s[lev];
-        for (int tb = wave * 8; tb < na; tb += NW * 8) {
+        // tiles of 8 positions, tile q on wave q % NW; predictions go
+        // straight to ez, where the E update leaves their cells alone
+        const int npos = nact_s[lev];
+        for (int tb = wave * 8; tb < npos; tb += NW * 8) {
             const int q = tb + (c & 7);
             float x[NF];
-            if (q < na) {
+            if (q < npos) {
                 const float *src = S.ring[q][(g + 1 - lev) & 3];   // level lev - 1 - g
 #pragma unroll
                 for (int i = 0; i < NF; ++i) x[i] = src[i];
@@ -386,8 +469,8 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
             float mx = 0.0f;
 #pragma unroll
             for (int i = 0; i < NF; ++i) mx = fmaxf(mx, fabsf(x[i]));
-            mx = fmaxf(mx, __shfl_xor(mx, 16));
-            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            mx = max16(mx);
+            mx = max32(mx);
             const float inv = mx > S_MIN ? 1.0f / mx : 0.0f;
             // FP32 linear path: lanes c and c + 8 hold the same position and
             // split its 27 features of age g (0..13 and 14..26)
@@ -407,9 +490,9 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
 #pragma unroll
                     for (int i = 0; i < 14; ++i)
                         if (i < 13 || c < 8) a = __builtin_fmaf(w[i], xs[i], a);
-                    a = a + __shfl_xor(a, 8);
-                    a = a + __shfl_xor(a, 16);
-                    a = a + __shfl_xor(a, 32);
+                    a = a + xor8(a);
+                    a = add16(a);
+                    a = add32(a);
                     lin[o] = a;
                 }
             }
@@ -455,80 +538,80 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
             // column pair (c, c + 8)
 #pragma unroll
             for (int v = 0; v < OUT; ++v) {
-                const float other = __shfl_xor(y[v], 8);
-                if (g == 0 && c < 8 && q < na) {
+                const float other = xor8(y[v]);
+                if (g == 0 && c < 8 && q < npos) {
                     const float yo = 0.5f * (y[v] - other);
                     const float b = base_of(v, S.ring[q][(2 - lev) & 3]);
-                    S.pred[q][v] = mx > S_MIN ? b + mx * (lin[v] + yo) : b;
+                    const int d = S.dst[q][v];
+                    if (d >= 0) S.fld[EZ + d] = mx > S_MIN ? b + mx * (lin[v] + yo) : b;
                 }
             }
         }
         // ------------------------------------------------------ D, E update
-        for (int k = tid, r = r_start, cc = c_start; k < NC; k += NT) {
-            const int i = G.ri0 + r, j = G.rj0 + cc;
-            float dz = S.dz[k];
-            if (i >= 1 && j >= 1 && r >= 1 && cc >= 1) {
-                const float curl = S.hy[k] - S.hy[k - RW] - S.hx[k] + S.hx[k - 1];
-                dz = dz + 0.5f * curl;
-                S.dz[k] = dz;
+#pragma unroll
+        for (int n = 0; n < NCELL; ++n) {
+            const int k = tid + n * NT;
+            if (e_ok >> n & 1u) {
+                const float curl = hy[n] - S.fld[HY + k - RW] - hx[n] + S.fld[HX + k - 1];
+                dz[n] = dz[n] + 0.5f * curl;
             }
+            float ez;
             if (P.nbz) {
-                const float iz = S.iz[k];
-                const float ez = S.na[k] * (dz - iz);
-                S.ez[k] = ez;
-                S.iz[k] = iz + S.nb[k] * ez;
+                ez = na[n] * (dz[n] - iz[n]);
+                iz[n] = iz[n] + nb[n] * ez;
             } else {
-                S.ez[k] = S.na[k] * dz;
+                ez = na[n] * dz[n];
             }
-            r += DR; cc += DC;
-            if (cc >= RW) { cc -= RW; ++r; }
-        }
-        __syncthreads();
-        // ------------------------------------------------------ learned cells
-        for (int k = tid; k < na * OUT; k += NT) {
-            const int p = k / OUT, d = k % OUT;
-            const int e = S.pos[p] >> 24, t = S.pos[p] & 0xFFFFFF;
-            int i, j;
-            cell_of(e, d, t, nx, ny, i, j);
-            const int r = i - G.ri0, cc = j - G.rj0;
-            if (r >= 0 && r < RH && cc >= 0 && cc < RW) S.ez[r * RW + cc] = S.pred[p][d];
+            if (k < NC && by[n] >= npos) S.fld[EZ + k] = ez;
         }
         __syncthreads();
         // ------------------------------------------------------ H update
-        for (int k = tid, r = r_start, cc = c_start; k < NC; k += NT) {
-            const int i = G.ri0 + r, j = G.rj0 + cc;
-            if (i < nx - 1 && j < ny - 1 && r + 1 < RH && cc + 1 < RW) {
-                const float ez = S.ez[k];
-                S.hx[k] = S.hx[k] + 0.5f * (ez - S.ez[k + 1]);
-                S.hy[k] = S.hy[k] - 0.5f * (ez - S.ez[k + RW]);
+#pragma unroll
+        for (int n = 0; n < NCELL; ++n) {
+            const int k = tid + n * NT;
+            if (h_ok >> n & 1u) {
+                const float ez = S.fld[EZ + k];
+                hx[n] = hx[n] + 0.5f * (ez - S.fld[EZ + k + 1]);
+                hy[n] = hy[n] - 0.5f * (ez - S.fld[EZ + k + RW]);
+                S.fld[HX + k] = hx[n];
+                S.fld[HY + k] = hy[n];
             }
-            r += DR; cc += DC;
-            if (cc >= RW) { cc -= RW; ++r; }
         }
         __syncthreads();
         // ------------------------------------------------------ new samples
-        for (int k = tid; k < na * NS; k += NT) {
-            const int p = k / NS, i = k % NS;
-            const unsigned sv = S.src[p][i];
-            const unsigned f = (sv >> 12) & 3u, cell = sv & 0xFFFu;
-            float v = f == 0 ? S.ez[cell] : (f == 1 ? S.hx[cell] : (f == 2 ? S.hy[cell] : 0.0f));
-            if (sv & 0x8000u) v = -v;
-            S.ring[p][(-lev) & 3][i] = v;
+        {
+            float *ring = &S.ring[0][(-lev) & 3][0];
+            int p = tid / NS, i = tid % NS;
+#pragma unroll
+            for (int n = 0; n < NSAMP; ++n) {
+                if (p < npos) {
+                    const float v = S.fld[from[n] & 0x7FFFFFFFu];
+                    ring[p * (HIST * NS) + i] =
+                        __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) ^ (from[n] & 0x80000000u));
+                }
+                p += NT / NS; i += NT % NS;
+                if (i >= NS) { i -= NS; ++p; }
+            }
         }
         __syncthreads();
     }
 
     // ---------------------------------------------------------- store
-    for (int k = tid; k < NC; k += NT) {
-        const int r = k / RW, cc = k % RW;
-        const int i = G.ri0 + r, j = G.rj0 + cc;
-        if (i < G.oi0 || i >= G.oi1 || j < G.oj0 || j >= G.oj1) continue;
-        const long o = (long)i * ny + j;
-        P.dz_o[o] = S.dz[k];
-        if (P.iz_o) P.iz_o[o] = S.iz[k];
-        P.hx_o[o] = S.hx[k];
-        P.hy_o[o] = S.hy[k];
-        if (P.ez_o) P.ez_o[o] = S.ez[k];
+    {
+        int r = tid / RW, cc = tid % RW;
+#pragma unroll
+        for (int n = 0; n < NCELL; ++n) {
+            if (mine >> n & 1u) {
+                const long o = (long)(G.ri0 + r) * ny + (G.rj0 + cc);
+                P.dz_o[o] = dz[n];
+                if (P.iz_o) P.iz_o[o] = iz[n];
+                P.hx_o[o] = hx[n];
+                P.hy_o[o] = hy[n];
+                if (P.ez_o) P.ez_o[o] = S.fld[EZ + tid + n * NT];
+            }
+            r += DR; cc += DC;
+            if (cc >= RW) { cc -= RW; ++r; }
+        }
     }
     for (int k = tid; k < np * HIST * NS; k += NT) {
         const int p = k / (HIST * NS), a = (k / NS) % HIST, i = k % NS;
@@ -574,16 +657,18 @@ int lbc_frame_blocks(int nx, int ny, int K)
 
 int launch_lbc_frame(const LbcFrameParams &p, hipStream_t s)
 {
-    static thread_local bool attr = false;
-    if (!attr) {
-        int rc = hip_check(hipFuncSetAttribute((const void *)lbc::frame_kernel,
+    const bool deep = p.K > 8;
+    const auto kernel = deep ? &lbc::frame_kernel<4, 8> : &lbc::frame_kernel<3, 7>;
+    static thread_local bool attr[2] = {};
+    if (!attr[deep]) {
+        int rc = hip_check(hipFuncSetAttribute((const void *)kernel,
                                                hipFuncAttributeMaxDynamicSharedMemorySize,
                                                (int)sizeof(lbc::FrameSmem)),
                            "lbc frame: shared memory");
         if (rc) return rc;
-        attr = true;
+        attr[deep] = true;
     }
-    hipLaunchKernelGGL(lbc::frame_kernel, dim3(lbc_frame_blocks(p.nx, p.ny, p.K)), dim3(lbc::NT),
+    hipLaunchKernelGGL(kernel, dim3(lbc_frame_blocks(p.nx, p.ny, p.K)), dim3(lbc::NT),
                        sizeof(lbc::FrameSmem), s, p);
     return hip_check(hipGetLastError(), "lbc frame kernel");
 }

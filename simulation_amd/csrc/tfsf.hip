@@ -161,10 +161,17 @@ __global__ void __launch_bounds__(1024) inc_chunk_kernel(int ny, float *ezi, flo
 // neighbour.  A step then needs DPP shifts only; every INC_HALO steps the
 // waves pass their owned edge cells through LDS.  The chunk's source values
 // and twiddles sit one step a lane.  What bounds it is the chain of one step
-// (some 25 dependent operations).  MI355X, 64 steps, with the launch: ny 150
-// ~60 us with the grid in LDS (four barriers a step), ~110 us with the probe's
-// DFT (a round trip to memory a step).
+// (some 25 dependent operations) and the two barriers every INC_HALO steps.
+// MI355X, ny 1024, three frequencies, 64 steps: 72 us with the grid in LDS
+// (four barriers a step, the probe's transforms through memory), 27 us with
+// branches around the table's stores, 21 us.
 constexpr int INC_HALO = 8;
+
+// LDS traffic done, then the barrier: the table's stores stay in flight
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
 
 template <int M>
 __global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi, float *hxi,
@@ -202,6 +209,18 @@ __global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi,
     }
     const bool src = a.inc_pos >= base && a.inc_pos < base + S;
     const bool right = ny - 1 < base + S;                        // the window holds cell ny-1
+    // a step's table row: byte offsets of the lane's cells in it, past its end
+    // where a cell is not the wave's to store (the range check drops those:
+    // no branches in a step)
+    unsigned eoff[M], hoff[M];
+#pragma unroll
+    for (int c = 0; c < M; ++c) {
+        const int j = j0 + c;
+        const bool own = j >= o0 && j < o1;
+        eoff[c] = own && j >= m - 1 && j <= ny - m ? (unsigned)(2 + j - (m - 1)) * 4u : 0xFFFFFFFCu;
+        hoff[c] = own && j == m - 2 ? 0u : own && j == ny - m ? 4u : 0xFFFFFFFCu;
+    }
+    const bool side = (m - 2 >= o0 && m - 2 < o1) || (ny - m >= o0 && ny - m < o1);
     // cell j's value (in the window), in every lane
     auto cell = [&](const float (&v)[M], int j) __attribute__((always_inline)) {
         const int k = j - base;
@@ -217,7 +236,7 @@ __global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi,
         for (int c = M - 1; c >= 0; --c) e[c] = e[c] + 0.5f * ((c ? h[c ? c - 1 : 0] : hl) - h[c]);
         // two-step boundary (it replaces cells 0 and ny-1), then the source
         if (w == 0) {
-            if (lane == 0) e[0] = b0;
+            e[0] = lane == 0 ? b0 : e[0];
             b0 = b1;
             b1 = cell(e, 1);
         }
@@ -232,15 +251,15 @@ __global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi,
 #pragma unroll
             for (int c = 0; c < M; ++c) e[c] = j0 + c == a.inc_pos ? v : e[c];
         }
-        float *row = table + (size_t)s * a.stride;
+        const auto row = __builtin_amdgcn_make_buffer_rsrc(table + (size_t)s * a.stride, (short)0,
+                                                           a.stride * 4, 0x00020000);
 #pragma unroll
-        for (int c = 0; c < M; ++c) {
-            const int j = j0 + c;
-            if (j >= o0 && j < o1) {
-                if (j >= m - 1 && j <= ny - m) row[2 + j - (m - 1)] = e[c];
-                if (j == m - 2) row[0] = h[c];
-                if (j == ny - m) row[1] = h[c];
-            }
+        for (int c = 0; c < M; ++c)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, e[c]), row, eoff[c], 0, 0);
+        if (side) {
+#pragma unroll
+            for (int c = 0; c < M; ++c)
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, h[c]), row, hoff[c], 0, 0);
         }
         if (dft) {
             const float v = cell(e, a.probe);
@@ -266,7 +285,7 @@ __global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi,
                     xch[w][1][1][k - (S - 2 * H)] = h[c];
                 }
             }
-            __syncthreads();
+            lds_barrier();
 #pragma unroll
             for (int c = 0; c < M; ++c) {
                 const int k = k0 + c;
@@ -276,7 +295,7 @@ __global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi,
                     h[c] = xch[w + 1][0][1][k - (S - H)];
                 }
             }
-            __syncthreads();
+            lds_barrier();
         }
     }
 #pragma unroll

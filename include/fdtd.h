@@ -356,7 +356,8 @@ typedef struct fd2d_batch_desc {
     int nunits;
     int depth, rows, cols;        /* fixed when the work list is made */
     int waves;                    /* workgroups of a launch */
-    int vec;                      /* 1: every grid allows vector loads */
+    int vec;                      /* 1: every grid allows vector loads; 2:
+                                     register tiles (rows: of a tile) */
     int wave_len;                 /* smallest wave_len over grids with a source
                                      (INT_MAX: none), set by fd2d_batch_upload */
     int probe_len;                /* smallest probe_len over grids with a probe
@@ -374,10 +375,12 @@ typedef struct fd2d_batch_desc {
 } fd2d_batch_desc;
 
 /* Number of work units (and so ints/4 of units_dev) a batch needs for the
- * given depth, rows per block (both 0: by the cells of all grids, 6 and 12
- * below 5 million, 8 and 24 below 8 million, 10 and 32 below 30 million, else
- * 10 and 48) and columns per lane (0 = 1).  A unit is 4 ints: grid, strip,
- * first row, one past the last row.                                       */
+ * given depth, rows per block (0: by the cells of all grids, 6 and 12 below 5
+ * million, 8 and 24 below 8 million, 10 and 32 below 30 million, else 10 and
+ * 48) and columns per lane (0 = 1).  A unit is 4 ints: grid, strip, first
+ * row, one past the last row.  With all three 0 and less than 5 million cells
+ * the batch runs register tiles, as a small single grid does: grid, tile
+ * column, tile row, 0.                                                     */
 int fd2d_batch_units(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols,
                      int *nunits);
 

@@ -62,29 +62,37 @@ template <int N> struct Int { static constexpr int v = N; };
 
 constexpr int R = RT_ROWS;
 
-template <bool LOSSY, bool PML, bool TF, int NF>
-__global__ void __launch_bounds__(64 * RT_WAVES) tm_rt_kernel(const RtParams P)
-{
-    __shared__ float up[RT_WAVES + 1][64];   // up[w]: hy of the row above wave w's first
-    __shared__ float dn[RT_WAVES + 1][64];   // dn[w]: ez of wave w's first row
-    __shared__ float srcv[FDTD_MAX_SOURCES * RT_MAX_STEPS];
+struct RtSmem {
+    float up[RT_WAVES + 1][64];   // up[w]: hy of the row above wave w's first
+    float dn[RT_WAVES + 1][64];   // dn[w]: ez of wave w's first row
+    float src[FDTD_MAX_SOURCES * RT_MAX_STEPS];
+};
 
+// Tiles along n cells: spans of `span` cells that share 2H with each neighbour.
+__host__ __device__ inline int rt_along(int n, int span, int H)
+{
+    return n <= span ? 1 : 1 + (n - span + span - 2 * H - 1) / (span - 2 * H);
+}
+
+// Tile (by, bx) of nsy x nsx, P.K steps; H >= P.K: the overlap the tiles are
+// cut with.  PR: RtParams or RtGrid.
+template <bool LOSSY, bool PML, bool TF, int NF, class PR>
+__device__ __forceinline__ void rt_tile(PR &P, int H, int bx, int by, int nsx, int nsy,
+                                        RtSmem &S)
+{
+    auto &up = S.up;
+    auto &dn = S.dn;
+    auto &srcv = S.src;
     const int nx = P.nx, ny = P.ny, K = P.K;
     const int W = (int)blockDim.x >> 6, T = W * R;
     const int lane = (int)threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    // workgroup L runs on XCD L % 8: the workgroups of one XCD take a
-    // contiguous run of tiles, which share their halos in its L2
-    const unsigned nt = gridDim.x, xcd = blockIdx.x % 8u, q8 = nt / 8u, rem = nt % 8u;
-    const unsigned tile = xcd * q8 + min(xcd, rem) + blockIdx.x / 8u;
-    const int bx = (int)(tile % (unsigned)P.nsx), by = (int)(tile / (unsigned)P.nsx);
-    const int nsy = (int)(nt / (unsigned)P.nsx);
     // the tile's window starts at (bi, bj) -- the last one of a row or column
     // ends with the grid -- and its own cells are rows [o0, o1), columns [c0, c1)
-    const int bi = min(by * (T - 2 * K), max(nx - T, 0));
-    const int bj = min(bx * (64 - 2 * K), max(ny - 64, 0));
-    const int o0 = by ? by * (T - 2 * K) + K : 0, o1 = by == nsy - 1 ? nx : by * (T - 2 * K) + T - K;
-    const int c0 = bx ? bx * (64 - 2 * K) + K : 0, c1 = bx == P.nsx - 1 ? ny : bx * (64 - 2 * K) + 64 - K;
+    const int bi = min(by * (T - 2 * H), max(nx - T, 0));
+    const int bj = min(bx * (64 - 2 * H), max(ny - 64, 0));
+    const int o0 = by ? by * (T - 2 * H) + H : 0, o1 = by == nsy - 1 ? nx : by * (T - 2 * H) + T - H;
+    const int c0 = bx ? bx * (64 - 2 * H) + H : 0, c1 = bx == nsx - 1 ? ny : bx * (64 - 2 * H) + 64 - H;
     const int i0 = bi + w * R, j = bj + lane, jc = min(j, ny - 1);
     const bool own_col = j >= c0 && j < c1;
 
@@ -330,6 +338,7 @@ __global__ void __launch_bounds__(64 * RT_WAVES) tm_rt_kernel(const RtParams P)
         lds_barrier();
     }
     if (!rows_own || !own_col) return;
+    P.outputs();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int i = i0 + r;
@@ -352,6 +361,107 @@ __global__ void __launch_bounds__(64 * RT_WAVES) tm_rt_kernel(const RtParams P)
     }
 }
 
+// workgroup b of n runs on XCD b % 8: the workgroups of one XCD take a
+// contiguous run of tiles, which share their halos in its L2
+__device__ __forceinline__ unsigned rt_slot(unsigned b, unsigned n)
+{
+    const unsigned xcd = b % 8u;
+    return xcd * (n / 8u) + min(xcd, n % 8u) + b / 8u;
+}
+
+template <bool LOSSY, bool PML, bool TF, int NF>
+__global__ void __launch_bounds__(64 * RT_WAVES) tm_rt_kernel(const RtParams P)
+{
+    __shared__ RtSmem S;
+    const unsigned tile = rt_slot(blockIdx.x, gridDim.x), nsx = (unsigned)P.nsx;
+    rt_tile<LOSSY, PML, TF, NF>(P, P.K, (int)(tile % nsx), (int)(tile / nsx), P.nsx,
+                                (int)(gridDim.x / nsx), S);
+}
+
+// One grid of a batch (fd2d_grid): at most one source and one probe.
+struct RtGrid {
+    const fd2d_grid *g;
+    bool swap, write_ez;            // odd launches read the partner set
+    int nx, ny, K;
+    const float *dz_i, *iz_i, *hx_i, *hy_i, *ihx_i, *ihy_i;
+    float *dz_o, *iz_o, *hx_o, *hy_o, *ihx_o, *ihy_o, *ez_o;
+    const float *naz, *nbz;
+    PmlPtrs pml;
+    int rlo, rhi, clo, chi;
+    int t_first;
+    struct One {
+        int v;
+        __device__ int operator[](int) const { return v; }
+    };
+    int nsrc;
+    One src_i, src_j;
+    const float *src_wave;
+    int wave_len;
+    int nprobe;
+    One probe_i, probe_j;
+    float *probe_out;
+    int probe_len;
+    static constexpr int tf_npml = 0, inc_t0 = 0, inc_stride = 0;
+    static constexpr const float *inc = nullptr;
+    // read from the record when the steps are done: kept over them, the
+    // pointers cost 26 scalar registers, which spill into vector ones (88 of
+    // those a lane instead of 80: two tiles a CU instead of three)
+    __device__ __forceinline__ void outputs()
+    {
+        asm volatile("" : "+s"(g));
+        dz_o = swap ? g->dz : g->dz2;
+        iz_o = swap ? g->iz : g->iz2;
+        hx_o = swap ? g->hx : g->hx2;
+        hy_o = swap ? g->hy : g->hy2;
+        ihx_o = swap ? g->ihx : g->ihx2;
+        ihy_o = swap ? g->ihy : g->ihy2;
+        ez_o = write_ez ? g->ez : nullptr;
+    }
+};
+
+// Many grids, one workgroup a tile or fewer that take several; units: grid,
+// tile column, tile row.  Lossy PML form.  Six waves a SIMD: two 12-wave tiles
+// a CU.
+__global__ void __launch_bounds__(64 * RT_WAVES) __attribute__((amdgpu_waves_per_eu(6)))
+tm_rt_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ units, int nunits,
+                   int K, int H, int parity, int t_first, int write_ez)
+{
+    __shared__ RtSmem S;
+    const int T = ((int)blockDim.x >> 6) * R;
+    for (int u = (int)rt_slot(blockIdx.x, gridDim.x); u < nunits; u += (int)gridDim.x) {
+        const int gi = units[4 * u], bx = units[4 * u + 1], by = units[4 * u + 2];
+        const fd2d_grid &G = grids[gi];
+        RtGrid P;
+        P.g = &G;
+        P.swap = parity != 0;
+        P.write_ez = write_ez != 0;
+        P.nx = G.nx; P.ny = G.ny; P.K = K;
+        P.dz_i = P.swap ? G.dz2 : G.dz;
+        P.iz_i = P.swap ? G.iz2 : G.iz;
+        P.hx_i = P.swap ? G.hx2 : G.hx;
+        P.hy_i = P.swap ? G.hy2 : G.hy;
+        P.ihx_i = P.swap ? G.ihx2 : G.ihx;
+        P.ihy_i = P.swap ? G.ihy2 : G.ihy;
+        P.naz = G.md.naz; P.nbz = G.md.nbz;
+        P.pml = PmlPtrs{G.pml.fx1, G.pml.fx2, G.pml.fx3, G.pml.fy1, G.pml.fy2, G.pml.fy3,
+                        G.pml.gx2, G.pml.gx3, G.pml.gy2, G.pml.gy3};
+        const int *br = G.band_rows, *bc = G.band_cols;
+        P.rlo = br[1] > br[0] ? max(br[0], 1) : 0;
+        P.rhi = br[1] > br[0] ? min(br[1], G.nx - 1) : 0;
+        P.clo = bc[1] > bc[0] ? max(bc[0], 1) : 0;
+        P.chi = bc[1] > bc[0] ? min(bc[1], G.ny - 1) : 0;
+        P.t_first = t_first;
+        P.nsrc = G.src_i >= 0 ? 1 : 0;
+        P.src_i.v = G.src_i; P.src_j.v = G.src_j;
+        P.src_wave = G.src_wave; P.wave_len = G.wave_len;
+        P.nprobe = G.probe_i >= 0 ? 1 : 0;
+        P.probe_i.v = G.probe_i; P.probe_j.v = G.probe_j;
+        P.probe_out = G.probe_out; P.probe_len = G.probe_len;
+        rt_tile<true, true, false, 0>(P, H, bx, by, rt_along(G.ny, 64, H), rt_along(G.nx, T, H), S);
+        lds_barrier();                        // the next tile rewrites S
+    }
+}
+
 template <bool TF, int NF>
 void launch_form(const RtParams &p, int waves, int tiles, bool lossy, bool pml, hipStream_t s)
 {
@@ -368,10 +478,7 @@ void launch_form(const RtParams &p, int waves, int tiles, bool lossy, bool pml, 
 
 int rt_tiles(int nx, int ny, int waves, int K)
 {
-    auto along = [K](int n, int span) {
-        return n <= span ? 1 : 1 + (n - span + span - 2 * K - 1) / (span - 2 * K);
-    };
-    return along(nx, waves * R) * along(ny, 64);
+    return rt_along(nx, waves * R, K) * rt_along(ny, 64, K);
 }
 
 int preload_rt()
@@ -396,6 +503,16 @@ int launch_fd2d_rt(const RtParams &p, int waves, int nf, bool lossy, bool pml, h
     else if (nf == 3) launch_form<true, 3>(q, waves, tiles, lossy, pml, s);
     else return fail("register tiles: %d frequencies", nf);
     return hip_check(hipGetLastError(), "register tiles launch");
+}
+
+int launch_fd2d_rt_batch(const fd2d_grid *grids, const int *units, int nunits, int groups, int waves,
+                         int K, int H, int parity, int t_first, int write_ez, hipStream_t s)
+{
+    if (waves < 1 || waves > RT_WAVES || K < 1 || K > H || H > RT_MAX_STEPS || 2 * H >= waves * R)
+        return fail("register tiles: %d of %d steps a launch in tiles of %dx64", K, H, waves * R);
+    hipLaunchKernelGGL(tm_rt_batch_kernel, dim3(groups), dim3(64 * waves), 0, s, grids, units, nunits,
+                       K, H, parity, t_first, write_ez);
+    return hip_check(hipGetLastError(), "fd2d_batch_run launch");
 }
 
 }  // namespace fdtd

@@ -136,8 +136,8 @@ struct Plan {
     int rt;                // 1: register tiles (depth: steps of a launch, rows: of a tile)
 };
 
-// Register tiles (fd2d_rt.hip), where the caller leaves form, depth, rows and
-// columns to the library and the grid is small enough; tf: a plane-wave run.
+// Waves and depth (*K) of register tiles (fd2d_rt.hip) by the number of tiles
+// a shape makes, tiles(waves, depth).
 // MI355X, us of 192 steps (lossy, npml 8; strips / tiles of 8, 12, 16 waves
 // at their best depth): 400^2 1070 / 274, 286, 293; 500^2 1089 / 323, 309,
 // 305; 600^2 1080 / 349, 353, 350; 850^2 1108 / 518, 466, 572; 1100^2 1109 /
@@ -151,29 +151,29 @@ struct Plan {
 // 150^2 2038 / 784 at depth 12, 832 at 8; 400^2 2191 / 953, 863; 1024^2 3413
 // / 2378, 1914; 1500^2 4970 / 3972, 2961; 128 steps: 4096^2 17230 / 9342 with
 // three frequencies, 6990 / 6555 without.
+template <class Tiles>
+int rt_shape(const Tiles &tiles, int *K)
+{
+    for (int k : {14, 12, 10, 8})
+        if (tiles(8, *K = k) <= 256) return 8;
+    for (int most : {256, 512})
+        for (int k : {12, 10, 8})
+            if (tiles(12, *K = k) <= most) return 12;
+    *K = 7;
+    return 8;
+}
+
+// Register tiles, where the caller leaves form, depth, rows and columns to the
+// library and the grid is small enough; tf: a plane-wave run.
 constexpr long RT_MAX_CELLS = 2700000, RT_MAX_CELLS_TF = 17000000;
 bool plan_rt(const fd2d_tm_desc *d, int nsteps, bool tf, Plan *pl)
 {
     if (d->form != FDTD_TM_FORM_AUTO || d->depth || d->rows || d->cols || nsteps < 2) return false;
     if ((long)d->nx * d->ny > (tf ? RT_MAX_CELLS_TF : RT_MAX_CELLS)) return false;
-    auto deepest = [&](int waves, std::initializer_list<int> depths, int most) {
-        for (int k : depths)
-            if (rt_tiles(d->nx, d->ny, waves, k) <= most) return k;
-        return 0;
-    };
+    auto tiles = [&](int waves, int k) { return rt_tiles(d->nx, d->ny, waves, k); };
     int W = 8, K;
-    if (tf) {
-        K = deepest(8, {12}, 256);
-        if (!K) K = 8;
-    } else {
-        K = deepest(8, {14, 12, 10, 8}, 256);
-        if (!K) {
-            W = 12;
-            K = deepest(12, {12, 10, 8}, 256);
-            if (!K) K = deepest(12, {12, 10, 8}, 512);
-            if (!K) { W = 8; K = 7; }
-        }
-    }
+    if (tf) K = tiles(8, 12) <= 256 ? 12 : 8;
+    else W = rt_shape(tiles, &K);
     // an even number of launches: the result ends in the caller's state set
     int L = (nsteps + K - 1) / K;
     L += L % 2;
@@ -301,11 +301,18 @@ int aux_for_current_device(Aux **out)
 
 struct BatchGeom {
     int depth, rows, cols, halo;
+    bool tiles;                    // register tiles (rows: of a tile)
 };
 
 // The launch shape of a batch; depth, rows, cols 0: the library's choice, by
-// the cells of all grids together -- few cells want many short units, whose
-// warm-up rows cost less than idle SIMDs.  MI355X, ms of 120 steps at depth /
+// the cells of all grids together.  Below 5 million: register tiles, in the
+// shape a single grid of that many tiles has, past two tiles a CU 12 waves at
+// depth 8.  MI355X, us of 112 steps, strips (at their best shape below) / tiles
+// of 8 waves, depth 7 / 12 waves, depth 8 / 12: sides 96-250, 0.5M cells: 807 /
+// 329 / 333 / 282; 150-500, 1.8M: 950 / 677 / 652 / 705; 96-200, 4.5M: 1986 /
+// 1730 / 1563 / 1640; 300-500, 6.6M: 1733 / 2566 / 2161 / 2317.
+// Strips -- few cells want many short units, whose warm-up rows cost less
+// than idle SIMDs.  MI355X, ms of 120 steps at depth /
 // rows, sides and cells: 96-200, 4.5M: 6/12 2.38, 8/24 2.74, 10/32 3.34;
 // 300-500, 6.6M: 2.60, 2.16, 2.61; 700-900, 10M: 3.65, 2.83, 2.64; 300-700,
 // 27M: 10.4, 7.91, 7.23; 150-900, 38M: 13.7, 10.4, 9.56 (10/48: 9.56);
@@ -315,6 +322,23 @@ int batch_geom(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols
 {
     long long cells = 0;
     for (int k = 0; k < ngrids; ++k) cells += (long long)grids[k].nx * grids[k].ny;
+    g->tiles = !depth && !rows && !cols && cells < 5000000;
+    if (g->tiles) {
+        auto tiles = [&](int waves, int K) {
+            long long n = 0;
+            for (int k = 0; k < ngrids; ++k) n += rt_tiles(grids[k].nx, grids[k].ny, waves, K);
+            return n;
+        };
+        int W = rt_shape(tiles, &g->depth);
+        if (tiles(W, g->depth) > 512) {
+            W = 12;
+            g->depth = 8;
+        }
+        g->rows = W * RT_ROWS;
+        g->cols = 1;
+        g->halo = g->depth;
+        return 0;
+    }
     g->depth = depth ? depth : cells < 5000000 ? 6 : cells < 8000000 ? 8 : 10;
     g->rows = rows ? rows
                    : cells < 5000000 ? 12 : cells < 8000000 ? 24 : cells < 30000000 ? 32 : 48;
@@ -343,13 +367,17 @@ int check_grid(const fd2d_grid &G, int k)
     return 0;
 }
 
+// fd2d_batch_desc.vec of a batch in register tiles
+constexpr int BATCH_TILES = 2;
+
 // launches of one batched run (shared by fd2d_batch_run and the graph capture)
 int batch_launches(const fd2d_batch_desc *b, int t0, int nsteps, int max_wave_len,
                    int max_probe_len, hipStream_t s)
 {
     if (!b || !b->grids_dev || !b->units_dev || b->nunits <= 0 || b->waves <= 0)
         return fail("fd2d_batch_run: incomplete batch descriptor");
-    if (!tb_supported(b->depth, b->cols)) return fail("fd2d_batch_run: depth/cols");
+    const bool tiles = b->vec == BATCH_TILES;
+    if (!tiles && !tb_supported(b->depth, b->cols)) return fail("fd2d_batch_run: depth/cols");
     if (t0 < 0 || nsteps < 0) return fail("fd2d_batch_run: t0=%d nsteps=%d", t0, nsteps);
     // the device indexes each grid's waveform and probe trace at t-1 with
     // that grid's own lengths: the recorded minima bound every grid
@@ -377,7 +405,10 @@ int batch_launches(const fd2d_batch_desc *b, int t0, int nsteps, int max_wave_le
     for (int l = 0; l < L; ++l) {
         const int k = nsteps / L + (l < nsteps % L ? 1 : 0);
         vac.mode = b->unit_work ? (l == 0 ? 1 : 2) : 0;
-        int rc = launch_fd2d_batch(b->grids_dev, b->units_dev, b->nunits, b->waves, k, b->cols,
+        int rc = tiles ? launch_fd2d_rt_batch(b->grids_dev, b->units_dev, b->nunits, b->waves,
+                                              b->rows / RT_ROWS, k, D, l % 2, t0 + done + 1,
+                                              l == L - 1, s)
+                       : launch_fd2d_batch(b->grids_dev, b->units_dev, b->nunits, b->waves, k, b->cols,
                                    b->vec != 0, l % 2, t0 + done + 1, l == L - 1, halo, vac, s);
         if (rc) return rc;
         done += k;
@@ -1553,6 +1584,10 @@ int fd2d_batch_units(const fd2d_grid *grids, int ngrids, int depth, int rows, in
     long long n = 0;
     for (int k = 0; k < ngrids; ++k) {
         if (grids[k].nx < 2 || grids[k].ny < 2) return fail("fd2d_batch_units: grid %d size", k);
+        if (g.tiles) {
+            n += rt_tiles(grids[k].nx, grids[k].ny, g.rows / RT_ROWS, g.depth);
+            continue;
+        }
         const int h = std::min(g.rows, grids[k].nx);
         n += (long long)((grids[k].ny + w - 1) / w) * ((grids[k].nx + h - 1) / h);
     }
@@ -1587,6 +1622,12 @@ int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, i
     std::vector<int> edge, inner;
     for (int k = 0; k < ngrids; ++k) {
         const fd2d_grid &G = grids[k];
+        if (g.tiles) {
+            const int nt = rt_tiles(G.nx, G.ny, g.rows / RT_ROWS, g.depth);
+            const int nsx = rt_tiles(1, G.ny, g.rows / RT_ROWS, g.depth);
+            for (int q = 0; q < nt; ++q) edge.insert(edge.end(), {k, q % nsx, q / nsx, 0});
+            continue;
+        }
         const int h = std::min(g.rows, G.nx);
         const int ns = (G.ny + w - 1) / w, nb = (G.nx + h - 1) / h;
         const int rlo = G.band_rows[1] > G.band_rows[0] ? std::max(G.band_rows[0], 1) : 0;
@@ -1621,7 +1662,10 @@ int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, i
     // L2.  MI355X, the 256-grid batch, depth 10, 64 rows: persistent waves
     // 29.2 ms; one workgroup a unit, runs of 1 / 4 / 16 / 64 / 256 units dealt
     // to the XCDs in turn 27.1 / 25.2 / 24.4 / 23.9 / 23.4, eighths 23.2.
-    if (waves <= 0) {
+    if (g.tiles) {
+        // all alike: grid by grid, an eighth of the list an XCD
+        waves = waves <= 0 ? n : std::min(waves, n);
+    } else if (waves <= 0) {
         waves = n;
         std::vector<int> lay;
         lay.reserve(4 * (size_t)n);
@@ -1682,7 +1726,7 @@ int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, i
     out->rows = g.rows;
     out->cols = g.cols;
     out->waves = waves;
-    out->vec = vec ? 1 : 0;
+    out->vec = g.tiles ? BATCH_TILES : vec ? 1 : 0;
     out->wave_len = min_wave;
     out->probe_len = min_probe;
     out->unit_work = nullptr;

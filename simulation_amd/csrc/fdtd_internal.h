@@ -157,12 +157,17 @@ struct RtParams {
     const float *inc;
     float *ft_r, *ft_i;
     float tw[RT_MAX_STEPS][2 * TB_MAX_FREQ];    // per step: cosines, then sines
+    __device__ void outputs() const {}          // the output pointers are here already
 };
 // Tiles of waves * RT_ROWS rows by 64 columns that cover the grid, each
 // sharing 2K rows or columns with its neighbours.
 int rt_tiles(int nx, int ny, int waves, int K);
 // One launch of p.K steps.  The input and output sets must differ.
 int launch_fd2d_rt(const RtParams &p, int waves, int nf, bool lossy, bool pml, hipStream_t s);
+// The same over a batch's tiles (units: grid, tile column, tile row, unused),
+// K steps of tiles cut with an overlap of H.
+int launch_fd2d_rt_batch(const fd2d_grid *grids, const int *units, int nunits, int groups, int waves,
+                         int K, int H, int parity, int t_first, int write_ez, hipStream_t s);
 int preload_rt();
 
 // Arguments of one learned-boundary frame launch (lbc_frame.hip).

@@ -1,8 +1,8 @@
-"""Batches in the library's own launch shapes -- one workgroup a unit, depth and
-rows by the cells of all grids -- and in persistent waves against single-grid
-runs, bit for bit: fewer units than XCDs, unit counts that 8 does not divide,
-grids of edge units only, row blocks cut short, row-, column-only and corner
-units, both sides of each change of shape."""
+"""Batches in the library's own launch shapes -- register tiles or strips, one
+workgroup a unit, depth and rows by the cells of all grids -- and in persistent
+waves against single-grid runs, bit for bit: fewer units than XCDs, unit counts
+that 8 does not divide, grids of edge units only, row blocks cut short, row-,
+column-only and corner units, both sides of each change of shape."""
 import pytest
 
 from conftest import same_bits
@@ -22,13 +22,21 @@ def _specs(sides):
 
 
 @pytest.mark.parametrize("sides,depth,rows,steps,waves", [
-    ([(20, 30)], 6, 12, 13, 0),
-    ([(40, 33), (64, 48), (25, 130)], 6, 12, 26, 0),
-    ([(150, 170), (97, 211), (300, 49), (211, 64)], 6, 12, 50, 0),
-    ([(2200, 2200), (150, 1200)], 8, 24, 17, 0),             # 5.0 million cells
-    ([(2700, 2960), (61, 333)], 10, 32, 21, 0),              # 8.0 million
-    ([(5300, 5650), (700, 90)], 10, 48, 20, 0),              # 30 million
-    ([(150, 170), (97, 211), (300, 49)], 6, 12, 26, 7),      # persistent waves
+    # register tiles: one tile, tiles of one grid cut and another not, 14 to 8
+    # steps a launch, past two tiles a CU, fewer workgroups than tiles
+    ([(20, 30)], 14, 32, 13, 0),
+    ([(32, 64), (33, 65), (64, 48), (25, 130)], 14, 32, 29, 0),
+    ([(150, 170), (97, 211)], 14, 32, 50, 0),
+    ([(150, 170), (97, 211), (300, 49), (211, 64)], 12, 32, 50, 0),
+    ([(200, 210)] * 4 + [(250, 140)] * 3, 12, 48, 31, 0),
+    ([(260, 310)] * 7 + [(100, 640)], 10, 48, 25, 0),
+    ([(260, 310)] * 9 + [(100, 640)], 8, 48, 25, 0),
+    ([(700, 900), (1500, 600), (1200, 1100)], 8, 48, 17, 0),
+    ([(150, 170), (97, 211), (300, 49)], 12, 32, 30, 7),
+    # strips: 5.0, 8.0 and 30 million cells
+    ([(2200, 2200), (150, 1200)], 8, 24, 17, 0),
+    ([(2700, 2960), (61, 333)], 10, 32, 21, 0),
+    ([(5300, 5650), (700, 90)], 10, 48, 20, 0),
 ])
 def test_default_shapes_match_single_grids(gpu, sides, depth, rows, steps, waves):
     from simulation_amd.batch import BatchSolver, single_solver
@@ -48,3 +56,39 @@ def test_default_shapes_match_single_grids(gpu, sides, depth, rows, steps, waves
             assert same_bits(a[f], r[f]), (k, f)
         if sp.probe is not None:
             assert same_bits(b.probe_trace(k), s.probe_traces()[0]), k
+
+
+@pytest.mark.parametrize("depth,rows,steps,waves", [(6, 12, 26, 0), (6, 12, 26, 7), (8, 24, 21, 3)])
+def test_strip_units_match_single_grids(gpu, depth, rows, steps, waves):
+    from simulation_amd.batch import BatchSolver, single_solver
+    print(f"[batch units] strips {depth}/{rows} waves={waves}", flush=True)
+    specs = _specs([(40, 33), (150, 170), (97, 211), (300, 49), (25, 130)])
+    b = BatchSolver(specs, steps, depth=depth, rows=rows, waves=waves, device=gpu)
+    b.run(steps)
+    for k, sp in enumerate(specs):
+        s = single_solver(sp, steps, gpu, depth=5, rows=37)
+        s.run(steps)
+        a, r = b.grid_state(k), s.state()
+        for f in ("dz", "iz", "ez", "hx", "hy", "ihx", "ihy"):
+            assert same_bits(a[f], r[f]), (k, f)
+
+
+def test_tile_batch_replayed_as_a_graph(gpu):
+    """A captured tile batch replayed three times, eager work in between,
+    against eager runs."""
+    import torch
+    from simulation_amd.batch import BatchSolver
+    print("[batch units] graph", flush=True)
+    specs = _specs([(150, 170), (97, 211), (64, 48)])
+    with torch.cuda.stream(torch.cuda.Stream()):
+        a, b = BatchSolver(specs, 60, device=gpu), BatchSolver(specs, 60, device=gpu)
+        for _ in range(3):
+            a.t = b.t = 0                        # steps 1 .. 30 again
+            a.run_graph(30)
+            b.run(30)
+            torch.cuda.synchronize()
+            for k in range(len(specs)):
+                x, y = a.grid_state(k), b.grid_state(k)
+                for f in x:
+                    assert same_bits(x[f], y[f]), (k, f)
+        a.close()

@@ -60,6 +60,7 @@ constexpr int RMAX = ((RMAX_C > RMAX_E ? RMAX_C : RMAX_E) + 3) / 4 * 4;   // kee
 constexpr int PMAX = 136;                     // positions per workgroup (130 at K = 10)
 
 struct FrameSmem {
+    bf16x8 w1[16][64];      // W1's operands of each lane: hidden tile, K step
     // ez, hx, hy of the region (the other fields are in registers), then one
     // element that stays 0: the source of constant samples
     float fld[3 * RMAX + 4];
@@ -112,7 +113,6 @@ __device__ inline int gidx(int e, int t, int nx, int ny)
 // Layer weights of one lane in MFMA A-operand form (W_FRM of the bf16
 // buffer, in frm_slot's order).
 struct LaneW {
-    bf16x8 w1[4][4];        // hidden tile mt, K step ks
     bf16x8 w2[4][2];
     bf16x8 w3[2];
 };
@@ -120,10 +120,6 @@ struct LaneW {
 __device__ __forceinline__ void load_lane_w(LaneW &W, const uint16_t *wbuf, int lane)
 {
     const uint16_t *b = wbuf + W_FRM + lane * FRM_OPS * 8;
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks) W.w1[mt][ks] = ld8(b + (mt * 4 + ks) * 8);
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -426,6 +422,8 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
         S.b1[k] = P.params[P_B1 + k];
         S.b2[k] = P.params[P_B2 + k];
     }
+    for (int k = tid; k < 16 * 64; k += NT)
+        S.w1[k / 64][k % 64] = ld8(P.w + W_FRM + ((k % 64) * FRM_OPS + k / 64) * 8);
     LaneW LW;
     load_lane_w(LW, P.w, lane);
     // a network whose hidden layers' output layer is zero adds exactly
@@ -519,7 +517,7 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
             for (int mt = 0; mt < 4; ++mt) {
                 z[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) z[mt] = mfma(LW.w1[mt][ks], xb[ks], z[mt]);
+                for (int ks = 0; ks < 4; ++ks) z[mt] = mfma(S.w1[mt * 4 + ks][lane], xb[ks], z[mt]);
             }
             bf16x8 a1[2];
             act_pack(z, S.b1, g, a1);

@@ -30,8 +30,8 @@
 // accumulator (hidden units 16 mt + 4 g + v of column c) is, after GELU and
 // rounding, the next layer's input operand once the next layer's weight
 // columns are permuted to match (unit (2 ks + v/4) 16 + 4 g + v%4 at K index
-// 32 ks + 8 g + v): no LDS between the layers.  The layer weights sit in
-// registers for the whole kernel; the FP32 linear path and the biases in
+// 32 ks + 8 g + v): no LDS between the layers.  The layer weights, the
+// FP32 linear path and the biases sit in
 // LDS.  b3 is left out: the odd combination cancels it.  The ring enters
 // and leaves through a global history buffer (four samples per position,
 // newest first; ping-ponged between launches).  Expressions follow
@@ -51,37 +51,41 @@ constexpr int CH = 32;                        // chunk length along the edge (at
                                               // 256 workgroups, one per CU)
 constexpr int KMAX = 10;                      // steps per launch
 constexpr int NT = 512;                       // threads per workgroup (8 waves)
-// region cells: corner chunks (3K+6) x (CH + 2K + 1), others at most
-// (2K+6) x (CH + 3K + 2) (30 x 49 and 22 x 58 at K = 8, 36 x 53 and
-// 26 x 64 at K = 10)
-constexpr int RMAX_C = (3 * KMAX + 6) * (CH + 2 * KMAX + 1);
-constexpr int RMAX_E = (2 * KMAX + 6) * (CH + 3 * KMAX + 2);
-constexpr int RMAX = ((RMAX_C > RMAX_E ? RMAX_C : RMAX_E) + 3) / 4 * 4;   // keeps the ring 16-byte aligned
 constexpr int PMAX = 136;                     // positions per workgroup (130 at K = 10)
 
+// cells of a region and positions of a workgroup at depth K, at most (rounded
+// so that what follows in LDS stays aligned)
+constexpr int region_cells(int K)
+{
+    const int corner = (3 * K + 6) * (CH + 2 * K + 1), edge = (2 * K + 6) * (CH + 3 * K + 2);
+    return ((corner > edge ? corner : edge) + 3) / 4 * 4;
+}
+constexpr int positions(int K) { return (CH + 3 * K + 2 + 2 * (3 * K + 3) + 7) / 8 * 8; }
+
+// LDS of a launch of at most KD steps
+template <int KD>
 struct FrameSmem {
-    bf16x8 w1[16][64];      // W1's operands of each lane: hidden tile, K step
+    static constexpr int RM = region_cells(KD), PM = positions(KD);
+    bf16x8 w[FRM_OPS][64];  // MFMA A operands of each lane, in frm_slot's order
     // ez, hx, hy of the region (the other fields are in registers), then one
     // element that stays 0: the source of constant samples
-    float fld[3 * RMAX + 4];
-    float ring[PMAX][HIST][NS];
+    float fld[3 * RM + 4];
+    float ring[PM][HIST][NS];
     float L[OUT][IN];       // linear path (FP32)
     float b1[HID], b2[HID];
-    int own[PMAX];          // global history index, or -1 when not owned
-    int16_t dst[PMAX][OUT]; // region cell of each prediction, or -1
-    uint8_t by[RMAX];       // position that predicts a cell, or 255
+    int own[PM];          // global history index, or -1 when not owned
+    int16_t dst[PM][OUT]; // region cell of each prediction, or -1
+    uint8_t by[RM];       // position that predicts a cell, or 255
 };
 static_assert(PMAX < 255, "positions in a byte");
 
-static_assert(sizeof(FrameSmem) + 64 <= 160 * 1024, "frame kernel LDS above 160 KiB");
+static_assert(sizeof(FrameSmem<KMAX>) + 64 <= 160 * 1024, "frame kernel LDS above 160 KiB");
 static_assert(CH + 3 * KMAX + 2 + 2 * (3 * KMAX + 3) <= PMAX && PMAX % 8 == 0,
               "positions of a frame workgroup above PMAX");
 // cells and samples of a workgroup at depth K fit n a thread
 constexpr bool fits(int K, int ncell, int nsamp)
 {
-    const int corner = (3 * K + 6) * (CH + 2 * K + 1), edge = (2 * K + 6) * (CH + 3 * K + 2);
-    return corner <= ncell * NT && edge <= ncell * NT &&
-           (CH + 3 * K + 2 + 2 * (3 * K + 3)) * NS <= nsamp * NT;
+    return region_cells(K) <= ncell * NT && positions(K) * NS <= nsamp * NT;
 }
 static_assert(fits(8, 3, 7) && fits(KMAX, 4, 8), "cells and samples a thread");
 
@@ -108,24 +112,6 @@ __device__ inline int gidx(int e, int t, int nx, int ny)
     case 2: return 2 * ny + t - 3;
     default: return 2 * ny + (nx - 6) + t - 3;
     }
-}
-
-// Layer weights of one lane in MFMA A-operand form (W_FRM of the bf16
-// buffer, in frm_slot's order).
-struct LaneW {
-    bf16x8 w2[4][2];
-    bf16x8 w3[2];
-};
-
-__device__ __forceinline__ void load_lane_w(LaneW &W, const uint16_t *wbuf, int lane)
-{
-    const uint16_t *b = wbuf + W_FRM + lane * FRM_OPS * 8;
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) W.w2[mt][ks] = ld8(b + (16 + mt * 2 + ks) * 8);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) W.w3[ks] = ld8(b + (24 + ks) * 8);
 }
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -332,19 +318,24 @@ __device__ __forceinline__ float add32(float v) { const Pair p = swap32(v); retu
 __device__ __forceinline__ float max16(float v) { const Pair p = swap16(v); return fmaxf(p.a, p.b); }
 __device__ __forceinline__ float max32(float v) { const Pair p = swap32(v); return fmaxf(p.a, p.b); }
 
-// NCELL cells and NSAMP samples a thread (3 and 7 up to depth 8, 4 and 8 up
-// to 10): fixed for the launch, so their fields and addresses stay in
+// Up to KD steps, NCELL cells and NSAMP samples a thread (3 and 7 up to depth
+// 8, 4 and 8 up to 10): fixed for the launch, so their fields and addresses stay in
 // registers (with all fields and the sample table in LDS, predictions through
 // a buffer of their own and the exchanges by __shfl_xor: 48 us a launch of 8
 // steps at 2048^2 against 36).  What bounds it is the latency of a level:
 // three phases between barriers (network with D and E; H; samples) on two
 // waves a SIMD, of which the network's exponentials and matrix products are
-// the longest.
-template <int NCELL, int NSAMP>
+// the longest.  The weights are read from LDS, not held (254 registers a lane
+// then, 150 now): two waves of the TM launches fit beside the frame's two on
+// a SIMD, and the LDS is sized by the depth so that they find room there too
+// (160 steps at 2048^2: 1386 us with the weights in registers, 1275 with W1 in
+// LDS, 1257 with all).
+template <int KD, int NCELL, int NSAMP>
 __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    FrameSmem &S = *reinterpret_cast<FrameSmem *>(smem_raw);
+    FrameSmem<KD> &S = *reinterpret_cast<FrameSmem<KD> *>(smem_raw);
+    constexpr int RMAX = FrameSmem<KD>::RM;
     const int nx = P.nx, ny = P.ny, K = P.K;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
     constexpr int NW = NT / 64, EZ = 0, HX = RMAX, HY = 2 * RMAX, ZERO = 3 * RMAX;
@@ -422,10 +413,8 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
         S.b1[k] = P.params[P_B1 + k];
         S.b2[k] = P.params[P_B2 + k];
     }
-    for (int k = tid; k < 16 * 64; k += NT)
-        S.w1[k / 64][k % 64] = ld8(P.w + W_FRM + ((k % 64) * FRM_OPS + k / 64) * 8);
-    LaneW LW;
-    load_lane_w(LW, P.w, lane);
+    for (int k = tid; k < FRM_OPS * 64; k += NT)
+        S.w[k / 64][k % 64] = ld8(P.w + W_FRM + ((k % 64) * FRM_OPS + k / 64) * 8);
     // a network whose hidden layers' output layer is zero adds exactly
     // nothing (y = 0, so the odd part 0.5 (y - y') is +0, as computed): skip
     // those layers
@@ -517,7 +506,7 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
             for (int mt = 0; mt < 4; ++mt) {
                 z[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int ks = 0; ks < 4; ++ks) z[mt] = mfma(S.w1[mt * 4 + ks][lane], xb[ks], z[mt]);
+                for (int ks = 0; ks < 4; ++ks) z[mt] = mfma(S.w[mt * 4 + ks][lane], xb[ks], z[mt]);
             }
             bf16x8 a1[2];
             act_pack(z, S.b1, g, a1);
@@ -525,12 +514,12 @@ __global__ void __launch_bounds__(NT) frame_kernel(LbcFrameParams P)
             for (int mt = 0; mt < 4; ++mt) {
                 z[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int ks = 0; ks < 2; ++ks) z[mt] = mfma(LW.w2[mt][ks], a1[ks], z[mt]);
+                for (int ks = 0; ks < 2; ++ks) z[mt] = mfma(S.w[16 + mt * 2 + ks][lane], a1[ks], z[mt]);
             }
             bf16x8 a2[2];
             act_pack(z, S.b2, g, a2);
 #pragma unroll
-            for (int ks = 0; ks < 2; ++ks) y = mfma(LW.w3[ks], a2[ks], y);
+            for (int ks = 0; ks < 2; ++ks) y = mfma(S.w[24 + ks][lane], a2[ks], y);
             }   // mlp
             // outputs v = 0..2 of column c in lanes g = 0: odd part from the
             // column pair (c, c + 8)
@@ -626,7 +615,7 @@ int preload_lbc_frame()
     return preload_kernel(reinterpret_cast<const void *>(&lbc::frame_setup_kernel));
 }
 
-size_t lbc_frame_smem() { return sizeof(lbc::FrameSmem); }
+size_t lbc_frame_smem() { return sizeof(lbc::FrameSmem<lbc::KMAX>); }
 
 size_t lbc_frame_table_bytes(int nx, int ny, int K)
 {
@@ -656,18 +645,19 @@ int lbc_frame_blocks(int nx, int ny, int K)
 int launch_lbc_frame(const LbcFrameParams &p, hipStream_t s)
 {
     const bool deep = p.K > 8;
-    const auto kernel = deep ? &lbc::frame_kernel<4, 8> : &lbc::frame_kernel<3, 7>;
+    const auto kernel = deep ? &lbc::frame_kernel<lbc::KMAX, 4, 8> : &lbc::frame_kernel<8, 3, 7>;
+    const size_t lds = deep ? sizeof(lbc::FrameSmem<lbc::KMAX>) : sizeof(lbc::FrameSmem<8>);
     static thread_local bool attr[2] = {};
     if (!attr[deep]) {
         int rc = hip_check(hipFuncSetAttribute((const void *)kernel,
                                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)sizeof(lbc::FrameSmem)),
+                                               (int)lds),
                            "lbc frame: shared memory");
         if (rc) return rc;
         attr[deep] = true;
     }
     hipLaunchKernelGGL(kernel, dim3(lbc_frame_blocks(p.nx, p.ny, p.K)), dim3(lbc::NT),
-                       sizeof(lbc::FrameSmem), s, p);
+                       lds, s, p);
     return hip_check(hipGetLastError(), "lbc frame kernel");
 }
 

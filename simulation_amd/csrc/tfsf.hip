@@ -298,6 +298,8 @@ __global__ void __launch_bounds__(1024) inc_chunk_reg_kernel(int ny, float *ezi,
             lds_barrier();
         }
     }
+    // in place: every wave has read its cells (and bc) before any are written
+    if (W > 1) __syncthreads();
 #pragma unroll
     for (int c = 0; c < M; ++c) {
         const int j = j0 + c;

@@ -369,8 +369,10 @@ __device__ __forceinline__ unsigned rt_slot(unsigned b, unsigned n)
     return xcd * (n / 8u) + min(xcd, n % 8u) + b / 8u;
 }
 
-template <bool LOSSY, bool PML, bool TF, int NF>
-__global__ void __launch_bounds__(64 * RT_WAVES) tm_rt_kernel(const RtParams P)
+// EU: waves a SIMD the registers are held to.
+template <bool LOSSY, bool PML, bool TF, int NF, int EU = 4>
+__global__ void __launch_bounds__(64 * RT_WAVES) __attribute__((amdgpu_waves_per_eu(EU)))
+tm_rt_kernel(const RtParams P)
 {
     __shared__ RtSmem S;
     const unsigned tile = rt_slot(blockIdx.x, gridDim.x), nsx = (unsigned)P.nsx;
@@ -466,6 +468,16 @@ template <bool TF, int NF>
 void launch_form(const RtParams &p, int waves, int tiles, bool lossy, bool pml, hipStream_t s)
 {
     const dim3 g(tiles), b(64 * waves);
+    // a plane wave without DFT planes needs 83 registers a lane: two tiles of 8
+    // waves a CU.  Held to 80 it spills three, and three tiles fit: from three a
+    // CU on that wins (MI355X, 256 steps: 700^2 813 -> 779 us, 1024^2 1171 ->
+    // 1054, 1500^2 1923 -> 1642), below it costs (400^2 497 -> 540).
+    if constexpr (TF && NF == 0) {
+        if (pml && lossy && tiles > 512) {
+            hipLaunchKernelGGL((tm_rt_kernel<true, true, TF, NF, 6>), g, b, 0, s, p);
+            return;
+        }
+    }
     if (pml && lossy) hipLaunchKernelGGL((tm_rt_kernel<true, true, TF, NF>), g, b, 0, s, p);
     else if (pml) hipLaunchKernelGGL((tm_rt_kernel<false, true, TF, NF>), g, b, 0, s, p);
     else if constexpr (!TF) {

@@ -313,7 +313,7 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream);
 /* The launch plan fd2d_tm_run would use for this descriptor and nsteps:
  * number of launches and the chosen depth/rows/cols.  Defaults (measured on
  * MI355X): with form, depth, rows and cols all 0, grids of up to 2.7 million
- * cells run register tiles of `rows` rows (32 or 48; depth 7 to 14 by the
+ * cells run register tiles of `rows` rows (32 to 64; depth 8 to 14 by the
  * number of tiles); otherwise strips of one column per lane, by the cells N
  * of the grid: depth 8 below 5.5 million, 10 below 11 million, else 11; rows
  * N/330000 below 6.6 million, N/230000 (at most 80) below 100 million, else

@@ -28,13 +28,13 @@
 // profile values (constants, no edge tests; the terms 0 * ihx and 0 * ihy
 // left out as in tm_tb_kernel), or the general one.
 //
-// What bounds it: on small grids the step itself (about 0.85 us a step for a
+// What bounds it: on small grids the step itself (about 0.7 us a step for a
 // 32-row tile at two waves a SIMD: instruction issue, then the two barriers)
 // and some 4 us a launch for the loads, stores and the gap; from 1000^2 on
 // the overlap (a third to a half of the cells computed) and the tiles' loads.
-// MI355X, strips before -> tiles, 192 steps, lossy, npml 8: 100^2 1055 -> 220
-// us, 400^2 1070 -> 274, 700^2 1085 -> 370, 1100^2 1109 -> 676, 1600^2 1181
-// -> 1120.
+// MI355X, strips before -> tiles, 192 steps, lossy, npml 8: 100^2 1055 -> 190
+// us, 400^2 1070 -> 235, 700^2 1085 -> 308, 1024^2 1120 -> 563, 1600^2 1181
+// -> 1050.
 #include "fdtd_internal.h"
 #include "lanes.h"
 
@@ -76,7 +76,13 @@ __host__ __device__ inline int rt_along(int n, int span, int H)
 
 // Tile (by, bx) of nsy x nsx, P.K steps; H >= P.K: the overlap the tiles are
 // cut with.  PR: RtParams or RtGrid.
-template <bool LOSSY, bool PML, bool TF, int NF, class PR>
+// SPLIT: one copy of the step loop per body.  Choosing the body again in every
+// phase took a seventh of a step (MI355X, 192 steps: 60^2 215 -> 185 us, 400^2
+// 265 -> 231, 1024^2 617 -> 563; plane wave 1024^2, three frequencies, 256
+// steps 1692 -> 1428), but the copies take 95 registers a lane instead of 78:
+// a batch of many tiles, which lives by three 8-wave or two 12-wave tiles a
+// CU, keeps the one loop (112 steps: 4.5 million cells 1563 us, 1870 split).
+template <bool LOSSY, bool PML, bool TF, int NF, bool SPLIT, class PR>
 __device__ __forceinline__ void rt_tile(PR &P, int H, int bx, int by, int nsx, int nsy,
                                         RtSmem &S)
 {
@@ -247,7 +253,7 @@ __device__ __forceinline__ void rt_tile(PR &P, int H, int bx, int by, int nsx, i
                 }
             }
         }
-        for (unsigned mk = pmask; mk; mk &= mk - 1u) {
+        for (unsigned mk = SP.v ? pmask : 0u; mk; mk &= mk - 1u) {
             const int k = __builtin_ctz(mk);
             const int rk = __builtin_amdgcn_readlane(sp_row, FDTD_MAX_SOURCES + k) - i0;
             float v = e[0];
@@ -317,24 +323,42 @@ __device__ __forceinline__ void rt_tile(PR &P, int H, int bx, int by, int nsx, i
         }
         up[w + 1][lane] = hy[R - 1];
     };
-    const bool sp = smask != 0 || tfw;
+    // steps in which a later own cell depends on the wave's rows (those within
+    // K-s of [o0, o1) at step s); in the others it only keeps the barriers
+    const int nact = i0 >= nx ? 0 : max(0, min(K, K - max(o0 - i0 - R, i0 - o1)));
+    auto steps = [&](auto G, auto SP) __attribute__((always_inline)) {
 #pragma unroll 1
-    for (int s = 0; s < K; ++s) {
-        // rows a later own cell depends on: K-s on either side of [o0, o1)
-        const bool act = i0 < nx && i0 + R > o0 - (K - s) && i0 < o1 + (K - s);
-        if (act) {
+        for (int s = 0; s < nact; ++s) {
+            e_phase(G, SP, s, up[w][lane]);
+            lds_barrier();
+            h_phase(G, SP, s, dn[w + 1][lane]);
+            lds_barrier();
+        }
+    };
+    const bool sp = smask || pmask || tfw;
+    // every wave passes the same number of barriers (K decides)
+    if constexpr (SPLIT) {
+        if (sp) steps(Int<1>{}, Int<1>{});
+        else if (plain) steps(Int<0>{}, Int<0>{});
+        else steps(Int<1>{}, Int<0>{});
+    } else {
+#pragma unroll 1
+        for (int s = 0; s < nact; ++s) {
             const float hu = up[w][lane];
             if (sp) e_phase(Int<1>{}, Int<1>{}, s, hu);
             else if (plain) e_phase(Int<0>{}, Int<0>{}, s, hu);
             else e_phase(Int<1>{}, Int<0>{}, s, hu);
-        }
-        lds_barrier();
-        if (act) {
+            lds_barrier();
             const float ed = dn[w + 1][lane];
             if (sp) h_phase(Int<1>{}, Int<1>{}, s, ed);
             else if (plain) h_phase(Int<0>{}, Int<0>{}, s, ed);
             else h_phase(Int<1>{}, Int<0>{}, s, ed);
+            lds_barrier();
         }
+    }
+#pragma unroll 1
+    for (int s = nact; s < K; ++s) {
+        lds_barrier();
         lds_barrier();
     }
     if (!rows_own || !own_col) return;
@@ -369,14 +393,12 @@ __device__ __forceinline__ unsigned rt_slot(unsigned b, unsigned n)
     return xcd * (n / 8u) + min(xcd, n % 8u) + b / 8u;
 }
 
-// EU: waves a SIMD the registers are held to.
-template <bool LOSSY, bool PML, bool TF, int NF, int EU = 4>
-__global__ void __launch_bounds__(64 * RT_WAVES) __attribute__((amdgpu_waves_per_eu(EU)))
-tm_rt_kernel(const RtParams P)
+template <bool LOSSY, bool PML, bool TF, int NF>
+__global__ void __launch_bounds__(64 * RT_WAVES) tm_rt_kernel(const RtParams P)
 {
     __shared__ RtSmem S;
     const unsigned tile = rt_slot(blockIdx.x, gridDim.x), nsx = (unsigned)P.nsx;
-    rt_tile<LOSSY, PML, TF, NF>(P, P.K, (int)(tile % nsx), (int)(tile / nsx), P.nsx,
+    rt_tile<LOSSY, PML, TF, NF, true>(P, P.K, (int)(tile % nsx), (int)(tile / nsx), P.nsx,
                                 (int)(gridDim.x / nsx), S);
 }
 
@@ -459,7 +481,7 @@ tm_rt_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ 
         P.nprobe = G.probe_i >= 0 ? 1 : 0;
         P.probe_i.v = G.probe_i; P.probe_j.v = G.probe_j;
         P.probe_out = G.probe_out; P.probe_len = G.probe_len;
-        rt_tile<true, true, false, 0>(P, H, bx, by, rt_along(G.ny, 64, H), rt_along(G.nx, T, H), S);
+        rt_tile<true, true, false, 0, false>(P, H, bx, by, rt_along(G.ny, 64, H), rt_along(G.nx, T, H), S);
         lds_barrier();                        // the next tile rewrites S
     }
 }
@@ -468,16 +490,6 @@ template <bool TF, int NF>
 void launch_form(const RtParams &p, int waves, int tiles, bool lossy, bool pml, hipStream_t s)
 {
     const dim3 g(tiles), b(64 * waves);
-    // a plane wave without DFT planes needs 83 registers a lane: two tiles of 8
-    // waves a CU.  Held to 80 it spills three, and three tiles fit: from three a
-    // CU on that wins (MI355X, 256 steps: 700^2 813 -> 779 us, 1024^2 1171 ->
-    // 1054, 1500^2 1923 -> 1642), below it costs (400^2 497 -> 540).
-    if constexpr (TF && NF == 0) {
-        if (pml && lossy && tiles > 512) {
-            hipLaunchKernelGGL((tm_rt_kernel<true, true, TF, NF, 6>), g, b, 0, s, p);
-            return;
-        }
-    }
     if (pml && lossy) hipLaunchKernelGGL((tm_rt_kernel<true, true, TF, NF>), g, b, 0, s, p);
     else if (pml) hipLaunchKernelGGL((tm_rt_kernel<false, true, TF, NF>), g, b, 0, s, p);
     else if constexpr (!TF) {

@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <atomic>
 #include <climits>
+#include <initializer_list>
 #include <mutex>
 #include <vector>
 
@@ -136,44 +137,46 @@ struct Plan {
     int rt;                // 1: register tiles (depth: steps of a launch, rows: of a tile)
 };
 
-// Waves and depth (*K) of register tiles (fd2d_rt.hip) by the number of tiles
-// a shape makes, tiles(waves, depth).
-// MI355X, us of 192 steps (lossy, npml 8; strips / tiles of 8, 12, 16 waves
-// at their best depth): 400^2 1070 / 274, 286, 293; 500^2 1089 / 323, 309,
-// 305; 600^2 1080 / 349, 353, 350; 850^2 1108 / 518, 466, 572; 1100^2 1109 /
-// 676, 659, 796; 1400^2 1132 / 908, 913, 1178; 1600^2 1181 / 1098, 1115,
-// 1549; 1531x2047 1254 / 1284, 1312, 1793.  So: while the tiles of 8 waves
-// number at most the 256 CUs, the deepest such launch (4 us a launch against
-// 0.85 us a step); then 12 waves, first one tile a CU, then two; past that 8
-// waves at depth 7, where the overlap costs as much as the launches.  Strips
-// are ahead from about 3 million cells on.
-// Plane waves (strips / tiles of 8 waves, 256 steps, three frequencies):
-// 150^2 2038 / 784 at depth 12, 832 at 8; 400^2 2191 / 953, 863; 1024^2 3413
-// / 2378, 1914; 1500^2 4970 / 3972, 2961; 128 steps: 4096^2 17230 / 9342 with
-// three frequencies, 6990 / 6555 without.
+// Register tiles (fd2d_rt.hip) in the first shape, of `waves` waves, whose
+// tiles(waves, depth) number at most `most`; sets *K to its depth, or returns
+// false.
 template <class Tiles>
-int rt_shape(const Tiles &tiles, int *K)
+bool rt_fits(const Tiles &tiles, int waves, std::initializer_list<int> depths, int most, int *K)
 {
-    for (int k : {14, 12, 10, 8})
-        if (tiles(8, *K = k) <= 256) return 8;
-    for (int most : {256, 512})
-        for (int k : {12, 10, 8})
-            if (tiles(12, *K = k) <= most) return 12;
-    *K = 7;
-    return 8;
+    for (int k : depths)
+        if (tiles(waves, *K = k) <= most) return true;
+    return false;
 }
 
 // Register tiles, where the caller leaves form, depth, rows and columns to the
-// library and the grid is small enough; tf: a plane-wave run.
+// library and the grid is small enough; tf: a plane-wave run.  MI355X, us of
+// 192 steps (lossy, npml 8; strips / tiles as waves/depth): 300^2 1069 / 8/12
+// 201, 12/12 231; 400^2 1070 / 8/8 235, 12/12 231, 16/12 262; 500^2 1089 / 8/10
+// 266, 12/12 242, 16/12 269; 600^2 1080 / 8/8 280, 12/8 298, 16/12 272; 700^2
+// 1085 / 8/8 374, 12/12 392, 16/10 308; 850^2 1108 / 8/8 464, 12/8 486, 16/12
+// 456; 1024^2 1120 / 8/8 563, 8/7 584, 16/10 607; 1600^2 1181 / 8/8 1050, 16/10
+// 1229.  So: while the tiles number at most the 256 CUs, the deepest such
+// launch of 8 waves (4 us a launch against 0.7 us a step), then 12, then 16
+// waves; past that 8 waves at depth 8, two tiles a CU at a time.  Strips are
+// ahead from about 3 million cells on.
+// Plane waves, 256 steps, three frequencies (strips / tiles): 150^2 2038 /
+// 8/12 499, 8/8 549; 400^2 2191 / 8/8 599, 8/12 605; 700^2 / 16/8 900, 8/8 980;
+// 1024^2 3413 / 8/8 1428, 16/8 1606; 1500^2 4970 / 8/8 2527, 16/8 2641.
 constexpr long RT_MAX_CELLS = 2700000, RT_MAX_CELLS_TF = 17000000;
 bool plan_rt(const fd2d_tm_desc *d, int nsteps, bool tf, Plan *pl)
 {
     if (d->form != FDTD_TM_FORM_AUTO || d->depth || d->rows || d->cols || nsteps < 2) return false;
     if ((long)d->nx * d->ny > (tf ? RT_MAX_CELLS_TF : RT_MAX_CELLS)) return false;
     auto tiles = [&](int waves, int k) { return rt_tiles(d->nx, d->ny, waves, k); };
-    int W = 8, K;
-    if (tf) K = tiles(8, 12) <= 256 ? 12 : 8;
-    else W = rt_shape(tiles, &K);
+    int W, K;
+    if (tf) {
+        W = rt_fits(tiles, 8, {12, 8}, 256, &K) || !rt_fits(tiles, 16, {8}, 256, &K) ? 8 : 16;
+    } else {
+        W = rt_fits(tiles, 8, {14, 12, 10, 8}, 256, &K) ? 8
+            : rt_fits(tiles, 12, {12}, 256, &K)         ? 12
+            : rt_fits(tiles, 16, {12, 10, 8}, 256, &K)  ? 16
+                                                        : 8;      // K is 8
+    }
     // an even number of launches: the result ends in the caller's state set
     int L = (nsteps + K - 1) / K;
     L += L % 2;
@@ -305,9 +308,9 @@ struct BatchGeom {
 };
 
 // The launch shape of a batch; depth, rows, cols 0: the library's choice, by
-// the cells of all grids together.  Below 5 million: register tiles, in the
-// shape a single grid of that many tiles has, past two tiles a CU 12 waves at
-// depth 8.  MI355X, us of 112 steps, strips (at their best shape below) / tiles
+// the cells of all grids together.  Below 5 million: register tiles, the
+// deepest launch of 8 waves whose tiles number at most the CUs, then of 12, then
+// twice as many; past that 12 waves at depth 8.  MI355X, us of 112 steps, strips (at their best shape below) / tiles
 // of 8 waves, depth 7 / 12 waves, depth 8 / 12: sides 96-250, 0.5M cells: 807 /
 // 329 / 333 / 282; 150-500, 1.8M: 950 / 677 / 652 / 705; 96-200, 4.5M: 1986 /
 // 1730 / 1563 / 1640; 300-500, 6.6M: 1733 / 2566 / 2161 / 2317.
@@ -329,11 +332,10 @@ int batch_geom(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols
             for (int k = 0; k < ngrids; ++k) n += rt_tiles(grids[k].nx, grids[k].ny, waves, K);
             return n;
         };
-        int W = rt_shape(tiles, &g->depth);
-        if (tiles(W, g->depth) > 512) {
-            W = 12;
-            g->depth = 8;
-        }
+        // the last test leaves depth 8 where nothing fits
+        const int W = rt_fits(tiles, 8, {14, 12, 10, 8}, 256, &g->depth) ? 8 : 12;
+        if (W == 12 && !rt_fits(tiles, 12, {12, 10, 8}, 256, &g->depth))
+            rt_fits(tiles, 12, {12, 10, 8}, 512, &g->depth);
         g->rows = W * RT_ROWS;
         g->cols = 1;
         g->halo = g->depth;

@@ -534,7 +534,7 @@ def bench_tfsf(a):
                                f"(fd2d/clang/test_3_4.c)", "grid": [n, n], "npml": npml,
                    "freq": list(freq),
                    # the fused run's defaults: register tiles of 32 rows,
-                   # depth 8 (12 while the tiles fit one a CU); strips from 17
+                   # depth 8 (small grids: 12, or 64 rows); strips from 17
                    # million cells on: with DFT planes depth 4 and rows
                    # max(4, n/220)
                    "depth": s.tm.depth or (8 if n * n <= 17000000 else 4),

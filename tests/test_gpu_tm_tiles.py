@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 # sides: one tile (32 x 64), one cell more, 2 cells; depth 14 (60, 130), 12
-# (300) and 8 (380) at 8 waves, 12 waves (490, 600 one tile a CU, 800 two), 8
-# waves at depth 7 (1200); cuts at depth 14: rows 18, 22, .., columns 50, 86, ..
+# (300) and 8 (380) at 8 waves, 12 waves (490), 16 waves at depth 12, 10 and 8
+# (600, 700, 740), 8 waves at depth 8 past that (800, 1200); cuts at depth 14: rows 18, 22, .., columns 50, 86, ..
 @pytest.mark.parametrize("nx,ny,npml,lossy,src,probes,chunks", [
     (2, 2, -1, False, [], [(1, 1)], (2, 3)),
     (5, 3, -1, True, [(0, 0), (4, 2)], [(4, 2)], (17,)),
@@ -29,6 +29,8 @@ pytestmark = pytest.mark.gpu
     (380, 377, 8, True, [(1, 1)], [(24, 56)], (33,)),
     (490, 501, 8, True, [(245, 250)], [(36, 52)], (26,)),
     (600, 607, 100, True, [(300, 300)], [(40, 56)], (17,)),
+    (700, 703, 8, True, [(350, 350)], [(54, 54)], (21,)),
+    (740, 737, 8, False, [(370, 370)], [(56, 56)], (17,)),
     (800, 797, 8, True, [(400, 400)], [(40, 56)], (18,)),
     (1200, 1203, 8, True, [(600, 600)], [(25, 57)], (15,)),
 ])
@@ -52,6 +54,7 @@ def test_tiles_general_body(gpu, oracle):
 @pytest.mark.parametrize("nx,ny,npml,nf,lossy,steps", [
     (40, 30, 8, 1, True, 70), (97, 131, 20, 3, True, 130), (150, 140, 8, 0, False, 64),
     (211, 190, 32, 2, False, 67), (400, 397, 20, 3, True, 96), (90, 64, 2, 3, True, 65),
+    (650, 640, 20, 3, True, 40), (800, 811, 20, 1, True, 33),
 ])
 def test_plane_wave_tiles_match_strips(gpu, nx, ny, npml, nf, lossy, steps):
     from simulation_amd import fd2d

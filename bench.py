@@ -555,7 +555,7 @@ def bench_dform(a):
     """The reference's 1-D Debye program (fd1d/clang/test_2_3.c main): 38000
     cells, Debye half space, additive Gaussian at 1, DFT at 50/200/500 MHz;
     one step = dxfield, exfield, fourier, hyfield (fd1d_dform_run, fused:
-    segments of 512 cells advance up to 32 steps per launch).  Algorithmic
+    register-resident waves advance up to 112 steps per launch).  Algorithmic
     bytes per cell-update: R+W dx ix sx hy (32), R nax..ndx (16), W ex (4),
     R+W 6 DFT planes (48) -- what one step of the per-step form moves, so
     `achieved` is an effective rate."""

@@ -41,8 +41,7 @@
 //     never read a cell another wave has already advanced.
 //   * Interior waves of tm_tb_kernel keep two sets of level carries and
 //     alternate them between sweep iterations (no register-to-register
-//     copies; the batch kernel keeps one set, which holds it at 4 waves per
-//     SIMD).  The profile values naz, nbz a level needs are not carried: the
+//     copies).  The profile values naz, nbz a level needs are not carried: the
 //     sweep keeps those of its last rows in a per-wave LDS ring (NaRing).
 //     All waves without DFT planes store through buffer resources
 //     whose range check drops the cells a wave does not own, so every
@@ -1221,8 +1220,7 @@ tm_tb_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ 
         // (those the sweep reads and one more below) and, if they are free
         // space, sweeps without them at once; its traffic is that of a
         // plain sweep.  (Recording inside the sweep, as tm_tb_kernel does,
-        // would take registers this kernel does not have at 4 waves per
-        // SIMD.)
+        // would take registers this kernel does not have.)
         if (!brow && !bcol && !sp) {
             bool v = vac.mode == 2 && ldu(vac.work, u) == (vac.tag | 1u);
             // the later launches move no iz in free-space units (+0 in both

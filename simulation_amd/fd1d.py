@@ -257,7 +257,7 @@ class DFormSolver:
     pulse added at src_pos striking a lossy (or Debye) half space, with the
     running DFT at freq, through fd1d_dform_run.  src_wave: host values of
     the additive source for steps 1.. (default gaussian(t, 50, 10)).
-    fused: the segment-blocked launches (up to 32 steps each, nf <= 3) with
+    fused: the segment-blocked launches (up to 112 steps each, nf <= 3) with
     the partner state set in a work buffer; else the per-step kernels."""
 
     def __init__(self, nx, md: medium1d, nsteps_max, freq=(), dt=None, src_pos=1,

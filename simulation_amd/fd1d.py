@@ -169,6 +169,8 @@ def simulate(cfg: Fd1dConfig, device=None) -> dict:
     if cfg.nx > _lib.lib().fd1d_run_max_nx(np.dtype(cfg.dtype).itemsize):
         # past fd1d_run's grid limit probes may count from the end, and be
         # more than a launch records: those are read between single steps
+        if cfg.ns > 0 and np.any((pk < -cfg.nx) | (pk >= cfg.nx)):
+            raise IndexError(f"probes {tuple(cfg.probes)} in a grid of {cfg.nx} cells")
         pk = np.where(pk < 0, pk + cfg.nx, pk).astype(np.int32)
         many = len(pk) > _lib.MAX_PROBES
     pk = np.ascontiguousarray(pk)

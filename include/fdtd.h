@@ -253,8 +253,9 @@ int fd2d_energy_diff(int wn, int wm, int nxa, int nya, int ia0, int ja0, const f
  *   space (ihx, ihy untouched).
  *   depth/rows/cols: temporal depth, rows per block and columns per lane;
  *   0 selects the built-in defaults (see fd2d_tm_plan).
- *   form: FDTD_TM_FORM_AUTO (0) lets the library choose (currently the
- *   single-wave strips, the faster form on MI355X); FDTD_TM_FORM_STRIP (1)
+ *   form: FDTD_TM_FORM_AUTO (0) lets the library choose: register tiles on
+ *   small grids (depth, rows and cols all 0, or cols FDTD_TILE_COLS), else
+ *   single-wave strips (see fd2d_tm_plan); FDTD_TM_FORM_STRIP (1)
  *   sweeps everything in single-wave strips (any cols);
  *   FDTD_TM_FORM_MULTIWAVE (2) sweeps the interior of the band in workgroups
  *   of four waves that exchange their edge columns through LDS (one column
@@ -308,17 +309,25 @@ typedef struct fd2d_tm_desc {
 #define FDTD_TM_FORM_STRIP 1
 #define FDTD_TM_FORM_MULTIWAVE 2
 
+/* cols of a shape in register tiles (a tile's columns; strips have columns
+ * per lane, 1 or 2).  With it, rows is a multiple of 4 up to 64 and depth up
+ * to 16 and below rows / 2.                                               */
+#define FDTD_TILE_COLS 64
+
 int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream);
 
 /* The launch plan fd2d_tm_run would use for this descriptor and nsteps:
  * number of launches and the chosen depth/rows/cols.  Defaults (measured on
  * MI355X): with form, depth, rows and cols all 0, grids of up to 2.7 million
- * cells run register tiles of `rows` rows (32 to 64; depth 8 to 14 by the
- * number of tiles); otherwise strips of one column per lane, by the cells N
+ * cells run register tiles of `rows` rows and FDTD_TILE_COLS columns (rows 32
+ * to 64; depth 8 to 14 by the number of tiles); otherwise strips of one column per lane, by the cells N
  * of the grid: depth 8 below 5.5 million, 10 below 11 million, else 11; rows
  * N/330000 below 6.6 million, N/230000 (at most 80) below 100 million, else
  * 96, at least 8.  The multi-wave form: depth 8, rows = nx/32 clamped to [32,
- * 512].  Depths go up to 12.  Host only.                                   */
+ * 512].  Depths of strips go up to 12.  The reported depth, rows and cols can
+ * be given back in the descriptor, with the same form, and make the same
+ * launches (register tiles then take grids of up to 17 million cells, also in
+ * fd2d_tfsf_run; fd2d_lbc_run takes them for 0, 0, 0).  Host only.         */
 int fd2d_tm_plan(const fd2d_tm_desc *d, int nsteps,
                  int *launches, int *depth, int *rows, int *cols);
 
@@ -354,7 +363,8 @@ typedef struct fd2d_batch_desc {
     const fd2d_grid *grids_dev;   /* device copy of the grid records */
     const int *units_dev;         /* device work list, 4 ints per unit */
     int nunits;
-    int depth, rows, cols;        /* fixed when the work list is made */
+    int depth, rows, cols;        /* fixed when the work list is made; a batch
+                                     given them runs the same launches */
     int waves;                    /* workgroups of a launch */
     int vec;                      /* 1: every grid allows vector loads; 2:
                                      register tiles (rows: of a tile) */
@@ -380,7 +390,8 @@ typedef struct fd2d_batch_desc {
  * 48) and columns per lane (0 = 1).  A unit is 4 ints: grid, strip, first
  * row, one past the last row.  With all three 0 and less than 5 million cells
  * the batch runs register tiles, as a small single grid does: grid, tile
- * column, tile row, 0.                                                     */
+ * column, tile row, 0 (cols FDTD_TILE_COLS: tiles of the depth and rows
+ * given).                                                                  */
 int fd2d_batch_units(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols,
                      int *nunits);
 

@@ -69,6 +69,7 @@ class Fd2dTmDesc(C.Structure):
 
 
 TM_FORM_AUTO, TM_FORM_STRIP, TM_FORM_MULTIWAVE = 0, 1, 2
+TILE_COLS = 64                   # cols of a shape in register tiles
 
 
 class Fd2dGrid(C.Structure):

@@ -134,7 +134,8 @@ struct Plan {
     int mw;                // 1: multi-wave form (rows = rows of its interior blocks)
     int frows;             // rows of the single-wave tiles (strips, or the frame of the
                            // multi-wave form)
-    int rt;                // 1: register tiles (depth: steps of a launch, rows: of a tile)
+    int rt;                // 1: register tiles (depth: steps of a launch, rows: of a tile;
+                           // cols: FDTD_TILE_COLS)
 };
 
 // Register tiles (fd2d_rt.hip) in the first shape, of `waves` waves, whose
@@ -162,14 +163,42 @@ bool rt_fits(const Tiles &tiles, int waves, std::initializer_list<int> depths, i
 // Plane waves, 256 steps, three frequencies (strips / tiles): 150^2 2038 /
 // 8/12 499, 8/8 549; 400^2 2191 / 8/8 599, 8/12 605; 700^2 / 16/8 900, 8/8 980;
 // 1024^2 3413 / 8/8 1428, 16/8 1606; 1500^2 4970 / 8/8 2527, 16/8 2641.
+// A reported tile shape given back (cols FDTD_TILE_COLS) is taken as it is, at
+// any length of run, up to the largest grid the tiles were measured on.
 constexpr long RT_MAX_CELLS = 2700000, RT_MAX_CELLS_TF = 17000000;
+int rt_check_shape(const char *fn, int nx, int ny, int depth, int rows)
+{
+    if (rows < RT_ROWS || rows % RT_ROWS || rows > RT_WAVES * RT_ROWS || depth < 1 ||
+        depth > RT_MAX_STEPS || 2 * depth >= rows)
+        return fail("%s: depth=%d rows=%d cols=%d is no register-tile shape", fn, depth, rows,
+                    FDTD_TILE_COLS);
+    if ((long long)nx * ny > RT_MAX_CELLS_TF)
+        return fail("%s: register tiles (cols=%d) take at most %ld cells, the grid is %dx%d", fn,
+                    FDTD_TILE_COLS, RT_MAX_CELLS_TF, nx, ny);
+    return 0;
+}
+
+// the caller gives a register-tile shape
+bool rt_given(const fd2d_tm_desc *d)
+{
+    return d->form == FDTD_TM_FORM_AUTO && d->cols == FDTD_TILE_COLS;
+}
+
+// tf: a plane-wave run.  A given shape has passed rt_check_shape.
 bool plan_rt(const fd2d_tm_desc *d, int nsteps, bool tf, Plan *pl)
 {
-    if (d->form != FDTD_TM_FORM_AUTO || d->depth || d->rows || d->cols || nsteps < 2) return false;
-    if ((long)d->nx * d->ny > (tf ? RT_MAX_CELLS_TF : RT_MAX_CELLS)) return false;
+    const bool given = rt_given(d);
+    if (nsteps < 2) return false;
+    if (!given) {
+        if (d->form != FDTD_TM_FORM_AUTO || d->depth || d->rows || d->cols) return false;
+        if ((long)d->nx * d->ny > (tf ? RT_MAX_CELLS_TF : RT_MAX_CELLS)) return false;
+    }
     auto tiles = [&](int waves, int k) { return rt_tiles(d->nx, d->ny, waves, k); };
     int W, K;
-    if (tf) {
+    if (given) {
+        W = d->rows / RT_ROWS;
+        K = d->depth;
+    } else if (tf) {
         W = rt_fits(tiles, 8, {12, 8}, 256, &K) || !rt_fits(tiles, 16, {8}, 256, &K) ? 8 : 16;
     } else {
         W = rt_fits(tiles, 8, {14, 12, 10, 8}, 256, &K) ? 8
@@ -178,14 +207,16 @@ bool plan_rt(const fd2d_tm_desc *d, int nsteps, bool tf, Plan *pl)
                                                         : 8;      // K is 8
     }
     // an even number of launches: the result ends in the caller's state set
+    // (an odd number of single steps leaves one for the per-step kernels)
     int L = (nsteps + K - 1) / K;
-    L += L % 2;
     *pl = Plan{};
     pl->rt = 1;
+    pl->tail_unfused = L % 2 && L == nsteps;
+    L += pl->tail_unfused ? -1 : L % 2;
     pl->launches = L;
-    pl->depth = (nsteps + L - 1) / L;
+    pl->depth = (nsteps - pl->tail_unfused + L - 1) / L;
     pl->rows = W * RT_ROWS;
-    pl->cols = 1;
+    pl->cols = FDTD_TILE_COLS;
     return true;
 }
 
@@ -227,8 +258,20 @@ void tm_defaults(int nx, int ny, int *depth, int *rows)
 
 int plan_tm(const fd2d_tm_desc *d, int nsteps, Plan *pl)
 {
+    if (rt_given(d)) {
+        const int rc = rt_check_shape("fd2d_tm", d->nx, d->ny, d->depth, d->rows);
+        if (rc) return rc;
+    }
     if (plan_rt(d, nsteps, false, pl)) return 0;
     pl->rt = 0;
+    if (rt_given(d)) {                     // no step, or one by the per-step kernels
+        pl->depth = d->depth; pl->rows = d->rows; pl->cols = d->cols;
+        pl->halo = pl->mw = pl->launches = 0;
+        pl->frows = d->rows;
+        pl->rt = 1;
+        pl->tail_unfused = nsteps == 1;
+        return 0;
+    }
     int D0 = 8, H0 = 16;
     tm_defaults(d->nx, d->ny, &D0, &H0);
     int D = d->depth ? d->depth : (d->form == FDTD_TM_FORM_MULTIWAVE ? 8 : D0);
@@ -325,7 +368,17 @@ int batch_geom(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols
 {
     long long cells = 0;
     for (int k = 0; k < ngrids; ++k) cells += (long long)grids[k].nx * grids[k].ny;
-    g->tiles = !depth && !rows && !cols && cells < 5000000;
+    g->tiles = cols == FDTD_TILE_COLS || (!depth && !rows && !cols && cells < 5000000);
+    if (cols == FDTD_TILE_COLS) {          // a reported tile shape given back
+        for (int k = 0; k < ngrids; ++k) {
+            const int rc = rt_check_shape("fd2d_batch", grids[k].nx, grids[k].ny, depth, rows);
+            if (rc) return rc;
+        }
+        g->depth = g->halo = depth;
+        g->rows = rows;
+        g->cols = cols;
+        return 0;
+    }
     if (g->tiles) {
         auto tiles = [&](int waves, int K) {
             long long n = 0;
@@ -337,7 +390,7 @@ int batch_geom(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols
         if (W == 12 && !rt_fits(tiles, 12, {12, 10, 8}, 256, &g->depth))
             rt_fits(tiles, 12, {12, 10, 8}, 512, &g->depth);
         g->rows = W * RT_ROWS;
-        g->cols = 1;
+        g->cols = FDTD_TILE_COLS;
         g->halo = g->depth;
         return 0;
     }
@@ -910,7 +963,6 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream)
     p.nprobe = d->nprobe;
     for (int k = 0; k < d->nprobe; ++k) { p.probe_i[k] = d->probe_i[k]; p.probe_j[k] = d->probe_j[k]; }
     p.probe_out = d->probe_out; p.probe_len = d->probe_len;
-    if (pl.rt) return rt_run(d, p, pl, t0, nsteps, nullptr, 0.f, S(stream));
     float *A[6] = {d->dz, d->iz, d->hx, d->hy, d->ihx, d->ihy};
     float *B[6] = {d->dz2, d->iz2, d->hx2, d->hy2, d->ihx2, d->ihy2};
     const int L = pl.launches;
@@ -920,7 +972,7 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream)
     // unless the caller promises an unchanged medium (tile_keep) and the
     // flags were recorded with this workspace, arrays and tile geometry at
     // a depth at least this call's
-    const bool vac = d->tile_work && !pl.mw && L >= 2 && d->tile_elems >= tm_tiles(d, pl);
+    const bool vac = d->tile_work && !pl.mw && !pl.rt && L >= 2 && d->tile_elems >= tm_tiles(d, pl);
     bool reuse = false;
     if (vac) {
         const int kmax = nfused / L + (nfused % L ? 1 : 0);
@@ -949,7 +1001,12 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream)
         p.tile_vac = d->tile_work;
     }
     int done = 0;
-    for (int l = 0; l < L; ++l) {
+    if (pl.rt && L) {
+        rc = rt_run(d, p, pl, t0, nfused, nullptr, 0.f, S(stream));
+        if (rc) return rc;
+        done = nfused;
+    }
+    for (int l = 0; l < L && !pl.rt; ++l) {
         const int k = nfused / L + (l < nfused % L ? 1 : 0);
         p.vac_mode = vac ? ((l == 0 && !reuse) ? 1 : 2) : 0;
         float **in = (l % 2 == 0) ? A : B;
@@ -1258,6 +1315,11 @@ static int tfsf_fused(const fd2d_tm_desc *d, const fd2d_tfsf_desc *b, int t0, in
     const fd2d_tm_desc *own = d;           // as the caller gave it
     fd2d_tm_desc dd = *d;
     dd.form = FDTD_TM_FORM_STRIP;          // TF/SF corrections and DFT: strip form
+    if (rt_given(own)) {
+        rc = rt_check_shape("fd2d_tfsf_run", d->nx, d->ny, d->depth, d->rows);
+        if (rc) return rc;
+        dd.depth = dd.rows = dd.cols = 0;  // of a chunk too short for tiles
+    }
     if (b->nf && !dd.depth) dd.depth = 4;
     // the plane-wave launches run the instantiation that carries the DFT
     // planes, whose level loop stays unrolled up to depth 8 only (past it the
@@ -1444,6 +1506,7 @@ int fd2d_lbc_run(const fd2d_tm_desc *d, const fd2d_lbc_desc *b, int t0, int nste
     Plan pl;
     fd2d_tm_desc ds = *d;
     ds.form = FDTD_TM_FORM_STRIP;         // the split launches are single-wave strips
+    if (rt_given(d)) ds.depth = ds.rows = ds.cols = 0;    // a tile shape is none of theirs
     if (!ds.depth) ds.depth = 8;          // and fuse at most LBC_MAX_DEPTH steps (the frame's tables)
     rc = plan_tm(&ds, 2 * LBC_MAX_DEPTH, &pl);
     if (rc) return rc;

@@ -267,7 +267,8 @@ class TMSolver:
     the same shapes is allocated for the ping-pong launches.  form:
     _lib.TM_FORM_AUTO (the library's choice), _lib.TM_FORM_STRIP (single-wave
     strips) or _lib.TM_FORM_MULTIWAVE (interior blocks swept by four waves
-    that exchange their edge columns); all give the same bits.
+    that exchange their edge columns); all give the same bits.  depth, rows,
+    cols: a launch shape, as plan() reports it (0: the library's choice).
     """
 
     def __init__(self, nx, ny, pml, md, sources=(), probes=(), nsteps_max=None,

@@ -364,10 +364,10 @@ typedef struct fd2d_batch_desc {
     const int *units_dev;         /* device work list, 4 ints per unit */
     int nunits;
     int depth, rows, cols;        /* fixed when the work list is made; a batch
-                                     given them runs the same launches */
+                                     given them runs the same launches (cols
+                                     FDTD_TILE_COLS: register tiles) */
     int waves;                    /* workgroups of a launch */
-    int vec;                      /* 1: every grid allows vector loads; 2:
-                                     register tiles (rows: of a tile) */
+    int vec;                      /* 1: every grid allows vector loads */
     int wave_len;                 /* smallest wave_len over grids with a source
                                      (INT_MAX: none), set by fd2d_batch_upload */
     int probe_len;                /* smallest probe_len over grids with a probe

@@ -422,17 +422,19 @@ int check_grid(const fd2d_grid &G, int k)
     return 0;
 }
 
-// fd2d_batch_desc.vec of a batch in register tiles
-constexpr int BATCH_TILES = 2;
-
 // launches of one batched run (shared by fd2d_batch_run and the graph capture)
 int batch_launches(const fd2d_batch_desc *b, int t0, int nsteps, int max_wave_len,
                    int max_probe_len, hipStream_t s)
 {
     if (!b || !b->grids_dev || !b->units_dev || b->nunits <= 0 || b->waves <= 0)
         return fail("fd2d_batch_run: incomplete batch descriptor");
-    const bool tiles = b->vec == BATCH_TILES;
-    if (!tiles && !tb_supported(b->depth, b->cols)) return fail("fd2d_batch_run: depth/cols");
+    const bool tiles = b->cols == FDTD_TILE_COLS;
+    if (tiles) {
+        const int rc = rt_check_shape("fd2d_batch_run", 0, 0, b->depth, b->rows);
+        if (rc) return rc;
+    } else if (!tb_supported(b->depth, b->cols)) {
+        return fail("fd2d_batch_run: depth/cols");
+    }
     if (t0 < 0 || nsteps < 0) return fail("fd2d_batch_run: t0=%d nsteps=%d", t0, nsteps);
     // the device indexes each grid's waveform and probe trace at t-1 with
     // that grid's own lengths: the recorded minima bound every grid
@@ -1791,7 +1793,7 @@ int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, i
     out->rows = g.rows;
     out->cols = g.cols;
     out->waves = waves;
-    out->vec = g.tiles ? BATCH_TILES : vec ? 1 : 0;
+    out->vec = vec ? 1 : 0;
     out->wave_len = min_wave;
     out->probe_len = min_probe;
     out->unit_work = nullptr;

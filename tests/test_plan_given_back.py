@@ -68,3 +68,16 @@ def test_batch_shape_given_back(sides, shape):
     assert L.lib().fd2d_batch_units(grids, len(sides), 0, 0, 0, C.byref(a)) == 0
     assert L.lib().fd2d_batch_units(grids, len(sides), *shape, L.TILE_COLS, C.byref(b)) == 0
     assert a.value == b.value
+
+
+@pytest.mark.parametrize("depth,rows,cols,vec", [(0, 32, 64, 0), (0, 0, 64, 0), (0, 32, 64, 2), (0, 32, 1, 2),
+                                                 (16, 32, 64, 0), (8, 30, 64, 0), (13, 32, 1, 2)])
+def test_batch_descriptor_without_a_shape(depth, rows, cols, vec):
+    """An incomplete descriptor is an error, not a division by zero."""
+    from simulation_amd import _lib as L
+    d = L.Fd2dBatchDesc()
+    d.grids_dev = d.units_dev = 0x1000
+    d.nunits = d.waves = 1
+    d.wave_len = d.probe_len = 100
+    d.depth, d.rows, d.cols, d.vec = depth, rows, cols, vec
+    assert L.lib().fd2d_batch_run(C.byref(d), 0, 4, 100, 100, None) == L.FDTD_EINVAL

@@ -161,7 +161,7 @@ def incthy(nx: int, ny: int, npml: int, ezi, hy) -> None:
 
 
 def _ft_struct(ft: ftrans) -> _lib.FdtdFtrans:
-    return pack(_lib.FdtdFtrans, *ft)
+    return pack(_lib.FdtdFtrans, *[getattr(ft, k) for k in ftrans._fields])
 
 
 def fourier(t: int, nf: int, nx: int, ny: int, dt: float, freq, ezi, ez, ft: ftrans) -> None:

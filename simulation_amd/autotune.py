@@ -42,10 +42,12 @@ def candidates(nx: int):
 
 
 def batch_candidates():
-    """(depth, rows, cols, waves) shapes tried for a batch: depth 10 with 32-64
+    """(depth, rows, cols, waves) shapes tried for a batch: the library's own
+    choice (by the cells of all grids: register tiles or strips), depth 10 with 32-64
     rows (on MI355X the 256-grid batch of sides 128-1024 peaks at depth 10,
     48 rows), shallower and shorter ones for smaller batches, and two columns
     per lane."""
+    yield 0, 0, 0, 0
     for rows in (32, 48, 64):
         yield 10, rows, 1, 0
     yield 8, 24, 1, 0
@@ -148,17 +150,20 @@ def tune_batch(b, steps: int = 48, use_cache: bool = True, configs=None,
     if b.t != 0:
         raise ValueError("tune_batch runs before the first step")
     sig = hashlib.sha1(repr([(s.nx, s.ny, s.npml) for s in b.specs]).encode()).hexdigest()[:16]
-    key = f"batch2|{_device()}|{len(b.specs)} grids|{sig}"
+    key = f"batch3|{_device()}|{len(b.specs)} grids|{sig}"
     db = _load() if use_cache and configs is None else {}
     if key in db:
         best = db[key]
     else:
         results = []
         for depth, rows, cols, waves in (configs or batch_candidates()):
-            n = 2 * depth * max(1, steps // (2 * depth))
-            if n > b.nsteps_max:
-                continue
             b.plan(depth, rows, cols, waves)
+            pair = 2 * b.desc.depth
+            n = pair * max(1, steps // pair)
+            if n > b.nsteps_max:
+                if depth or b.nsteps_max < 2:
+                    continue
+                n = b.nsteps_max - b.nsteps_max % 2      # the library's choice is always timed
 
             def go():
                 b.t = 0

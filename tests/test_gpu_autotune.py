@@ -49,3 +49,27 @@ def test_tune_batch_plans_fastest_and_resets(gpu):
         for f in ("dz", "iz", "ez", "hx", "hy", "ihx", "ihy"):
             assert same_bits(x[f], y[f]), (k, f)
         assert same_bits(b.probe_trace(k), ref.probe_trace(k))
+
+
+@pytest.mark.parametrize("nsteps_max,steps", [(64, 48), (20, 48)])
+def test_tune_batch_times_the_library_choice(gpu, nsteps_max, steps):
+    """A small batch tuned with the library's own shape (register tiles) among
+    the shapes: timed whatever its depth, kept where it is the faster, exact."""
+    from simulation_amd import autotune
+    from simulation_amd.batch import BatchSolver, c3_specs
+    assert next(autotune.batch_candidates()) == (0, 0, 0, 0)
+    print(f"[autotune batch] own shape, at most {nsteps_max} steps", flush=True)
+    specs = c3_specs(5, count=16, lo=96, hi=250)
+    ref = BatchSolver(specs, nsteps_max, depth=4, rows=30, device=gpu)
+    ref.run(nsteps_max)
+    b = BatchSolver(specs, nsteps_max, device=gpu)
+    # a strip of 128 rows takes some three times as long as the tiles
+    best = autotune.tune_batch(b, steps=steps, configs=[(0, 0, 0, 0), (8, 128, 1, 0)])
+    print("[autotune batch] best", best, flush=True)
+    assert [best[k] for k in ("depth", "rows", "cols", "waves")] == [0, 0, 0, 0]
+    assert b.desc.cols == 64 and b.t == 0
+    b.run(nsteps_max)
+    for k in range(len(specs)):
+        x, y = b.grid_state(k), ref.grid_state(k)
+        for f in x:
+            assert same_bits(x[f], y[f]), (k, f)

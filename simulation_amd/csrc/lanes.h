@@ -44,5 +44,16 @@ __device__ __forceinline__ double lane_get(double v, int lane)
     return __builtin_bit_cast(double, Int2{__builtin_amdgcn_readlane(q.lo, lane),
                                            __builtin_amdgcn_readlane(q.hi, lane)});
 }
+// the value of the lane that each lane names (from: 4 times its number)
+__device__ __forceinline__ float lane_pick(float v, int from)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, v)));
+}
+__device__ __forceinline__ double lane_pick(double v, int from)
+{
+    const Int2 q = __builtin_bit_cast(Int2, v);
+    return __builtin_bit_cast(double, Int2{__builtin_amdgcn_ds_bpermute(from, q.lo),
+                                           __builtin_amdgcn_ds_bpermute(from, q.hi)});
+}
 
 }  // namespace fdtd

@@ -86,3 +86,45 @@ def test_simulate_past_the_single_launch_limit(gpu, oracle, dt, nx, probes):
     assert same_bits(out["ex"], ex) and same_bits(out["hy"], hy) and same_bits(out["bc"], bc)
     if len(probes) <= 16:
         assert same_bits(out["probe"], np.concatenate(traces, 1))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("nx,ns,mode,pos,probes", [
+    (3, 70, 1, 1, (2, 0, 1, 1, 0, 2) * 2 + (1, 1, 0, 2)),
+    (64, 131, 2, 30, tuple(range(20, 36))),
+    (64, 9, 1, 63, (63, 0, 63, 5)),
+    (592, 77, 2, 300, tuple(range(290, 306))),
+    (1500, 300, 1, 40, tuple(range(33, 49))),
+    (3001, 130, 2, 1499, (1499, 1500) * 8),
+])
+def test_many_probes_of_one_wave_match_oracle(gpu, oracle, dt, nx, ns, mode, pos, probes):
+    from simulation_amd import fd1d
+    print(f"[fd1d probes] nx={nx} ns={ns} {np.dtype(dt)}", flush=True)
+    ex, hy, bc = _fields(nx, dt, nx + ns)
+    wave = np.random.default_rng(ns).standard_normal(ns).astype(dt)
+    d = [torch.from_numpy(a.copy()).to(gpu) for a in (ex, hy, bc, wave)]
+    pr = fd1d.run(nx, ns, d[0], d[1], d[2], None, None, mode, pos, d[3], probes)
+    ref = oracle.fd1d_run(nx, 0, ns, ex, hy, bc, None, None, mode, pos, wave, probes)
+    assert same_bits(d[0].cpu().numpy(), ex) and same_bits(d[1].cpu().numpy(), hy)
+    assert same_bits(pr.cpu().numpy(), ref)
+
+
+def test_many_probes_of_one_wave_cost_no_loop(gpu):
+    """16 probes in a wave: an exchange and a store a step (a loop over them
+    took 16 times as long as one probe; the bar is half of that)."""
+    from simulation_amd import fd1d
+    print("[fd1d probes] time", flush=True)
+    ex, hy = torch.zeros(64, device=gpu), torch.zeros(64, device=gpu)
+    best = []
+    for probes in ((20,), tuple(range(20, 36))):
+        us = []
+        for _ in range(12):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            fd1d.run(64, 4000, ex, hy, probes=probes)
+            b.record()
+            b.synchronize()
+            us.append(a.elapsed_time(b) * 1e3)
+        best.append(min(us))
+    print(f"[fd1d probes] {best[0]:.0f} us, 16 probes {best[1]:.0f} us", flush=True)
+    assert best[1] < 8 * best[0]

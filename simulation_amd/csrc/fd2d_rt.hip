@@ -444,8 +444,14 @@ struct RtGrid {
 };
 
 // Many grids, one workgroup a tile or fewer that take several; units: grid,
-// tile column, tile row.  Lossy PML form.  Six waves a SIMD: two 12-wave tiles
-// a CU.
+// tile column, tile row of tiles cut for H steps.  CUT: a launch of fewer steps
+// K cuts its own, as a single grid's does; the units left without a tile lie
+// evenly among the others, for at the end of a grid's they would idle whole
+// XCDs.  An instance of its own: the map spills scalars of the step loop.
+// MI355X, two launches of one step, cut for 8 steps / for one: 200 grids of
+// 150^2 179 / 160 us, 100 of 30x1000 100 / 78 (with 12 / 8 waves a tile).
+// Lossy PML form.  Six waves a SIMD: two 12-wave tiles a CU.
+template <bool CUT>
 __global__ void __launch_bounds__(64 * RT_WAVES) __attribute__((amdgpu_waves_per_eu(6)))
 tm_rt_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ units, int nunits,
                    int K, int H, int parity, int t_first, int write_ez)
@@ -453,8 +459,19 @@ tm_rt_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ 
     __shared__ RtSmem S;
     const int T = ((int)blockDim.x >> 6) * R;
     for (int u = (int)rt_slot(blockIdx.x, gridDim.x); u < nunits; u += (int)gridDim.x) {
-        const int gi = units[4 * u], bx = units[4 * u + 1], by = units[4 * u + 2];
-        const fd2d_grid &G = grids[gi];
+        const fd2d_grid &G = grids[units[4 * u]];
+        int bx = units[4 * u + 1], by = units[4 * u + 2];
+        int nsx = rt_along(G.ny, 64, H), nsy = rt_along(G.nx, T, H);
+        if constexpr (CUT) {
+            const long long q = (long long)by * nsx + bx, listed = (long long)nsx * nsy;
+            nsx = rt_along(G.ny, 64, K);
+            nsy = rt_along(G.nx, T, K);
+            const long long n = (long long)nsx * nsy;
+            const int tile = (int)(q * n / listed);
+            if (tile == (int)((q + 1) * n / listed)) continue;
+            by = tile / nsx;
+            bx = tile % nsx;
+        }
         RtGrid P;
         P.g = &G;
         P.swap = parity != 0;
@@ -481,7 +498,7 @@ tm_rt_batch_kernel(const fd2d_grid *__restrict__ grids, const int *__restrict__ 
         P.nprobe = G.probe_i >= 0 ? 1 : 0;
         P.probe_i.v = G.probe_i; P.probe_j.v = G.probe_j;
         P.probe_out = G.probe_out; P.probe_len = G.probe_len;
-        rt_tile<true, true, false, 0, false>(P, H, bx, by, rt_along(G.ny, 64, H), rt_along(G.nx, T, H), S);
+        rt_tile<true, true, false, 0, false>(P, CUT ? K : H, bx, by, nsx, nsy, S);
         lds_barrier();                        // the next tile rewrites S
     }
 }
@@ -534,8 +551,10 @@ int launch_fd2d_rt_batch(const fd2d_grid *grids, const int *units, int nunits, i
 {
     if (waves < 1 || waves > RT_WAVES || K < 1 || K > H || H > RT_MAX_STEPS || 2 * H >= waves * R)
         return fail("register tiles: %d of %d steps a launch in tiles of %dx64", K, H, waves * R);
-    hipLaunchKernelGGL(tm_rt_batch_kernel, dim3(groups), dim3(64 * waves), 0, s, grids, units, nunits,
-                       K, H, parity, t_first, write_ez);
+    // up to two tiles a CU, more and smaller tiles are as well
+    const auto kernel = K < H && nunits > 512 ? tm_rt_batch_kernel<true> : tm_rt_batch_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3(groups), dim3(64 * waves), 0, s, grids, units, nunits, K, H, parity,
+                       t_first, write_ez);
     return hip_check(hipGetLastError(), "fd2d_batch_run launch");
 }
 

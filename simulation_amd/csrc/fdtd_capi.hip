@@ -386,9 +386,15 @@ int batch_geom(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols
             return n;
         };
         // the last test leaves depth 8 where nothing fits
-        const int W = rt_fits(tiles, 8, {14, 12, 10, 8}, 256, &g->depth) ? 8 : 12;
+        int W = rt_fits(tiles, 8, {14, 12, 10, 8}, 256, &g->depth) ? 8 : 12;
         if (W == 12 && !rt_fits(tiles, 12, {12, 10, 8}, 256, &g->depth))
             rt_fits(tiles, 12, {12, 10, 8}, 512, &g->depth);
+        // grids of up to 32 rows: no wave without rows (40 grids of 30x3000, 8
+        // waves instead of 12: 112 steps 982 -> 810 us)
+        int tall = 0;
+        for (int k = 0; k < ngrids; ++k) tall = std::max(tall, grids[k].nx);
+        if (tall <= 8 * RT_ROWS)
+            W = std::max((tall + RT_ROWS - 1) / RT_ROWS, 2 * g->depth / RT_ROWS + 1);
         g->rows = W * RT_ROWS;
         g->cols = FDTD_TILE_COLS;
         g->halo = g->depth;

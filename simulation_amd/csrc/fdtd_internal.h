@@ -165,7 +165,7 @@ int rt_tiles(int nx, int ny, int waves, int K);
 // One launch of p.K steps.  The input and output sets must differ.
 int launch_fd2d_rt(const RtParams &p, int waves, int nf, bool lossy, bool pml, hipStream_t s);
 // The same over a batch's tiles (units: grid, tile column, tile row, unused),
-// K steps of tiles cut with an overlap of H.
+// K steps; the list is of tiles cut for H.
 int launch_fd2d_rt_batch(const fd2d_grid *grids, const int *units, int nunits, int groups, int waves,
                          int K, int H, int parity, int t_first, int write_ez, hipStream_t s);
 int preload_rt();

@@ -92,3 +92,34 @@ def test_tile_batch_replayed_as_a_graph(gpu):
                 for f in x:
                     assert same_bits(x[f], y[f]), (k, f)
         a.close()
+
+
+@pytest.mark.parametrize("sides,shape,runs,waves", [
+    # more than two tiles a CU: launches shallower than the list cut their own
+    # tiles; flat grids: tiles no taller than they are
+    ([(30, 3000)] * 13 + [(20, 30), (3, 500), (32, 64)], (8, 32), (2, 3, 7, 16, 21), 0),
+    ([(20, 2500)] * 14, (8, 20), (2, 9, 34), 0),
+    ([(20, 2500)] * 14, (8, 20), (2, 9, 34), 150),
+    ([(33, 1700), (1500, 40), (61, 60)] * 9 + [(700, 700)], (8, 48), (2, 5, 11), 0),
+    ([(30, 700)] * 3, (14, 32), (2, 3, 5), 0),
+    ([(30, 1000)] * 20, (12, 32), (3, 24), 0),
+])
+def test_shallow_launches_match_single_grids(gpu, sides, shape, runs, waves):
+    from simulation_amd.batch import BatchSolver, GridSpec, single_solver
+    print(f"[batch units] shallow {sides[:3]} waves={waves}", flush=True)
+    specs = [GridSpec(nx, ny, 8 if nx > 16 and ny > 16 else 1, [],
+                      (nx // 3, ny // 2, 20, 6.0) if k % 3 != 1 else None,
+                      (nx // 3 + 1, ny // 2) if k % 3 != 2 else None) for k, (nx, ny) in enumerate(sides)]
+    b = BatchSolver(specs, sum(runs), waves=waves, device=gpu)
+    assert (b.desc.depth, b.desc.rows, b.desc.cols) == (*shape, 64)
+    for n in runs:
+        b.run(n)
+    for k, sp in list(enumerate(specs))[:4] + list(enumerate(specs))[-3:]:
+        s = single_solver(sp, sum(runs), gpu, depth=5, rows=37)
+        for n in runs:
+            s.run(n)
+        a, r = b.grid_state(k), s.state()
+        for f in ("dz", "iz", "ez", "hx", "hy", "ihx", "ihy"):
+            assert same_bits(a[f], r[f]), (k, f)
+        if sp.probe is not None:
+            assert same_bits(b.probe_trace(k), s.probe_traces()[0]), k

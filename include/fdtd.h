@@ -399,7 +399,8 @@ int fd2d_batch_units(const fd2d_grid *grids, int ngrids, int depth, int rows, in
  * into the caller's device buffers (asynchronously on stream; the host
  * arrays may be released on return) and fill *out.  units_dev holds
  * 4*max_units ints, grids_dev ngrids records.  waves = 0 gives every unit a
- * workgroup of its own; otherwise `waves` persistent ones take units w, w +
+ * workgroup of its own (so does one per unit or more); otherwise `waves`
+ * persistent ones, at most those the device holds at once, take units w, w +
  * waves, ..., sorted by estimated cost and dealt out round by round in
  * alternating directions.                                                  */
 int fd2d_batch_upload(const fd2d_grid *grids, int ngrids, int depth, int rows, int cols,

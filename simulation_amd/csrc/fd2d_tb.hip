@@ -97,4 +97,23 @@ int launch_fd2d_batch(const fd2d_grid *grids, const int *units, int nunits, int 
 #undef FDTD_BATCH_CASE
 }
 
+int fd2d_batch_resident(int depth, int cols, bool vec, int *waves)
+{
+    switch (depth) {
+    case 1: return fd2d_batch_resident_depth<1>(cols, vec, waves);
+    case 2: return fd2d_batch_resident_depth<2>(cols, vec, waves);
+    case 3: return fd2d_batch_resident_depth<3>(cols, vec, waves);
+    case 4: return fd2d_batch_resident_depth<4>(cols, vec, waves);
+    case 5: return fd2d_batch_resident_depth<5>(cols, vec, waves);
+    case 6: return fd2d_batch_resident_depth<6>(cols, vec, waves);
+    case 7: return fd2d_batch_resident_depth<7>(cols, vec, waves);
+    case 8: return fd2d_batch_resident_depth<8>(cols, vec, waves);
+    case 9: return fd2d_batch_resident_depth<9>(cols, vec, waves);
+    case 10: return fd2d_batch_resident_depth<10>(cols, vec, waves);
+    case 11: return fd2d_batch_resident_depth<11>(cols, vec, waves);
+    case 12: return fd2d_batch_resident_depth<12>(cols, vec, waves);
+    default: return fail("temporal depth %d not built", depth);
+    }
+}
+
 }  // namespace fdtd

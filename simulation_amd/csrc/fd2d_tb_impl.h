@@ -1254,6 +1254,20 @@ int launch_batch_kv(const fd2d_grid *grids, const int *units, int nunits, int wa
     return hip_check(hipGetLastError(), "fd2d_batch_run launch");
 }
 
+template <int K, int C, bool VEC>
+int batch_resident_kv(int *waves)
+{
+    int per_cu = 0, dev = 0, ncu = 0;
+    int rc = hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                           &per_cu, (const void *)tm_tb_batch_kernel<K, C, VEC>, 64, 0),
+                       "occupancy query");
+    if (!rc) rc = hip_check(hipGetDevice(&dev), "hipGetDevice");
+    if (!rc) rc = hip_check(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev),
+                            "CU count");
+    if (!rc) *waves = per_cu * ncu;
+    return rc;
+}
+
 }  // namespace tb
 
 template <int K>
@@ -1270,6 +1284,15 @@ int launch_fd2d_batch_depth(const fd2d_grid *grids, const int *units, int nunits
     if (cols == 1)
         return tb::launch_batch_kv<K, 1, false>(grids, units, nunits, waves, parity, t_first, write_ez,
                                                 halo, vac, s);
+    return fail("columns per lane %d not built", cols);
+}
+
+template <int K>
+int fd2d_batch_resident_depth(int cols, bool vec, int *waves)
+{
+    if (cols == 2 && vec) return tb::batch_resident_kv<K, 2, true>(waves);
+    if (cols == 2) return tb::batch_resident_kv<K, 2, false>(waves);
+    if (cols == 1) return tb::batch_resident_kv<K, 1, false>(waves);
     return fail("columns per lane %d not built", cols);
 }
 

@@ -338,6 +338,10 @@ struct BatchVac {
 int launch_fd2d_batch(const fd2d_grid *grids, const int *units, int nunits, int waves, int depth,
                       int cols, bool vec, int parity, int t_first, int write_ez, int halo,
                       BatchVac vac, hipStream_t s);
+// waves of such a launch the device holds at once
+int fd2d_batch_resident(int depth, int cols, bool vec, int *waves);
+template <int K>
+int fd2d_batch_resident_depth(int cols, bool vec, int *waves);
 template <int K>
 int launch_fd2d_batch_depth(const fd2d_grid *grids, const int *units, int nunits, int waves,
                             int cols, bool vec, int parity, int t_first, int write_ez, int halo,

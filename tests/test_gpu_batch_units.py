@@ -123,3 +123,28 @@ def test_shallow_launches_match_single_grids(gpu, sides, shape, runs, waves):
             assert same_bits(a[f], r[f]), (k, f)
         if sp.probe is not None:
             assert same_bits(b.probe_trace(k), s.probe_traces()[0]), k
+
+
+@pytest.mark.parametrize("depth,rows,cols", [(4, 4, 1), (8, 4, 1), (11, 4, 1), (12, 4, 1), (8, 4, 2)])
+def test_persistent_waves_at_most_those_held_at_once(gpu, depth, rows, cols):
+    """Waves past those resident together, each with a share of the units,
+    would run as a second, partial round; as many as the units: one each."""
+    from simulation_amd.batch import BatchSolver, single_solver
+    print(f"[batch units] resident {depth}/{rows}/{cols}", flush=True)
+    specs = _specs([(700, 900), (1500, 600), (1201, 1100)])
+    b = BatchSolver(specs, 30, depth=depth, rows=rows, cols=cols, waves=4096, device=gpu)
+    per_simd = 4 if depth <= 7 else 3 if depth <= 11 else 2
+    assert b.desc.nunits > 4096
+    assert 1024 <= b.desc.waves <= 4096 and (cols > 1 or b.desc.waves == 1024 * per_simd)
+    b.run(30)
+    n = b.desc.nunits
+    c = BatchSolver(specs, 30, depth=depth, rows=rows, cols=cols, waves=n, device=gpu)
+    assert c.desc.waves == n
+    c.run(30)
+    for k, sp in enumerate(specs):
+        s = single_solver(sp, 30, gpu, depth=5, rows=37)
+        s.run(30)
+        r = s.state()
+        for x in (b.grid_state(k), c.grid_state(k)):
+            for f in r:
+                assert same_bits(x[f], r[f]), (k, f)

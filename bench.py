@@ -47,6 +47,7 @@ sys.path.insert(0, ROOT)
 
 B_ALG = 60          # bytes per cell-update, lossy PML form
 HBM_PEAK = 8000.0   # GB/s, MI355X
+TILE_COLS = 64      # cols of a launch shape in register tiles
 METRIC = "2D TM Mcell-updates/s + HBM roofline frac; learned-BC vs PML at equal reflection"
 
 
@@ -315,6 +316,17 @@ def bench_large_learned(cfg, W: int, K: int, dev) -> dict:
     return out
 
 
+def tm_kernel(cols, form="auto") -> str:
+    """The kernel of a 2-D launch shape."""
+    return ("tm_rt_kernel" if cols == TILE_COLS else
+            "tm_mw_kernel" if form == "multiwave" else "tm_tb_kernel")
+
+
+def tm_shape(depth, rows, cols, form="auto") -> str:
+    """A launch shape as the traffic records name it (tiles: 64 columns)."""
+    return f"d{depth}_r{rows}_c{cols}" + ("_mw" if form == "multiwave" else "")
+
+
 def bench_batch(a):
     """Batched workload: 256 square grids, sides uniform in [128, 1024] (seed
     0), 1-5 lossy cylinders each, npml=8, hard Gaussian point source, one probe
@@ -381,7 +393,8 @@ def bench_batch(a):
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 4),
                      "traffic": traffic_for(key), "traffic_key": key,
-                     "kernel": "tm_tb_batch_kernel", "avg_launch_ms": round(launch_ms, 4),
+                     "kernel": tm_kernel(b.desc.cols).replace("_kernel", "_batch_kernel"),
+                     "avg_launch_ms": round(launch_ms, 4),
                      "min_bytes_per_launch": int(min_bytes),
                      "effective_GBps_per_step": round(effective, 1),
                      "effective_frac": round(effective / HBM_PEAK, 4)},
@@ -521,6 +534,8 @@ def bench_tfsf(a):
     torch.cuda.synchronize()
     per_step = n * n * kp / (time.perf_counter() - tp) / 1e6
     del ps
+    given = a.depth or a.rows or a.cols
+    kernel = tm_kernel(a.cols if given or n * n > 17000000 else TILE_COLS)
     b_alg = 60 + 16 * len(freq)
     achieved = b_alg * n * n / (step_ms * 1e-3) / 1e9
     cpu = None if a.no_cpu else cpu_baseline_tfsf(n, a.cpu_seconds, npml, rgrid, freq)
@@ -533,17 +548,14 @@ def bench_tfsf(a):
                                f"cylinder r={rgrid} eps_r=30 sigma=0.3, DFT at 3 frequencies "
                                f"(fd2d/clang/test_3_4.c)", "grid": [n, n], "npml": npml,
                    "freq": list(freq),
-                   # the fused run's defaults: register tiles of 32 rows,
-                   # depth 8 (small grids: 12, or 64 rows); strips from 17
-                   # million cells on: with DFT planes depth 4 and rows
-                   # max(4, n/220)
-                   "depth": s.tm.depth or (8 if n * n <= 17000000 else 4),
-                   "rows": s.tm.rows or (32 if n * n <= 17000000 else max(4, min(512, n // 220))),
-                   "cols": s.tm.cols or 1,
+                   # the caller's shape; null: the library's choice (register
+                   # tiles up to 17 million cells, else strips)
+                   "depth": s.tm.depth or None, "rows": s.tm.rows or None,
+                   "cols": s.tm.cols or None,
                    "per_step_kernels_value": round(per_step, 1)},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK, 4), "traffic": None,
-                     "kernel": "fused fd2d_tfsf_run, effective per step (tm_rt_kernel "
+                     "kernel": f"fused fd2d_tfsf_run, effective per step ({kernel} "
                                "with TF/SF + DFT, and the incident chunk)",
                      "avg_launch_ms": round(step_ms, 4), "alg_bytes_per_launch": b_alg * n * n},
         "cpu_baseline": cpu,
@@ -797,7 +809,7 @@ def main():
     # the counter record of the launches' depth (of nearly all of them: 2000
     # steps at depth 11 are 180 launches of 11 and 2 of 10)
     mode = max(set(depths), key=depths.count) if depths else 0
-    shape = (f"d{mode}_r{plan['rows']}_c{plan['cols']}" + ("_mw" if a.form == "multiwave" else "")
+    shape = (tm_shape(mode, plan["rows"], plan["cols"], a.form)
              if depths and depths.count(mode) >= 0.9 * len(depths) else None)
     rec = {
         "metric": METRIC,
@@ -830,7 +842,7 @@ def main():
             "frac": round(achieved / HBM_PEAK, 4),
             "traffic": traffic_for(f"{workload}_{shape}") if shape else None,
             "traffic_key": f"{workload}_{shape}" if shape else None,
-            "kernel": "tm_mw_kernel" if a.form == "multiwave" else "tm_tb_kernel",
+            "kernel": tm_kernel(plan["cols"], a.form),
             "avg_launch_ms": round(launch_ms, 4),
             "min_bytes_per_launch": int(min_bytes),
             "effective_GBps_per_step": round(effective, 1),

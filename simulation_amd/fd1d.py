@@ -104,11 +104,21 @@ def run(nx: int, nsteps: int, ex, hy, bc=None, ca=None, cb=None, src_mode=SRC_NO
     dt = ex.dtype
     pk = np.ascontiguousarray(np.asarray(probes, dtype=np.int32).reshape(-1))
     pout = torch.empty((len(pk), max(nsteps, 0)), dtype=dt, device=ex.device)
-    if nx > _lib.lib().fd1d_run_max_nx(dt.itemsize):
-        name = "fd1d_run_f64" if dt == torch.float64 else "fd1d_run"      # refuses the size
-        call(name, int(nx), int(t0), int(nsteps), ptr(ca, dt), ptr(cb, dt), ptr(ex, dt),
-             ptr(hy, dt), ptr(bc, dt), int(src_mode), int(src_pos), ptr(src_wave, dt), 0, None,
-             None, stream())
+    L = _lib.lib()
+    # A few steps past one workgroup's registers (592 cells): one launch with
+    # the fields in LDS, where the blocked run needs two and a work buffer.
+    # MI355X, us of a call, LDS / blocked: FP32 593 cells, 1 / 4 / 8 steps 20.7
+    # / 20.6 / 22.7 against 22; 4096 cells, 1 / 2 steps 20.9 / 22.8 against 22.2;
+    # FP64 700 cells, 2 / 4 steps 20.2 / 21.3 against 21.7.  Past fd1d_run's limit
+    # the same call refuses the size.
+    if nx > L.fd1d_run_max_nx(dt.itemsize) or (nx * nsteps * dt.itemsize <= 20000
+                                               and L.fd1d_run_work_elems(int(nx))):
+        call("fd1d_run_f64" if dt == torch.float64 else "fd1d_run", int(nx), int(t0), int(nsteps),
+             ptr(ca, dt), ptr(cb, dt), ptr(ex, dt), ptr(hy, dt), ptr(bc, dt), int(src_mode),
+             int(src_pos), ptr(src_wave, dt), len(pk),
+             pk.ctypes.data_as(_lib._IP) if len(pk) else None,
+             ptr(pout, dt) if len(pk) else None, stream())
+        return pout
     _advance(nx, nsteps, ex, hy, bc, ca, cb, src_mode, src_pos, src_wave, pk, pout, t0)
     return pout
 

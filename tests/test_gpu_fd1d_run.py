@@ -48,3 +48,27 @@ def test_fd1d_run_matches_oracle(gpu, oracle, dt, nx, ns, form, mode, probes):
         assert same_bits(d[4].cpu().numpy(), bc)
     if probes:
         assert same_bits(out.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("nx", [592, 593, 1365, 2048, 4096])
+def test_short_runs_match_oracle(gpu, oracle, dt, nx):
+    """fd1d.run a few steps at a time: one launch in LDS while nx * steps is
+    small, the blocked run past that."""
+    from simulation_amd import _lib, fd1d
+    print(f"[fd1d short] nx={nx} {np.dtype(dt)}", flush=True)
+    rng = np.random.default_rng(nx)
+    ex, hy, bc, wave = (rng.standard_normal(n).astype(dt) for n in (nx, nx, 4, 40))
+    d = [torch.from_numpy(a.copy()).to(gpu) for a in (ex, hy, bc, wave)]
+    probes, t = (0, nx // 2, nx - 1), 0
+    for n in (1, 2, 3, 4, 6, 7, 12, 1):
+        pr = fd1d.run(nx, n, d[0], d[1], d[2], None, None, 2, nx // 3, d[3][t:t + n], probes, t)
+        ref = oracle.fd1d_run(nx, t, n, ex, hy, bc, None, None, 2, nx // 3,
+                              np.ascontiguousarray(wave[t:t + n]), probes)
+        assert same_bits(pr.cpu().numpy(), ref), n
+        t += n
+    assert fd1d.run(nx, 0, d[0], d[1], d[2]).shape == (0, 0)
+    with pytest.raises(_lib.FdtdError, match="probe_out"):       # an empty trace has no address
+        fd1d.run(nx, 0, d[0], d[1], d[2], probes=probes)
+    for a, b in zip(d, (ex, hy, bc)):
+        assert same_bits(a.cpu().numpy(), b)

@@ -321,11 +321,11 @@ int fd2d_tm_run(const fd2d_tm_desc *d, int t0, int nsteps, void *stream);
  * number of launches and the chosen depth/rows/cols.  Defaults (measured on
  * MI355X): with form, depth, rows and cols all 0, grids of up to 2.7 million
  * cells run register tiles of `rows` rows and FDTD_TILE_COLS columns (rows 32
- * to 64; depth 8 to 14 by the number of tiles); otherwise strips of one column per lane, by the cells N
- * of the grid: depth 8 below 5.5 million, 10 below 11 million, else 11; rows
- * N/330000 below 6.6 million, N/230000 (at most 80) below 100 million, else
- * 96, at least 8.  The multi-wave form: depth 8, rows = nx/32 clamped to [32,
- * 512].  Depths of strips go up to 12.  The reported depth, rows and cols can
+ * to 64; depth 8 to 14 by the number of tiles); otherwise strips of one column
+ * per lane, by the cells N of the grid: depth 8 below 5.5 million, 10 below 11
+ * million, else 11; rows N/330000 below 6.6 million, N/230000 (at most 80)
+ * below 100 million, else 96, at least 8.  The multi-wave form: depth 8, rows =
+ * nx/32 clamped to [32, 512].  Depths of strips go up to 12.  The reported depth, rows and cols can
  * be given back in the descriptor, with the same form, and make the same
  * launches (register tiles then take grids of up to 17 million cells, also in
  * fd2d_tfsf_run; fd2d_lbc_run takes them for 0, 0, 0).  Host only.         */
@@ -519,7 +519,8 @@ int lbc_train_grad(int n, const float *src, const long long *offs, long long tst
  * the frame kernel's geometry tables and the interior tiles' free-space
  * flags (recorded by the first launch of every call, as with
  * fd2d_tm_desc.tile_work; rewritten by every call; one run at a time per
- * work buffer).  nsteps >= 2 (an even number of launches).                 */
+ * work buffer).  nsteps >= 2 (an even number of launches).  Not into a stream
+ * that is being captured (an error).                                       */
 #define FDTD_LBC_MARGIN 32
 typedef struct fd2d_lbc_desc {
     const float *params;        /* lbc_param_count() FP32 parameters         */

@@ -1535,6 +1535,11 @@ int fd2d_lbc_run(const fd2d_tm_desc *d, const fd2d_lbc_desc *b, int t0, int nste
     const bool lossy = d->md.nbz != nullptr;
     if (!d->dz2 || !d->hx2 || !d->hy2 || (lossy && !d->iz2))
         return fail("fd2d_lbc_run: the partner state set (dz2, iz2, hx2, hy2) is required");
+    // its three streams order themselves by events that every launch records
+    // again; a capture of that ended in a segmentation fault on the host
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(S(stream), &cap) != hipSuccess) (void)hipGetLastError();
+    if (cap != hipStreamCaptureStatusNone) return fail("fd2d_lbc_run: the stream is being captured");
     int L = (nsteps + pl.depth - 1) / pl.depth;
     L += L % 2;
     TbParams p{};

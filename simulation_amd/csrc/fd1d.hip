@@ -240,7 +240,8 @@ __device__ __forceinline__ void run1d(Seg1d<T> &g, const Run1d<T> &P)
     for (int done = 0; done < P.n;) {
         const int n = min(g.chunk, P.n - done);
         T tr = 0;
-        T *out = P.probe_out + done + (PRB == 2 ? (size_t)lane : (size_t)g.pf) * P.probe_len;
+        T *out = P.probe_out + done;
+        if (PRB == 2) out += (size_t)lane * P.probe_len;
         if (SRC) {
             // the next chunk's values, in flight during this one
             const int k = done + n + lane;
@@ -248,7 +249,7 @@ __device__ __forceinline__ void run1d(Seg1d<T> &g, const Run1d<T> &P)
             sn = k < P.n ? P.src_wave[k] : T(0);
         }
         chunk1d<T, COEF, EDGE, SRC, PRB>(g, n, sw, tr, out);
-        if (PRB == 1 && lane < n) out[lane] = tr;
+        if (PRB == 1 && lane < n) out[(size_t)g.pf * P.probe_len + lane] = tr;
         done += n;
         if (g.many && done < P.n) {
             if (g.mine) { es[0] = g.e; es[P.region] = g.h; }

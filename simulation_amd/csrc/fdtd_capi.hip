@@ -159,7 +159,9 @@ bool rt_fits(const Tiles &tiles, int waves, std::initializer_list<int> depths, i
 // 1229.  So: while the tiles number at most the 256 CUs, the deepest such
 // launch of 8 waves (4 us a launch against 0.7 us a step), then 12, then 16
 // waves; past that 8 waves at depth 8, two tiles a CU at a time.  Strips are
-// ahead from about 3 million cells on.
+// ahead from about 3 million cells on in this form; the others cross later: 96
+// steps of 1640^2 in tiles / of 1700^2 in strips 548 / 632, lossless 446 / 565,
+// without a layer lossy 351 / 465, lossless 308 / 433.
 // Plane waves, 256 steps, three frequencies (strips / tiles): 150^2 2038 /
 // 8/12 499, 8/8 549; 400^2 2191 / 8/8 599, 8/12 605; 700^2 / 16/8 900, 8/8 980;
 // 1024^2 3413 / 8/8 1428, 16/8 1606; 1500^2 4970 / 8/8 2527, 16/8 2641.
